@@ -203,23 +203,25 @@ struct pp2p_ctx {
     long long walk_m2l_n = -1;      // -1: none since the last walk
     int walk_nnode = -1;        // nodes of the tree in the walk arrays (-1: none)
 
-    // device kd-tree (pp2p_build_tree): per level its segments and sons, and
-    // the per-particle arrays of the build; the finished tree goes to the
-    // walk arrays above, its leaf ranges to rng
+    // device kd-tree (pp2p_build_tree): per level its segments and sons in
+    // one buffer, the subtrees, and the per-particle arrays of the build; the
+    // finished tree goes to the walk arrays above, its leaf ranges to rng
     struct TreeLevel {
-        DevBuf<int2> seg, kid, leaf, below, idb;
-        DevBuf<float> split;
-        DevBuf<double> mean;
-        DevBuf<int> np0, kk;
-        DevBuf<float4> lo, hi;
-        int nseg = 0, nleaf = 0;
+        DevBuf<char> mem;
+        TreeLevelView v{};
+        int nseg = 0;
     };
     std::vector<TreeLevel> tl;
-    DevBuf<int> tx0, tx1, tx2, tidx, tsegof, tsmall, tsx, ttbl, ttag, tposi;
-    DevBuf<int> tnodef, tleaff, tnoff, tloff;
+    DevBuf<TreeSub> tsub;
+    DevBuf<unsigned short> tsuboff;     // level offsets of each subtree
+    DevBuf<TreeCounts> tcounts;
+    DevBuf<int> tx0, tx1, tx2, tidx, tla, tlb, tlc, tld, ttag, tposi;
+    DevBuf<unsigned long long> tmask;
+    DevBuf<int> ttcnt, ttmap;
     double tree_int2pos = 0.0;  // grid step of the last pp2p_build_tree
     bool tree_ready = false;    // walk arrays, tidx and rng hold the last pp2p_build_tree
-    int tree_levels = 0;        // levels of that tree (tl[0 .. tree_levels))
+    int tree_levels = 0;        // device-wide levels of that tree (tl[0 .. tree_levels))
+    int tree_nsub = 0;          // its subtrees (tsub), below them
 
     // M2L task loop and L2P: cells, their expansions, the task CSR
     DevBuf<float4> mcenter;
@@ -324,13 +326,12 @@ void pp2p_destroy(pp2p_ctx *c)
     }
     c->wcnt.release(); c->wpos_a.release(); c->wpos_b.release(); c->wemit.release();
     c->wsep.release(); c->wm2l_t.release(); c->wm2l_s.release();
-    for (auto &l : c->tl) {
-        l.seg.release(); l.kid.release(); l.leaf.release(); l.below.release(); l.idb.release(); l.split.release();
-        l.mean.release(); l.np0.release(); l.kk.release(); l.lo.release(); l.hi.release();
-    }
-    c->tx0.release(); c->tx1.release(); c->tx2.release(); c->tidx.release(); c->tsegof.release();
-    c->tsmall.release(); c->tsx.release(); c->ttbl.release(); c->ttag.release(); c->tposi.release();
-    c->tnodef.release(); c->tleaff.release(); c->tnoff.release(); c->tloff.release();
+    for (auto &l : c->tl)
+        l.mem.release();
+    c->tx0.release(); c->tx1.release(); c->tx2.release(); c->tidx.release(); c->tla.release();
+    c->tlb.release(); c->tlc.release(); c->tld.release(); c->ttag.release(); c->tposi.release();
+    c->tsub.release(); c->tsuboff.release(); c->tcounts.release();
+    c->tmask.release(); c->ttcnt.release(); c->ttmap.release();
     c->mcenter.release(); c->mM.release(); c->mL.release();
     for (DevBuf<int> *b : {&c->mtt, &c->mts, &c->mkey, &c->msrc, &c->mflag, &c->mrowidx, &c->mrow_tgt, &c->mrow_off})
         b->release();
@@ -880,6 +881,113 @@ int pp2p_walk_tasks(pp2p_ctx *c, int nnode, const int *node_son, const float *no
     return run_walk(c, open_angle, cutoff_radius, ntask);
 }
 
+// One level's arrays for up to cap segments in its buffer.
+static int tree_level_view(pp2p_ctx::TreeLevel &L, size_t cap)
+{
+    const size_t per[] = {sizeof(int2), sizeof(int), sizeof(int2), 2 * sizeof(int2), sizeof(double), sizeof(float),
+                          sizeof(int), sizeof(int), sizeof(int2), sizeof(int2), sizeof(float4), sizeof(float4)};
+    size_t at[12], end = 0;
+    for (int k = 0; k < 12; ++k) {
+        at[k] = end;
+        end += (per[k] * (cap + 1) + 255) & ~(size_t)255;       // toff holds one entry more
+    }
+    HIPCHK(L.mem.reserve(end));
+    char *p = L.mem.p;
+    L.v = TreeLevelView{(int2 *)(p + at[0]), (int *)(p + at[1]), (int2 *)(p + at[2]), (int2 *)(p + at[3]),
+                        (double *)(p + at[4]), (float *)(p + at[5]), (int *)(p + at[6]), (int *)(p + at[7]),
+                        (int2 *)(p + at[8]), (int2 *)(p + at[9]), (float4 *)(p + at[10]), (float4 *)(p + at[11])};
+    return PP2P_OK;
+}
+
+// The splits of the whole tree from the uploaded grid positions: segments of
+// more than gmax particles level by level (*levels of them in c->tl), then
+// the *nsub subtrees; *counts: nodes and leaves.  *fits = false: a subtree did
+// not fit its workgroup and nothing else is valid.  The levels' sizes stay
+// on the device: a group of levels is launched at once, with grids for as many
+// segments as they can hold (a level that turns out empty is a few empty
+// launches), and the host reads the sizes once per group.
+static int tree_split_all(pp2p_ctx *c, const TreeScratch &w, long long n, double int2pos, int maxleaf, int gmax,
+                          int *levels, int *nsub, int2 *counts, bool *fits)
+{
+    int st;
+    const hipStream_t sm = c->stream;
+    const bool subs = gmax > maxleaf;
+    const bool root_sub = subs && n <= gmax;
+    const long long cap_all = n / ((long long)gmax + 1) + 1;
+    const long long subcap = subs ? std::min(n / ((long long)maxleaf + 1) + 1, 64 * cap_all + 64) : 1;
+    HIPCHK(hipStreamSynchronize(sm));          // nothing in flight while buffers grow
+    HIPCHK(c->tsub.reserve(subcap));
+    HIPCHK(c->tcounts.reserve(1));
+    auto &tl = c->tl;
+    if (tl.empty())
+        tl.resize(1);
+    if ((st = tree_level_view(tl[0], 1)))
+        return st;
+    HIPCHK(tree_init(c->tposi.p, n, w, c->tcounts.p, root_sub ? nullptr : &tl[0].v, c->tsub.p, sm));
+    TreeCounts h;
+    h.nsub = root_sub ? 1 : 0;
+    h.misfit = 0;
+    int last = -1;
+    if (!root_sub) {
+        long long known = 1;                   // segments of level l
+        for (int l = 0;;) {
+            int group = 1;
+            if (subs) {
+                group = 3;
+                if (l == 0)
+                    while ((n >> (group - 2)) > gmax)
+                        ++group;
+            }
+            group = std::min(group, 1024 - l);
+            if (group <= 0)
+                return fail(PP2P_ERR_ARG, "tree deeper than 1024 levels (many coincident particles?)");
+            if ((int)tl.size() < l + group + 1)
+                tl.resize(l + group + 1);
+            auto cap = [&](int k) { return std::min(cap_all, k - l < 40 ? known << (k - l) : cap_all); };
+            auto tiles = [&](int k) { return n / kTreeTile + cap(k); };
+            for (int k = l + 1; k <= l + group; ++k)
+                if ((st = tree_level_view(tl[k], (size_t)cap(k))))
+                    return st;
+            const size_t nt = (size_t)tiles(l + group - 1);
+            HIPCHK(c->tmask.reserve(nt * (kTreeTile / 64)));
+            HIPCHK(c->ttcnt.reserve(nt));
+            HIPCHK(c->ttmap.reserve(nt));
+            for (int k = l; k < l + group; ++k)
+                HIPCHK(tree_level(w, tl[k].v, tl[k + 1].v, k, (int)cap(k), tiles(k), int2pos, maxleaf, gmax,
+                                  c->tmask.p, c->ttcnt.p, c->ttmap.p, c->tcounts.p, c->tsub.p,
+                                  subs ? (int)subcap : 0, sm));
+            HIPCHK(hipMemcpyAsync(&h, c->tcounts.p, sizeof(int) * (size_t)(2 + l + group + 1), hipMemcpyDeviceToHost,
+                                  sm));
+            HIPCHK(hipStreamSynchronize(sm));
+            if (h.misfit)
+                return PP2P_OK;
+            for (int k = l; k < l + group && last < 0; ++k) {
+                tl[k].nseg = h.nseg[k];
+                if (h.nseg[k + 1] == 0)
+                    last = k;
+            }
+            if (last >= 0)
+                break;
+            l += group;
+            known = h.nseg[l];
+        }
+    }
+    *levels = last + 1;
+    *nsub = h.nsub;
+    HIPCHK(c->tsuboff.reserve(std::max<size_t>((size_t)*nsub * kSubLevels, 1)));
+    HIPCHK(tree_subs(w, c->tsub.p, *nsub, int2pos, maxleaf, c->tsuboff.p, c->tcounts.p, sm));
+    for (int l = last; l >= 0; --l)
+        HIPCHK(tree_below(tl[l].v, tl[l].nseg, l < last ? tl[l + 1].v.below : nullptr, c->tsub.p, sm));
+    HIPCHK(hipMemcpyAsync(&h, c->tcounts.p, 2 * sizeof(int), hipMemcpyDeviceToHost, sm));
+    if (root_sub)
+        HIPCHK(hipMemcpyAsync(counts, &c->tsub.p->nnode, sizeof(int2), hipMemcpyDeviceToHost, sm));
+    else
+        HIPCHK(hipMemcpyAsync(counts, tl[0].v.below, sizeof(int2), hipMemcpyDeviceToHost, sm));
+    HIPCHK(hipStreamSynchronize(sm));
+    *fits = h.misfit == 0;
+    return PP2P_OK;
+}
+
 int pp2p_build_tree(pp2p_ctx *c, long long n, const int *posi, const int *tag, double int2pos, int maxleaf,
                     const float *bdl, const float *bdr, int *nleaf_out, int *nnode_out)
 {
@@ -893,12 +1001,11 @@ int pp2p_build_tree(pp2p_ctx *c, long long n, const int *posi, const int *tag, d
     if (maxleaf < 1 || !(int2pos > 0.0) || std::isinf(int2pos))
         return fail(PP2P_ERR_ARG, "invalid maxleaf or int2pos");
     const hipStream_t sm = c->stream;
+    c->tree_ready = false;                      // the build's arrays are the tree's
     HIPCHK(c->tposi.reserve(3 * n));
     HIPCHK(c->ttag.reserve(n));
-    for (DevBuf<int> *b : {&c->tx0, &c->tx1, &c->tx2, &c->tidx, &c->tsegof, &c->ttbl})
+    for (DevBuf<int> *b : {&c->tx0, &c->tx1, &c->tx2, &c->tidx, &c->tla, &c->tlb, &c->tlc, &c->tld})
         HIPCHK(b->reserve(n));
-    HIPCHK(c->tsmall.reserve(n + 1));
-    HIPCHK(c->tsx.reserve(n + 1));
     {
         const size_t np3 = 3 * (size_t)n;
         HIPCHK(c->h_stage.reserve(sizeof(int) * (np3 + (size_t)n)));
@@ -909,72 +1016,18 @@ int pp2p_build_tree(pp2p_ctx *c, long long n, const int *posi, const int *tag, d
             std::memcpy(stage + sizeof(int) * u0, tag + u0, sizeof(int) * (u1 - u0));
         }));
     }
-    int *const xs[3] = {c->tx0.p, c->tx1.p, c->tx2.p};
-    const TreeScratch w{{c->tx0.p, c->tx1.p, c->tx2.p}, c->tidx.p, c->tsegof.p, c->tsmall.p, c->tsx.p, c->ttbl.p};
-    HIPCHK(tree_init(c->tposi.p, n, xs, c->tidx.p, c->tsegof.p, sm));
-    auto &tl = c->tl;
-    if (tl.empty())
-        tl.resize(1);
-    HIPCHK(tl[0].seg.reserve(1));
-    const int2 root = make_int2(0, (int)n);
-    HIPCHK(hipMemcpyAsync(tl[0].seg.p, &root, sizeof(int2), hipMemcpyHostToDevice, sm));
-    tl[0].nseg = 1;
-    // levels: split every segment, then its sons become the next level or leaves
-    int last = 0;
-    for (int l = 0;; ++l) {
-        if (l >= 1024)
-            return fail(PP2P_ERR_ARG, "tree deeper than 1024 levels (many coincident particles?)");
-        HIPCHK(hipStreamSynchronize(sm));      // nothing in flight while buffers grow
-        auto &L = tl[l];
-        const int ns = L.nseg;
-        HIPCHK(L.mean.reserve(ns));
-        HIPCHK(L.split.reserve(ns));
-        HIPCHK(L.np0.reserve(ns));
-        HIPCHK(L.kk.reserve(ns));
-        HIPCHK(L.kid.reserve(ns));
-        for (DevBuf<int> *b : {&c->tnodef, &c->tleaff, &c->tnoff, &c->tloff})
-            HIPCHK(b->reserve(2 * (size_t)ns + 1));
-        size_t t1 = 0, t2 = 0;
-        HIPCHK(tree_split(w, L.seg.p, ns, l % 3, int2pos, n, nullptr, nullptr, nullptr, nullptr, nullptr, &t1, sm));
-        HIPCHK(tree_children(L.seg.p, ns, nullptr, maxleaf, nullptr, nullptr, nullptr, nullptr, nullptr, &t2, sm));
-        if ((st = ensure_temp(c, std::max(t1, t2))))
-            return st;
-        t1 = t2 = c->temp.cap;
-        HIPCHK(tree_split(w, L.seg.p, ns, l % 3, int2pos, n, L.mean.p, L.split.p, L.np0.p, L.kk.p, c->temp.p, &t1,
-                          sm));
-        HIPCHK(tree_children(L.seg.p, ns, L.np0.p, maxleaf, c->tnodef.p, c->tleaff.p, c->tnoff.p, c->tloff.p,
-                             c->temp.p, &t2, sm));
-        int tot[2] = {0, 0};
-        HIPCHK(hipMemcpyAsync(&tot[0], c->tnoff.p + 2 * ns, sizeof(int), hipMemcpyDeviceToHost, sm));
-        HIPCHK(hipMemcpyAsync(&tot[1], c->tloff.p + 2 * ns, sizeof(int), hipMemcpyDeviceToHost, sm));
-        HIPCHK(hipStreamSynchronize(sm));
-        if ((int)tl.size() < l + 2)
-            tl.resize(l + 2);
-        auto &N = tl[l + 1];
-        HIPCHK(N.seg.reserve(std::max(tot[0], 1)));
-        HIPCHK(tl[l].leaf.reserve(std::max(tot[1], 1)));
-        N.nseg = tot[0];
-        tl[l].nleaf = tot[1];
-        HIPCHK(tree_next(w, tl[l].seg.p, ns, tl[l].np0.p, c->tnodef.p, c->tnoff.p, c->tloff.p, N.seg.p, tl[l].leaf.p,
-                         tl[l].kid.p, n, sm));
-        if (tot[0] == 0) {
-            last = l;
-            break;
-        }
-    }
-    HIPCHK(hipStreamSynchronize(sm));
-    // subtree sizes, deepest level first
-    for (int l = last; l >= 0; --l) {
-        HIPCHK(tl[l].below.reserve(tl[l].nseg));
-        HIPCHK(tl[l].idb.reserve(tl[l].nseg));
-        HIPCHK(tl[l].lo.reserve(tl[l].nseg));
-        HIPCHK(tl[l].hi.reserve(tl[l].nseg));
-    }
-    for (int l = last; l >= 0; --l)
-        HIPCHK(tree_below(tl[l].kid.p, tl[l].nseg, l < last ? tl[l + 1].below.p : nullptr, tl[l].below.p, sm));
-    int2 counts;
-    HIPCHK(hipMemcpyAsync(&counts, tl[0].below.p, sizeof(int2), hipMemcpyDeviceToHost, sm));
-    HIPCHK(hipStreamSynchronize(sm));
+    const TreeScratch w{{c->tx0.p, c->tx1.p, c->tx2.p}, c->tidx.p, c->tla.p, c->tlb.p, c->tlc.p, c->tld.p};
+    int levels = 0, nsub = 0;
+    int2 counts = make_int2(0, 0);
+    bool fits = false;
+    // segments of up to kSubMax particles become subtrees; should one not fit
+    // its workgroup (more nodes than particles, which empty sons of coincident
+    // coordinates can give), every level runs over the device
+    if ((st = tree_split_all(c, w, n, int2pos, maxleaf, std::max(maxleaf, kSubMax), &levels, &nsub, &counts, &fits)))
+        return st;
+    if (!fits &&
+        (st = tree_split_all(c, w, n, int2pos, maxleaf, maxleaf, &levels, &nsub, &counts, &fits)))
+        return st;
     const int nnode = counts.x, nleaf = counts.y;
     // ids and boxes, root first
     HIPCHK(c->wson.reserve(nnode));
@@ -985,27 +1038,22 @@ int pp2p_build_tree(pp2p_ctx *c, long long n, const int *posi, const int *tag, d
     HIPCHK(c->wact.reserve(nleaf));
     HIPCHK(c->rng.reserve(nleaf));
     HIPCHK(c->x3.reserve(3 * n));
-    const int2 idb0 = make_int2(0, 0);
     const float4 lo0 = make_float4(bdl[0], bdl[1], bdl[2], 0.f), hi0 = make_float4(bdr[0], bdr[1], bdr[2], 0.f);
-    HIPCHK(hipMemcpyAsync(tl[0].idb.p, &idb0, sizeof(int2), hipMemcpyHostToDevice, sm));
-    HIPCHK(hipMemcpyAsync(tl[0].lo.p, &lo0, sizeof(float4), hipMemcpyHostToDevice, sm));
-    HIPCHK(hipMemcpyAsync(tl[0].hi.p, &hi0, sizeof(float4), hipMemcpyHostToDevice, sm));
+    auto &tl = c->tl;
+    HIPCHK(tree_root(levels > 0 ? &tl[0].v : nullptr, c->tsub.p, lo0, hi0, sm));
     const TreeOut out{c->wson.p, c->wnc.p, c->wnw.p, c->wlc.p, c->wlw.p, c->rng.p, c->wact.p};
-    auto view = [&](int l) {
-        if (l > last)
-            return TreeLevelView{0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-        auto &L = tl[l];
-        return TreeLevelView{L.nseg, L.kid.p, L.leaf.p, L.split.p, L.below.p, L.idb.p, L.lo.p, L.hi.p};
-    };
-    for (int l = 0; l <= last; ++l)
-        HIPCHK(tree_place(view(l), view(l + 1), l % 3, out, sm));
+    for (int l = 0; l < levels; ++l)
+        HIPCHK(tree_place(tl[l].v, tl[l].nseg, l + 1 < levels ? tl[l + 1].v : TreeLevelView{}, l % 3, c->tsub.p, out,
+                          sm));
+    HIPCHK(tree_place_subs(w, c->tsub.p, nsub, out, sm));
     HIPCHK(tree_finish(w, out, nleaf, c->ttag.p, int2pos, n, c->x3.p, sm));
     if ((st = finish_particles(c, n, nleaf)))
         return st;
     c->walk_nnode = nnode;
     c->tree_ready = true;
     c->tree_int2pos = int2pos;
-    c->tree_levels = last + 1;
+    c->tree_levels = levels;
+    c->tree_nsub = nsub;
     c->fmm_ready = false;
     c->walk_m2l_n = -1;
     if (nleaf_out)
@@ -1232,8 +1280,9 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
     // upward: P2M of the leaves, M2M level by level from the deepest
     HIPCHK(launch_cell_centers(t, c->mcenter.p, sm));
     HIPCHK(launch_p2m(t, (float)c->params.mass, c->mM.p, sm));
+    HIPCHK(launch_m2m_subs(t, c->tsub.p, c->tree_nsub, c->tsuboff.p, c->tla.p, c->mM.p, sm));
     for (int l = c->tree_levels - 1; l >= 0; --l)
-        HIPCHK(launch_m2m_level(t, c->tl[l].idb.p, c->tl[l].nseg, c->mM.p, sm));
+        HIPCHK(launch_m2m_level(t, c->tl[l].v.idb, c->tl[l].nseg, c->mM.p, sm));
     HIPCHK(launch_zero_f32(c->mL.p, 20 * ncell, sm));
     HIPCHK(hipEventRecord(e1, sm));
     HIPCHK(hipEventSynchronize(e1));
@@ -1254,7 +1303,8 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
     // downward: L2L level by level from the root, then L2P into the accumulator
     HIPCHK(hipEventRecord(e0, sm));
     for (int l = 0; l < c->tree_levels; ++l)
-        HIPCHK(launch_l2l_level(t, c->tl[l].idb.p, c->tl[l].nseg, c->mL.p, sm));
+        HIPCHK(launch_l2l_level(t, c->tl[l].v.idb, c->tl[l].nseg, c->mL.p, sm));
+    HIPCHK(launch_l2l_subs(t, c->tsub.p, c->tree_nsub, c->tsuboff.p, c->tla.p, c->mL.p, sm));
     const L2PArgs a{c->rng.p, c->wlc.p, c->mL.p, c->x3.p, nleaf, c->npart, c->acc.p};
     HIPCHK(launch_l2p(a, sm));
     HIPCHK(hipEventRecord(e1, sm));

@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "p2p_tree.h"
+
 namespace pp2p {
 
 // M2L over the target CSR of a task list: row r adds the translations of
@@ -42,6 +44,11 @@ hipError_t launch_p2m(const FmmTree &t, float mass, float *M, hipStream_t st);
 // one level's nodes (idb[s].x = node id): M2M from their sons / L2L into them
 hipError_t launch_m2m_level(const FmmTree &t, const int2 *idb, int nseg, float *M, hipStream_t st);
 hipError_t launch_l2l_level(const FmmTree &t, const int2 *idb, int nseg, float *L, hipStream_t st);
+// the subtrees' nodes, all levels (off: level offsets, ids: node ids by breadth-first number)
+hipError_t launch_m2m_subs(const FmmTree &t, const TreeSub *sub, int nsub, const unsigned short *off, const int *ids,
+                           float *M, hipStream_t st);
+hipError_t launch_l2l_subs(const FmmTree &t, const TreeSub *sub, int nsub, const unsigned short *off, const int *ids,
+                           float *L, hipStream_t st);
 hipError_t launch_cell_centers(const FmmTree &t, float4 *center, hipStream_t st);
 hipError_t launch_zero_f32(float *p, long long n, hipStream_t st);
 hipError_t launch_m2l(const M2LArgs &a, hipStream_t st);

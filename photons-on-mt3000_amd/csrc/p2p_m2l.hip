@@ -278,13 +278,9 @@ __device__ __forceinline__ size_t cell_of(const FmmTree &t, int son)
     return son >= 0 ? (size_t)t.nleaf + son : (size_t)(-son - 1);
 }
 
-// M2M of one level's nodes: M[node] = sum over its two sons, son 0 first
-__global__ __launch_bounds__(kM2LBlock) void k_m2m_level(FmmTree t, const int2 *idb, int nseg, float *M)
+// M2M of node k: M[node] = sum over its two sons, son 0 first
+__device__ __forceinline__ void m2m_node(const FmmTree &t, int k, float *M)
 {
-    const int s = blockIdx.x * kM2LBlock + threadIdx.x;
-    if (s >= nseg)
-        return;
-    const int k = idb[s].x;
     const float4 c = t.node_center[k];
     const int2 son = t.son[k];
     float acc[20];
@@ -304,13 +300,9 @@ __global__ __launch_bounds__(kM2LBlock) void k_m2m_level(FmmTree t, const int2 *
         dst[n] = acc[n];
 }
 
-// L2L of one level's nodes into their sons
-__global__ __launch_bounds__(kM2LBlock) void k_l2l_level(FmmTree t, const int2 *idb, int nseg, float *L)
+// L2L of node k into its sons
+__device__ __forceinline__ void l2l_node(const FmmTree &t, int k, float *L)
 {
-    const int s = blockIdx.x * kM2LBlock + threadIdx.x;
-    if (s >= nseg)
-        return;
-    const int k = idb[s].x;
     const float4 c = t.node_center[k];
     const int2 son = t.son[k];
     float lp[20];
@@ -327,6 +319,50 @@ __global__ __launch_bounds__(kM2LBlock) void k_l2l_level(FmmTree t, const int2 *
         l2l_add(cs.x - c.x, cs.y - c.y, cs.z - c.z, lp, ls);
         for (int n = 0; n < 20; ++n)
             dst[n] = ls[n];
+    }
+}
+
+// one level's nodes
+__global__ __launch_bounds__(kM2LBlock) void k_m2m_level(FmmTree t, const int2 *idb, int nseg, float *M)
+{
+    const int s = blockIdx.x * kM2LBlock + threadIdx.x;
+    if (s < nseg)
+        m2m_node(t, idb[s].x, M);
+}
+
+__global__ __launch_bounds__(kM2LBlock) void k_l2l_level(FmmTree t, const int2 *idb, int nseg, float *L)
+{
+    const int s = blockIdx.x * kM2LBlock + threadIdx.x;
+    if (s < nseg)
+        l2l_node(t, idb[s].x, L);
+}
+
+// The nodes of the subtrees, one block per subtree, its levels (off) from the
+// deepest up (M2M) or from its root down (L2L) with a barrier between them.
+// ids: the subtree's node ids relative to its root's, breadth first (low 12 bits).
+constexpr int kSubNodesBlock = 128;
+
+__global__ __launch_bounds__(kSubNodesBlock) void k_m2m_subs(FmmTree t, const TreeSub *sub,
+                                                           const unsigned short *off, const int *ids, float *M)
+{
+    const TreeSub &s = sub[blockIdx.x];
+    off += (size_t)blockIdx.x * kSubLevels;
+    for (int l = s.nlev - 1; l >= 0; --l) {
+        for (int i = off[l] + (int)threadIdx.x; i < off[l + 1]; i += kSubNodesBlock)
+            m2m_node(t, s.id + (ids[s.start + i] & 0xfff), M);
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kSubNodesBlock) void k_l2l_subs(FmmTree t, const TreeSub *sub,
+                                                           const unsigned short *off, const int *ids, float *L)
+{
+    const TreeSub &s = sub[blockIdx.x];
+    off += (size_t)blockIdx.x * kSubLevels;
+    for (int l = 0; l < s.nlev; ++l) {
+        for (int i = off[l] + (int)threadIdx.x; i < off[l + 1]; i += kSubNodesBlock)
+            l2l_node(t, s.id + (ids[s.start + i] & 0xfff), L);
+        __syncthreads();
     }
 }
 
@@ -385,6 +421,22 @@ hipError_t launch_l2l_level(const FmmTree &t, const int2 *idb, int nseg, float *
 {
     if (nseg > 0)
         k_l2l_level<<<blocks(nseg), kM2LBlock, 0, st>>>(t, idb, nseg, L);
+    return hipGetLastError();
+}
+
+hipError_t launch_m2m_subs(const FmmTree &t, const TreeSub *sub, int nsub, const unsigned short *off, const int *ids,
+                           float *M, hipStream_t st)
+{
+    if (nsub > 0)
+        k_m2m_subs<<<(unsigned)nsub, kSubNodesBlock, 0, st>>>(t, sub, off, ids, M);
+    return hipGetLastError();
+}
+
+hipError_t launch_l2l_subs(const FmmTree &t, const TreeSub *sub, int nsub, const unsigned short *off, const int *ids,
+                           float *L, hipStream_t st)
+{
+    if (nsub > 0)
+        k_l2l_subs<<<(unsigned)nsub, kSubNodesBlock, 0, st>>>(t, sub, off, ids, L);
     return hipGetLastError();
 }
 

@@ -1,14 +1,17 @@
 // The kd-tree on the device: build_localtree's mean-split tree
 // (src/fmm.c:168-270), its boxes (center_kdtree, src/fmm.c:273-327) and the
-// target marking (src/fmm.c:1226-1236), built level by level instead of
-// recursively, with the reference's numbering and particle order.
+// target marking (src/fmm.c:1226-1236), with the reference's numbering and
+// particle order.
 //
-// Level l holds the nodes at depth l as particle ranges (segments), left to
-// right; all split along coordinate l % 3.  Per level:
-//   mean    one thread per segment sums the sampled coordinates in FP64 in
-//           the reference's order (stride len / 100000 above 10^5
-//           particles), so the split is the reference's to the bit
-//   flags   small = coordinate <= mean; an exclusive scan counts them
+// Segments (particle ranges) of more than kSubMax particles are split level by
+// level over the whole device, the smaller ones each by one workgroup that
+// keeps its particles in LDS and builds the whole subtree below them.  All
+// segments at depth l split along coordinate l % 3.  A split:
+//   mean    the sampled coordinates summed in FP64 in the reference's order
+//           (stride len / 100000 above 10^5 particles), so the split is the
+//           reference's to the bit; the additions run in parallel where their
+//           rounding allows it (p2p_seqsum.h)
+//   small   coordinate <= mean, as bit masks with their counts
 //   swaps   the reference's in-place partition (src/fmm.c:199-219) scans
 //           from the left for particles above the mean and swaps each with
 //           the next particle at or below it from the right.  Its outcome
@@ -18,16 +21,12 @@
 //           gets k particles, or len - 1 when every particle is at or below
 //           the mean (the scan then stops one short).  Two particles are
 //           ordered by a plain compare (src/fmm.c:180-187).
-//   children  sons with more than maxleaf particles are the next level's
-//           segments, the others are leaves (scans keep both in order)
+//   sons    more than maxleaf particles: a segment or subtree; else a leaf
 // Afterwards the subtree sizes are summed bottom-up and the depth-first ids
 // (nodes in creation order, leaves in creation order) and boxes handed
 // top-down.  FP64 sums and FP32 boxes are rounded per operation (no
 // contraction), as the host code computes them.
-#include <cstring>
-
-#include <rocprim/rocprim.hpp>
-
+#include "p2p_seqsum.h"
 #include "p2p_tree.h"
 
 #pragma clang fp contract(off)
@@ -42,69 +41,263 @@ inline unsigned grid_of(long long n) { return (unsigned)((n + kTreeBlock - 1) / 
 __device__ __forceinline__ long long gid() { return (long long)blockIdx.x * kTreeBlock + threadIdx.x; }
 
 __global__ __launch_bounds__(kTreeBlock) void k_tree_init(const int *__restrict__ posi, long long n,
-                                                        int *__restrict__ x0, int *__restrict__ x1,
-                                                        int *__restrict__ x2, int *__restrict__ idx,
-                                                        int *__restrict__ segof)
+                                                        TreeScratch w, TreeCounts *counts, TreeLevelView root,
+                                                        TreeSub *sub)
 {
     const long long i = gid();
+    if (i == 0) {
+        counts->nsub = sub ? 1 : 0;
+        counts->misfit = 0;
+        counts->nseg[0] = sub ? 0 : 1;
+        if (sub) {
+            sub[0].start = 0;
+            sub[0].len = (int)n;
+            sub[0].depth = 0;
+        } else {
+            root.seg[0] = make_int2(0, (int)n);
+            root.toff[0] = 0;
+            root.toff[1] = (int)((n + kTreeTile - 1) / kTreeTile);
+        }
+    }
     if (i >= n)
         return;
-    x0[i] = posi[3 * i];
-    x1[i] = posi[3 * i + 1];
-    x2[i] = posi[3 * i + 2];
-    idx[i] = (int)i;
-    segof[i] = 0;
+    w.x[0][i] = posi[3 * i];
+    w.x[1][i] = posi[3 * i + 1];
+    w.x[2][i] = posi[3 * i + 2];
+    w.idx[i] = (int)i;
 }
 
-// Split value of each segment (src/fmm.c:168-197): the sampled FP64 mean for
-// more than two particles, the midpoint of two, 0 for fewer.  One wave per
-// segment: the lanes load 512 samples at a time into the wave's LDS slice,
-// and every lane adds them to its sum one after the other in sample order
-// (the same chain in every lane, each value a broadcast LDS read), so the sum
-// is the reference's sequential one.  Padding the last block with +0.0
-// leaves the sum unchanged: it is never -0.0 (it starts at +0.0 and an exact
-// cancellation rounds to +0.0).
-constexpr int kMeanBatch = 512;
+// ------------------------------------------------------------- exact sums
 
-__global__ __launch_bounds__(kTreeBlock) void k_tree_mean(const int2 *__restrict__ seg, int nseg,
-                                                        const int *__restrict__ x, double int2pos,
-                                                        double *__restrict__ mean, float *__restrict__ split)
+__device__ __forceinline__ double lane_value(double v, int k)
 {
-    __shared__ double buf[kTreeBlock / 64][kMeanBatch];
-    const int s = blockIdx.x * (kTreeBlock / 64) + threadIdx.x / 64;
-    const int lane = threadIdx.x & 63;
-    if (s >= nseg)
+    const unsigned long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, k);
+    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), k);
+    return __longlong_as_double(((unsigned long long)hi << 32) | lo);
+}
+
+// Inclusive prefix sum over the wave by DPP (rows of 16, then the rows' totals
+// handed on): six steps of two moves and an addition.  The same by
+// __shfl_up (two LDS permutes per step) made the sums of the means three times
+// as long.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double v)
+{
+    const unsigned long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, ROWS, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, ROWS, 0xf, true);
+    return __longlong_as_double(((unsigned long long)hi << 32) | lo);
+}
+
+__device__ __forceinline__ double wave_prefix(double v)
+{
+    v += dpp_or_zero<0x111, 0xf>(v);                 // row_shr 1, 2, 4, 8
+    v += dpp_or_zero<0x112, 0xf>(v);
+    v += dpp_or_zero<0x114, 0xf>(v);
+    v += dpp_or_zero<0x118, 0xf>(v);
+    v += dpp_or_zero<0x142, 0xa>(v);                 // row_bcast 15 into rows 1 and 3
+    v += dpp_or_zero<0x143, 0xc>(v);                 // row_bcast 31 into rows 2 and 3
+    return v;
+}
+
+__device__ __forceinline__ double wave_sum(double v) { return lane_value(wave_prefix(v), 63); }
+
+// A lane's kV consecutive values as units of s's binade: their sums by sign,
+// and their round-ups, which are zero without a halfway case.
+template <int kV>
+__device__ __forceinline__ SeqTies lane_units(const double (&v)[kV], double scale, double &up, double &down)
+{
+    SeqTies run;
+    up = down = 0.0;
+#pragma unroll
+    for (int u = 0; u < kV; ++u) {
+        bool half;
+        const double r = seq_units(v[u], scale, half);
+        up += r > 0.0 ? r : 0.0;
+        down += r < 0.0 ? -r : 0.0;
+        run.out ^= seq_odd(r);
+        if (half) {
+            (run.any ? run.rest : run.first) += run.out;
+            run.any = 1;
+            run.out = 0;
+        }
+    }
+    return run;
+}
+
+// Parity before each lane's run when it is p before the first lane's; `all`
+// (the same in every lane) becomes the runs of all lanes as one, but for its
+// rest, which is each lane's share.
+__device__ __forceinline__ int lanes_parity(const SeqTies &run, int p, int lane, SeqTies &all)
+{
+    const unsigned long long outs = __ballot(run.out), any = __ballot(run.any);
+    const unsigned long long upto = ~0ull >> (63 - lane);
+    const int c = __popcll(outs & upto) & 1;         // parity of the outs up to and with this lane's
+    all.out = __popcll(outs) & 1;
+    if (!any) {
+        all.any = all.first = all.rest = 0;
+        return p ^ c ^ run.out;
+    }
+    const unsigned long long cs = __ballot(c), prev = any & (upto >> 1);
+    // outs of the lanes after the last halfway case's, and its own parity
+    auto since = [&](int k) { return (int)(cs >> k) ^ (int)(outs >> k); };
+    const int l = 63 - __clzll(any), f = __builtin_ctzll(any);
+    const int before = prev ? (c ^ run.out ^ since(63 - __clzll(prev))) & 1 : p ^ c ^ run.out;
+    const int first = __builtin_amdgcn_readlane(run.first, f) ^ ((int)((cs ^ outs) >> f) & 1);
+    all.any = 1;
+    all.first = first & 1;                           // with parity 0 before the first lane
+    all.rest = run.any ? run.rest + (lane != f ? run.first ^ before : 0) : 0;
+    all.out = (all.out ^ since(l)) & 1;
+    return before;
+}
+
+// s + a wave's 64 kV values, lane l's before lane l + 1's, the same in every
+// lane.  A pass adds the lanes up to the first whose values may leave the sum's
+// binade by one prefix sum, then that lane's one after the other.  A sum from zero
+// starts with eight lanes' values one after the other, where the binades are
+// short.
+template <int kV>
+__device__ double add_run(double s, const double (&v)[kV], int lane)
+{
+    auto serial = [&](int l) {
+#pragma unroll
+        for (int u = 0; u < kV; ++u)
+            s += lane_value(v[u], l);
+    };
+    int next = 0;
+    while (next < 64) {
+        const double scale = seq_scale(s);
+        if (scale == 0.0) {
+            const int e = next == 0 ? 8 : next + 1;
+            for (; next < e; ++next)
+                serial(next);
+            continue;
+        }
+        double up, down;
+        SeqTies run = lane_units(v, s < 0.0 ? -scale : scale, up, down), all;
+        if (lane < next) {
+            up = down = 0.0;
+            run = SeqTies();
+        }
+        if (__ballot(run.any)) {
+            int p = lanes_parity(run, seq_parity(s), lane, all);
+            up += (double)seq_roundups(run, p);
+        }
+        const double S = fabs(s) * scale, inc = up - down;
+        const double t = wave_prefix(inc);
+        const unsigned long long bad = __ballot(!seq_inside(S + (t - inc), up, down)) & (~0ull << next);
+        const int first = bad ? __builtin_ctzll(bad) : 64;
+        if (first > next) {
+            const double m = (S + lane_value(t, first - 1)) * seq_unit(scale);
+            s = s < 0.0 ? -m : m;
+        }
+        if (first < 64)
+            serial(first);
+        next = first + 1;
+    }
+    return s;
+}
+
+// ------------------------------------------------------------- level passes
+
+// Split value of each segment (src/fmm.c:168-197): the sampled FP64 mean for
+// more than two particles, the midpoint of two, 0 for fewer.  One block per
+// segment; the samples come 4096 at a time, the next ones loading meanwhile.
+// Each wave turns its 512 values into integers and round-ups, which every thread
+// then adds in wave order.  What bounds it: a chain of batches, each the latency of 4096 scattered
+// samples (stride up to n / 10^5).  Adding the samples one after the other, as
+// before, was a chain of dependent FP64 additions of about 19 cycles: 433 us
+// per level on the 256^3 clustered tree (1.9 10^7 particles).
+constexpr int kMeanThreads = 512;
+constexpr int kMeanValues = 8;
+constexpr int kMeanBatch = kMeanThreads * kMeanValues;
+
+__global__ __launch_bounds__(kMeanThreads) void k_tree_mean(TreeLevelView lv, const int *__restrict__ nseg,
+                                                          const int *__restrict__ x, double int2pos)
+{
+    constexpr int kWaves = kMeanThreads / 64;
+    __shared__ double2 sums[kWaves];
+    __shared__ int4 runs[kWaves];                    // SeqTies of each wave
+    __shared__ double s_sum;
+    const int s = blockIdx.x;
+    if (s >= *nseg)
         return;
-    double *wb = buf[threadIdx.x / 64];
-    const int a = seg[s].x, len = seg[s].y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int a = lv.seg[s].x, len = lv.seg[s].y;
     double m = 0.0;
     float sp = 0.0f;
     if (len > 2) {
         const long long mul = len > 100000 ? len / 100000 : 1;
-        const long long ns = (len + mul - 1) / mul;
-        constexpr int kU = kMeanBatch / 64;
-        for (long long b = 0; b < ns; b += kMeanBatch) {
-            // indices past the end are clamped for the load and masked after
-            int r[kU];
+        const int ns = (int)((len + mul - 1) / mul);
+        int r[kMeanValues];
+        // a thread's values are consecutive
+        auto at = [&](int u) { return (int)threadIdx.x * kMeanValues + u; };
+        auto load = [&](int b) {
 #pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                const long long k = b + u * 64 + lane;
+            for (int u = 0; u < kMeanValues; ++u) {
+                const int k = b + at(u);
                 r[u] = x[a + (k < ns ? k : ns - 1) * mul];
             }
+        };
+        load(0);
+        for (int b = 0; b < ns; b += kMeanBatch) {
+            double v[kMeanValues];
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
-                wb[u * 64 + lane] = b + u * 64 + lane < ns ? int2pos * (double)r[u] : 0.0;
-            __builtin_amdgcn_wave_barrier();
-            const int cnt = ns - b < kMeanBatch ? (int)(ns - b) : kMeanBatch;     // the same in every lane
-            int j = 0;
-            for (; j + 16 <= cnt; j += 16) {
-#pragma unroll
-                for (int q = 0; q < 16; ++q)
-                    m += wb[j + q];
+            for (int u = 0; u < kMeanValues; ++u)
+                v[u] = b + at(u) < ns ? int2pos * (double)r[u] : 0.0;
+            if (b + kMeanBatch < ns)
+                load(b + kMeanBatch);
+            // the waves' values in turn: all that keep the sum in its binade at
+            // once, then the wave that does not by itself, then on with the rest
+            int next = 0;
+            while (next < kWaves) {
+                const double scale = seq_scale(m);
+                __syncthreads();                     // the previous pass's reads
+                if (scale != 0.0 && wave >= next) {
+                    double up, down;
+                    const SeqTies run = lane_units(v, m < 0.0 ? -scale : scale, up, down);
+                    SeqTies all;
+                    if (__ballot(run.any)) {
+                        lanes_parity(run, 0, lane, all);
+                        for (int o = 32; o > 0; o >>= 1)
+                            all.rest += __shfl_xor(all.rest, o, 64);
+                    } else {
+                        all.out = __popcll(__ballot(run.out)) & 1;
+                    }
+                    up = wave_sum(up);
+                    down = wave_sum(down);
+                    if (lane == 0) {
+                        sums[wave] = make_double2(up, down);
+                        runs[wave] = make_int4(all.any, all.first, all.rest, all.out);
+                    }
+                }
+                __syncthreads();
+                if (scale != 0.0) {
+                    double S = fabs(m) * scale;
+                    int p = seq_parity(m);
+                    for (; next < kWaves; ++next) {
+                        const double2 ud = sums[next];
+                        const int4 q = runs[next];
+                        const double up = ud.x + (double)seq_roundups(SeqTies{q.x, q.y, q.z, q.w}, p);
+                        if (!seq_inside(S, up, ud.y))
+                            break;
+                        S = S + up - ud.y;
+                    }
+                    const double t = S * seq_unit(scale);
+                    m = m < 0.0 ? -t : t;
+                }
+                if (next < kWaves) {
+                    if (wave == next) {
+                        const double t = add_run(m, v, lane);
+                        if (lane == 0)
+                            s_sum = t;
+                    }
+                    __syncthreads();
+                    m = s_sum;
+                    ++next;
+                }
             }
-            for (; j < cnt; ++j)
-                m += wb[j];
-            __builtin_amdgcn_wave_barrier();
         }
         m /= (double)len;
         m *= (double)mul;
@@ -112,189 +305,603 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_mean(const int2 *__restrict
     } else if (len == 2) {
         sp = (float)(0.5 * (int2pos * (double)(x[a] + x[a + 1])));
     }
+    if (threadIdx.x == 0) {
+        lv.mean[s] = m;
+        lv.split[s] = sp;
+    }
+}
+
+// the segment holding a tile: the last s with toff[s] <= tile
+__device__ __forceinline__ int seg_of_tile(const int *__restrict__ toff, int nseg, int tile)
+{
+    int lo = 0, hi = nseg - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (toff[mid] <= tile)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+// Masks of the particles at or below the mean, 64 words and their total per
+// tile of kTreeTile positions of one segment; tmap[tile] = the segment.
+__global__ __launch_bounds__(kTreeBlock) void k_tree_flags(TreeLevelView lv, const int *__restrict__ nseg,
+                                                         const int *__restrict__ x, double int2pos,
+                                                         unsigned long long *__restrict__ mask,
+                                                         int *__restrict__ tcnt, int *__restrict__ tmap)
+{
+    __shared__ int part[kTreeBlock / 64];
+    const int ns = *nseg, tile = blockIdx.x;
+    if (ns == 0 || tile >= lv.toff[ns])
+        return;
+    const int s = seg_of_tile(lv.toff, ns, tile);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int2 sg = lv.seg[s];
+    const double mean = lv.mean[s];
+    const int base = (tile - lv.toff[s]) * kTreeTile;     // offset of the tile in its segment
+    constexpr int kWords = kTreeTile / kTreeBlock;        // words per wave
+    int r[kWords];
+#pragma unroll
+    for (int u = 0; u < kWords; ++u) {
+        const int p = base + (wave * kWords + u) * 64 + lane;
+        r[u] = p < sg.y ? x[sg.x + p] : 0;
+    }
+    int cnt = 0;
+    unsigned long long keep = 0;
+#pragma unroll
+    for (int u = 0; u < kWords; ++u) {
+        const int p = base + (wave * kWords + u) * 64 + lane;
+        const unsigned long long m = __ballot(p < sg.y && sg.y > 2 && !(int2pos * (double)r[u] > mean));
+        if (lane == u)
+            keep = m;
+        cnt += __popcll(m);
+    }
+    if (lane < kWords)
+        mask[(long long)tile * (kTreeTile / 64) + wave * kWords + lane] = keep;
+    if (lane == 0)
+        part[wave] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int q = 0; q < kTreeBlock / 64; ++q)
+            t += part[q];
+        tcnt[tile] = t;
+        tmap[tile] = s;
+    }
+}
+
+// The misplaced particles of each segment by rank: la[a + r] = the r-th
+// particle above the mean in the left part, lb[a + r] = the r-th at or below it
+// counted from the end of the right part; the left son's size and the
+// number of swaps.  A tile finds the counts before it by summing the tile
+// counts of its segment (at most n / 4096 integers from L2).
+__global__ __launch_bounds__(kTreeBlock) void k_tree_lists(TreeLevelView lv, const int *__restrict__ nseg,
+                                                         const int *__restrict__ x,
+                                                         const unsigned long long *__restrict__ mask,
+                                                         const int *__restrict__ tcnt,
+                                                         const int *__restrict__ tmap, int *__restrict__ la,
+                                                         int *__restrict__ lb)
+{
+    constexpr int kWords = kTreeTile / 64;
+    __shared__ int before_s[kTreeBlock / 64], total_s[kTreeBlock / 64];
+    __shared__ unsigned long long word[kWords];
+    __shared__ int wpre[kWords];
+    const int ns = *nseg, tile = blockIdx.x;
+    if (ns == 0 || tile >= lv.toff[ns])
+        return;
+    const int s = tmap[tile];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int a = lv.seg[s].x, len = lv.seg[s].y;
+    const int t0 = lv.toff[s], t1 = lv.toff[s + 1];
+    if (len <= 2) {                                  // one tile
+        if (threadIdx.x == 0) {
+            const bool sw = len == 2 && x[a] > x[a + 1];
+            lv.left[s] = len == 2 ? 1 : 0;
+            lv.swaps[s] = sw;
+            if (sw) {
+                la[a] = a;
+                lb[a] = a + 1;
+            }
+        }
+        return;
+    }
+    int before = 0, total = 0;
+    for (int t = t0 + (int)threadIdx.x; t < t1; t += kTreeBlock) {
+        const int c = tcnt[t];
+        total += c;
+        before += t < tile ? c : 0;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        before += __shfl_xor(before, o, 64);
+        total += __shfl_xor(total, o, 64);
+    }
     if (lane == 0) {
-        mean[s] = m;
-        split[s] = sp;
+        before_s[wave] = before;
+        total_s[wave] = total;
+    }
+    if (wave == 0) {
+        const unsigned long long m = mask[(long long)tile * kWords + lane];
+        const int c = __popcll(m);
+        int inc = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o, 64);
+            if (lane >= o)
+                inc += u;
+        }
+        word[lane] = m;
+        wpre[lane] = inc - c;
+    }
+    __syncthreads();
+    before = total = 0;
+    for (int q = 0; q < kTreeBlock / 64; ++q) {
+        before += before_s[q];
+        total += total_s[q];
+    }
+    if (total == len) {
+        if (tile == t0 && threadIdx.x == 0) {
+            lv.left[s] = len - 1;
+            lv.swaps[s] = 0;
+        }
+        return;
+    }
+    const int k = total;
+    if (tile == t0 && threadIdx.x == 0)
+        lv.left[s] = k;
+    const int base = (tile - t0) * kTreeTile;
+    for (int o = threadIdx.x; o < kTreeTile; o += kTreeBlock) {
+        const int p = base + o;
+        if (p >= len)
+            break;
+        const unsigned long long m = word[o >> 6];
+        const int sb = before + wpre[o >> 6] + __popcll(m & ((1ull << (o & 63)) - 1ull));   // small ones before p
+        const bool small = (m >> (o & 63)) & 1ull;
+        if (p == k)
+            lv.swaps[s] = k - sb;                    // k < len here: exactly one thread of the segment
+        if (p < k && !small)
+            la[a + (p - sb)] = a + p;
+        else if (p >= k && small)
+            lb[a + (k - sb - 1)] = a + p;
     }
 }
 
-__global__ __launch_bounds__(kTreeBlock) void k_tree_flags(const int *__restrict__ x, const int *__restrict__ segof,
-                                                         const int2 *__restrict__ seg,
-                                                         const double *__restrict__ mean, double int2pos,
-                                                         long long n, int *__restrict__ small)
+__device__ __forceinline__ void swap_part(int *x0, int *x1, int *x2, int *idx, int i, int j)
 {
-    const long long i = gid();
-    if (i >= n)
-        return;
-    const int s = segof[i];
-    int f = 0;
-    if (s >= 0 && seg[s].y > 2)
-        f = !(int2pos * (double)x[i] > mean[s]);
-    small[i] = f;
-}
-
-__global__ void k_tree_scan_end(int *__restrict__ sx, const int *__restrict__ v, long long n)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        sx[n] = sx[n - 1] + v[n - 1];
-}
-
-// Left child size np0 and the pairing bound kk (-1: no swaps) per segment.
-__global__ __launch_bounds__(kTreeBlock) void k_tree_count(const int2 *__restrict__ seg, int nseg,
-                                                         const int *__restrict__ sx, int *__restrict__ np0,
-                                                         int *__restrict__ kk)
-{
-    const long long s = gid();
-    if (s >= nseg)
-        return;
-    const int a = seg[s].x, len = seg[s].y;
-    int left = len == 2 ? 1 : 0, k = -1;
-    if (len > 2) {
-        const int sm = sx[a + len] - sx[a];
-        left = sm == len ? len - 1 : sm;
-        k = sm == len ? -1 : sm;
-    }
-    np0[s] = left;
-    kk[s] = k;
-}
-
-// tbl[a + r] = position of the r-th particle at or below the mean counted
-// from the end of the right part [a + k, a + len).
-__global__ __launch_bounds__(kTreeBlock) void k_tree_table(const int *__restrict__ segof,
-                                                         const int2 *__restrict__ seg, const int *__restrict__ kk,
-                                                         const int *__restrict__ small, const int *__restrict__ sx,
-                                                         long long n, int *__restrict__ tbl)
-{
-    const long long i = gid();
-    if (i >= n)
-        return;
-    const int s = segof[i];
-    if (s < 0 || !small[i])
-        return;
-    const int k = kk[s];
-    const int a = seg[s].x, len = seg[s].y;
-    if (k < 0 || i < a + k)
-        return;
-    tbl[a + (sx[a + len] - sx[i + 1])] = (int)i;
-}
-
-__device__ __forceinline__ void swap_part(int *x0, int *x1, int *x2, int *idx, long long i, long long j)
-{
-    int t = x0[i]; x0[i] = x0[j]; x0[j] = t;
-    t = x1[i]; x1[i] = x1[j]; x1[j] = t;
-    t = x2[i]; x2[i] = x2[j]; x2[j] = t;
-    t = idx[i]; idx[i] = idx[j]; idx[j] = t;
+    const int a0 = x0[i], a1 = x1[i], a2 = x2[i], a3 = idx[i];
+    const int b0 = x0[j], b1 = x1[j], b2 = x2[j], b3 = idx[j];
+    x0[i] = b0; x1[i] = b1; x2[i] = b2; idx[i] = b3;
+    x0[j] = a0; x1[j] = a1; x2[j] = a2; idx[j] = a3;
 }
 
 // The partition's swaps, in place: each swapped pair belongs to one thread.
-__global__ __launch_bounds__(kTreeBlock) void k_tree_swap(int *__restrict__ x0, int *__restrict__ x1,
-                                                        int *__restrict__ x2, int *__restrict__ idx, int dir,
-                                                        const int *__restrict__ segof,
-                                                        const int2 *__restrict__ seg, const int *__restrict__ kk,
-                                                        const int *__restrict__ small, const int *__restrict__ sx,
-                                                        const int *__restrict__ tbl, long long n)
+// Bound by HBM: 32 B read and written per pair and 8 B of lists; the level passes
+// together took 363 us per level on the 256^3 clustered tree when each ran
+// over every particle with its segment looked up per particle.
+__global__ __launch_bounds__(kTreeBlock) void k_tree_swap(TreeLevelView lv, const int *__restrict__ nseg,
+                                                        const int *__restrict__ tmap, TreeScratch w)
 {
-    const long long i = gid();
-    if (i >= n)
+    const int ns = *nseg, tile = blockIdx.x;
+    if (ns == 0 || tile >= lv.toff[ns])
         return;
-    const int s = segof[i];
-    if (s < 0)
-        return;
-    const int a = seg[s].x, len = seg[s].y;
-    if (len == 2) {
-        if (i == a) {
-            const int *x = dir == 0 ? x0 : dir == 1 ? x1 : x2;
-            if (x[a] > x[a + 1])
-                swap_part(x0, x1, x2, idx, a, a + 1);
+    const int s = tmap[tile];
+    const int a = lv.seg[s].x, r0 = (tile - lv.toff[s]) * kTreeTile;
+    const int r1 = min(r0 + kTreeTile, lv.swaps[s]);
+    for (int r = r0 + (int)threadIdx.x; r < r1; r += kTreeBlock)
+        swap_part(w.x[0], w.x[1], w.x[2], w.idx, w.la[a + r], w.lb[a + r]);
+}
+
+// The sons of a level, in order: the next level's segments with their tile
+// offsets, the new subtrees, this level's leaves.  One block: a level holds at
+// most n / kSubMax segments.
+constexpr int kNextBlock = 1024;
+
+__global__ __launch_bounds__(kNextBlock) void k_tree_next(TreeLevelView lv, TreeLevelView nx, int level, int maxleaf,
+                                                        int gmax, TreeCounts *counts, TreeSub *sub, int subcap)
+{
+    __shared__ int4 wtot[kNextBlock / 64];
+    const int ns = counts->nseg[level];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int4 base = make_int4(0, counts->nsub, 0, 0);    // next segments, subtrees, leaves, tiles
+    __syncthreads();                                 // every thread has read nsub before it changes
+    for (int b = 0; b < ns; b += kNextBlock) {
+        const int s = b + (int)threadIdx.x;
+        int rs[2] = {0, 0}, rn[2] = {0, 0}, kind[2] = {-1, -1};
+        int4 c = make_int4(0, 0, 0, 0);
+        if (s < ns) {
+            const int2 sg = lv.seg[s];
+            const int l = lv.left[s];
+            rs[0] = sg.x; rn[0] = l;
+            rs[1] = sg.x + l; rn[1] = sg.y - l;
+            for (int h = 0; h < 2; ++h) {
+                kind[h] = rn[h] > gmax ? 0 : rn[h] > maxleaf ? 1 : 2;
+                c.x += kind[h] == 0;
+                c.y += kind[h] == 1;
+                c.z += kind[h] == 2;
+                c.w += kind[h] == 0 ? (rn[h] + kTreeTile - 1) / kTreeTile : 0;
+            }
         }
-        return;
+        int4 inc = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int4 u = make_int4(__shfl_up(inc.x, o, 64), __shfl_up(inc.y, o, 64), __shfl_up(inc.z, o, 64),
+                                     __shfl_up(inc.w, o, 64));
+            if (lane >= o) {
+                inc.x += u.x; inc.y += u.y; inc.z += u.z; inc.w += u.w;
+            }
+        }
+        if (lane == 63)
+            wtot[wave] = inc;
+        __syncthreads();
+        int4 at = make_int4(base.x + inc.x - c.x, base.y + inc.y - c.y, base.z + inc.z - c.z, base.w + inc.w - c.w);
+        for (int q = 0; q < kNextBlock / 64; ++q) {
+            const int4 t = wtot[q];
+            if (q < wave) {
+                at.x += t.x; at.y += t.y; at.z += t.z; at.w += t.w;
+            }
+            base.x += t.x; base.y += t.y; base.z += t.z; base.w += t.w;
+        }
+        __syncthreads();                             // wtot is rewritten by the next chunk
+        if (s < ns) {
+            int code[2];
+            for (int h = 0; h < 2; ++h) {
+                const int2 rg = make_int2(rs[h], rn[h]);
+                if (kind[h] == 0) {
+                    nx.seg[at.x] = rg;
+                    nx.toff[at.x] = at.w;
+                    at.w += (rn[h] + kTreeTile - 1) / kTreeTile;
+                    code[h] = at.x++;
+                } else if (kind[h] == 1) {
+                    if (at.y < subcap) {
+                        sub[at.y].start = rg.x;
+                        sub[at.y].len = rg.y;
+                        sub[at.y].depth = level + 1;
+                    } else {
+                        counts->misfit = 1;
+                    }
+                    code[h] = kSubKid + at.y++;
+                } else {
+                    lv.leaf[at.z] = rg;
+                    code[h] = -at.z++ - 1;
+                }
+            }
+            lv.kid[s] = make_int2(code[0], code[1]);
+        }
     }
-    const int k = kk[s];
-    if (k < 0 || i >= a + k || small[i])
-        return;
-    const int rb = (int)(i - a) - (sx[i] - sx[a]);
-    swap_part(x0, x1, x2, idx, i, tbl[a + rb]);
+    if (threadIdx.x == 0) {
+        counts->nsub = base.y < subcap ? base.y : subcap;
+        counts->nseg[level + 1] = base.x;
+        nx.toff[base.x] = base.w;
+    }
 }
 
-// nodef/leaff[2s + c]: son c of segment s is a node / a leaf.
-__global__ __launch_bounds__(kTreeBlock) void k_tree_kidflags(const int2 *__restrict__ seg, int nseg,
-                                                            const int *__restrict__ np0, int maxleaf,
-                                                            int *__restrict__ nodef, int *__restrict__ leaff)
+// ------------------------------------------------------------- subtrees
+
+// A whole subtree of at most kSubMax particles by one workgroup, the particles
+// in LDS from the first split to the last.  Per level: the means (one thread
+// per segment when there are many, one wave per segment with the parallel sums
+// otherwise), the masks, the partners, the swaps, the sons.  The nodes are
+// numbered breadth first while they are made and depth first at the end.
+// Bound by the barriers and LDS latencies of about eight levels; it takes the
+// place of as many passes over all particles in HBM.  4096 particles with the
+// records fill one CU's LDS; the next level up costs the device passes less
+// than a second resident workgroup would gain.
+constexpr int kSubBlock = 1024;
+
+struct SubLds {
+    int x[3][kSubMax], idx[kSubMax];
+    unsigned short seg[kSubMax];                     // segment of the position (0xffff: in a leaf)
+    unsigned short partner[kSubMax];
+    unsigned long long mask[kSubMax / 64];
+    int wpre[kSubMax / 64 + 1];
+    unsigned short beg[2][kSubMax / 2], len[2][kSubMax / 2];
+    double mean[kSubMax / 2];
+    unsigned short left[kSubMax / 2], k[kSubMax / 2];    // k = 0xffff: no swaps
+    short kid[2][kSubMax];                           // by node, breadth first: node >= 0, leaf -(q + 1)
+    unsigned short lbeg[kSubMax], llen[kSubMax];     // leaves in creation order
+    int nnext, nleaf, misfit;
+};
+static_assert(sizeof(SubLds) <= 160 * 1024, "one CU's LDS");
+// the numbering reuses the particles' space
+struct SubNumber {
+    unsigned short nodes[kSubMax], leaves[kSubMax];  // below each node
+    unsigned short id[kSubMax], leaf0[kSubMax];
+    unsigned short up[kSubMax];                      // parent << 1 | side
+};
+static_assert(sizeof(SubNumber) <= sizeof(SubLds::x), "numbering overlaps more than the coordinates");
+
+__device__ __forceinline__ int sub_small_before(const SubLds &m, int p)
 {
-    const long long s = gid();
-    if (s >= nseg)
-        return;
-    const int np[2] = {np0[s], seg[s].y - np0[s]};
-    for (int c = 0; c < 2; ++c) {
-        nodef[2 * s + c] = np[c] > maxleaf;
-        leaff[2 * s + c] = np[c] <= maxleaf;
-    }
-    if (s == nseg - 1) {
-        // a trailing zero: the scans' last entries are the totals
-        nodef[2 * s + 2] = 0;
-        leaff[2 * s + 2] = 0;
-    }
+    const int w = p >> 6;
+    return m.wpre[w] + ((p & 63) ? __popcll(m.mask[w] & ((1ull << (p & 63)) - 1ull)) : 0);
 }
 
-// The next level's segments, this level's leaves, and kid[s] = the two sons
-// (>= 0: next-level segment, < 0: this level's leaf -(q + 1)).
-__global__ __launch_bounds__(kTreeBlock) void k_tree_next(const int2 *__restrict__ seg, int nseg,
-                                                        const int *__restrict__ np0, const int *__restrict__ nodef,
-                                                        const int *__restrict__ noff, const int *__restrict__ loff,
-                                                        int2 *__restrict__ next, int2 *__restrict__ leaf,
-                                                        int2 *__restrict__ kid)
+__global__ __launch_bounds__(kSubBlock) void k_tree_sub(TreeScratch w, TreeSub *__restrict__ sub, double int2pos,
+                                                      int maxleaf, unsigned short *__restrict__ off_all,
+                                                      TreeCounts *counts)
 {
-    const long long s = gid();
-    if (s >= nseg)
-        return;
-    const int a = seg[s].x, len = seg[s].y, l0 = np0[s];
-    int r[2];
-    for (int c = 0; c < 2; ++c) {
-        const int2 rg = c ? make_int2(a + l0, len - l0) : make_int2(a, l0);
-        if (nodef[2 * s + c]) {
-            next[noff[2 * s + c]] = rg;
-            r[c] = noff[2 * s + c];
+    __shared__ SubLds m;
+    TreeSub &me = sub[blockIdx.x];
+    unsigned short *off = off_all + (size_t)blockIdx.x * kSubLevels;
+    const int start = me.start, n = me.len, depth = me.depth;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int i = tid; i < kSubMax; i += kSubBlock) {
+        const bool in = i < n;
+        m.x[0][i] = in ? w.x[0][start + i] : 0;
+        m.x[1][i] = in ? w.x[1][start + i] : 0;
+        m.x[2][i] = in ? w.x[2][start + i] : 0;
+        m.idx[i] = in ? w.idx[start + i] : 0;
+        m.seg[i] = in ? 0 : 0xffff;
+    }
+    if (tid == 0) {
+        m.beg[0][0] = 0;
+        m.len[0][0] = (unsigned short)n;
+        m.nleaf = 0;
+        m.misfit = 0;
+        off[0] = 0;
+    }
+    __syncthreads();
+    int nseg = 1, first = 0, lev = 0, cur = 0;       // first: breadth-first number of the level's first node
+    // nodes and leaves have room for as many as the subtree has particles
+    while (nseg > 0) {
+        const int axis = (depth + lev) % 3;
+        const int *x = m.x[axis];
+        const unsigned short *beg = m.beg[cur], *slen = m.len[cur];
+        // means and split values
+        if (nseg >= 48) {
+            for (int s = tid; s < nseg; s += kSubBlock) {
+                const int b = beg[s], l = slen[s];
+                double sum = 0.0;
+                float sp = 0.0f;
+                if (l > 2) {
+                    int j = 0;
+                    for (; j + 8 <= l; j += 8) {
+                        int r[8];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q)
+                            r[q] = x[b + j + q];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q)
+                            sum += int2pos * (double)r[q];
+                    }
+                    for (; j < l; ++j)
+                        sum += int2pos * (double)x[b + j];
+                    sum /= (double)l;
+                    sp = (float)sum;
+                } else if (l == 2) {
+                    sp = (float)(0.5 * (int2pos * (double)(x[b] + x[b + 1])));
+                }
+                m.mean[s] = sum;
+                w.lc[start + first + s] = __float_as_int(sp);
+            }
         } else {
-            leaf[loff[2 * s + c]] = rg;
-            r[c] = -loff[2 * s + c] - 1;
+            for (int s = wave; s < nseg; s += kSubBlock / 64) {
+                const int b = beg[s], l = slen[s];
+                double sum = 0.0;
+                float sp = 0.0f;
+                if (l > 2) {
+                    for (int c = 0; c < l; c += 512) {
+                        double v[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            const int j = c + lane * 8 + u;
+                            v[u] = j < l ? int2pos * (double)x[b + (j < l ? j : 0)] : 0.0;
+                        }
+                        sum = add_run(sum, v, lane);
+                    }
+                    sum /= (double)l;
+                    sp = (float)sum;
+                } else if (l == 2) {
+                    sp = (float)(0.5 * (int2pos * (double)(x[b] + x[b + 1])));
+                }
+                if (lane == 0) {
+                    m.mean[s] = sum;
+                    w.lc[start + first + s] = __float_as_int(sp);
+                }
+            }
         }
+        if (tid == 0)
+            m.nnext = 0;
+        __syncthreads();
+        // masks of the particles at or below the mean
+#pragma unroll
+        for (int u = 0; u < kSubMax / kSubBlock; ++u) {
+            const int wd = wave * (kSubMax / kSubBlock) + u, i = wd * 64 + lane;
+            const int s = m.seg[i];
+            const bool f = s != 0xffff && slen[s == 0xffff ? 0 : s] > 2 &&
+                           !(int2pos * (double)x[i] > m.mean[s == 0xffff ? 0 : s]);
+            const unsigned long long b = __ballot(f);
+            if (lane == 0)
+                m.mask[wd] = b;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int c = __popcll(m.mask[lane]);
+            int inc = c;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(inc, o, 64);
+                if (lane >= o)
+                    inc += u;
+            }
+            m.wpre[lane] = inc - c;
+            if (lane == 63)
+                m.wpre[64] = inc;
+        }
+        __syncthreads();
+        auto before = [&](int p) { return p == kSubMax ? m.wpre[64] : sub_small_before(m, p); };
+        for (int s = tid; s < nseg; s += kSubBlock) {
+            const int b = beg[s], l = slen[s];
+            int left = l == 2 ? 1 : 0, k = 0xffff;
+            if (l > 2) {
+                const int sm = before(b + l) - before(b);
+                left = sm == l ? l - 1 : sm;
+                k = sm == l ? 0xffff : sm;
+            }
+            m.left[s] = (unsigned short)left;
+            m.k[s] = (unsigned short)k;
+        }
+        __syncthreads();
+        // partners from the right part
+        for (int i = tid; i < n; i += kSubBlock) {
+            const int s = m.seg[i];
+            if (s == 0xffff || m.k[s] == 0xffff || !((m.mask[i >> 6] >> (i & 63)) & 1ull))
+                continue;
+            const int b = beg[s];
+            if (i >= b + m.k[s])
+                m.partner[b + (m.k[s] - (before(i + 1) - before(b)))] = (unsigned short)i;
+        }
+        __syncthreads();
+        for (int i = tid; i < n; i += kSubBlock) {
+            const int s = m.seg[i];
+            if (s == 0xffff)
+                continue;
+            const int b = beg[s];
+            int j = -1;
+            if (slen[s] == 2) {
+                if (i == b && x[b] > x[b + 1])
+                    j = b + 1;
+            } else if (m.k[s] != 0xffff && i < b + m.k[s] && !((m.mask[i >> 6] >> (i & 63)) & 1ull)) {
+                j = m.partner[b + (i - b) - (before(i) - before(b))];
+            }
+            if (j >= 0)
+                swap_part(m.x[0], m.x[1], m.x[2], m.idx, i, j);
+        }
+        // sons: their breadth-first numbers in any order
+        const int nfirst = first + nseg;
+        for (int s = tid; s < nseg; s += kSubBlock) {
+            const int b = beg[s], l = slen[s], left = m.left[s];
+            for (int h = 0; h < 2; ++h) {
+                const int cb = h ? b + left : b, cl = h ? l - left : left;
+                int code = 0;
+                if (cl > maxleaf) {
+                    const int k = atomicAdd(&m.nnext, 1);
+                    if (nfirst + k < n) {
+                        m.beg[cur ^ 1][k] = (unsigned short)cb;
+                        m.len[cur ^ 1][k] = (unsigned short)cl;
+                        code = nfirst + k;
+                    } else {
+                        m.misfit = 1;
+                    }
+                } else {
+                    const int q = atomicAdd(&m.nleaf, 1);
+                    if (q < n) {
+                        m.lbeg[q] = (unsigned short)cb;
+                        m.llen[q] = (unsigned short)cl;
+                        code = -q - 1;
+                    } else {
+                        m.misfit = 1;
+                    }
+                }
+                m.kid[h][first + s] = (short)code;
+            }
+        }
+        __syncthreads();
+        if (m.misfit || lev + 1 >= kSubLevels || depth + lev + 1 >= kSubLevels) {
+            // more nodes than particles (empty sons) or too deep: not a
+            // subtree that fits here; the same decision in every thread
+            if (tid == 0) {
+                me.nnode = -1;
+                counts->misfit = 1;
+            }
+            return;
+        }
+        for (int i = tid; i < n; i += kSubBlock) {
+            const int s = m.seg[i];
+            if (s == 0xffff)
+                continue;
+            const int c = m.kid[i >= beg[s] + m.left[s]][first + s];
+            m.seg[i] = c >= 0 ? (unsigned short)(c - nfirst) : 0xffff;
+        }
+        ++lev;
+        if (tid == 0)
+            off[lev] = (unsigned short)nfirst;
+        nseg = m.nnext;
+        first = nfirst;
+        cur ^= 1;
+        __syncthreads();
     }
-    kid[s] = make_int2(r[0], r[1]);
+    for (int i = tid; i < n; i += kSubBlock) {
+        w.x[0][start + i] = m.x[0][i];
+        w.x[1][start + i] = m.x[1][i];
+        w.x[2][start + i] = m.x[2][i];
+        w.idx[start + i] = m.idx[i];
+    }
+    __syncthreads();
+    // depth-first numbers: sizes bottom-up, ids top-down, level by level
+    SubNumber &q = *reinterpret_cast<SubNumber *>(&m.x[0][0]);
+    for (int l = lev - 1; l >= 0; --l) {
+        const int b = off[l], e = off[l + 1];
+        for (int i = b + tid; i < e; i += kSubBlock) {
+            int nn = 1, nl = 0;
+            for (int h = 0; h < 2; ++h) {
+                const int c = m.kid[h][i];
+                nn += c >= 0 ? q.nodes[c] : 0;
+                nl += c >= 0 ? q.leaves[c] : 1;
+            }
+            q.nodes[i] = (unsigned short)nn;
+            q.leaves[i] = (unsigned short)nl;
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        q.id[0] = q.leaf0[0] = q.up[0] = 0;
+        me.nnode = q.nodes[0];
+        me.nleaf = q.leaves[0];
+        me.nlev = lev;
+    }
+    __syncthreads();
+    for (int l = 0; l < lev; ++l) {
+        const int b = off[l], e = off[l + 1];
+        for (int i = b + tid; i < e; i += kSubBlock) {
+            int id = q.id[i] + 1, lf = q.leaf0[i];
+            int son[2];
+            for (int h = 0; h < 2; ++h) {
+                const int c = m.kid[h][i];
+                if (c >= 0) {
+                    q.id[c] = (unsigned short)id;
+                    q.leaf0[c] = (unsigned short)lf;
+                    q.up[c] = (unsigned short)(i << 1 | h);
+                    son[h] = id;
+                    id += q.nodes[c];
+                    lf += q.leaves[c];
+                } else {
+                    w.ld[start + lf] = m.lbeg[-c - 1] | m.llen[-c - 1] << 16;
+                    son[h] = -lf - 1;
+                    ++lf;
+                }
+            }
+            w.la[start + i] = q.id[i] | q.up[i] << 12;
+            w.lb[start + i] = (son[0] & 0xffff) | son[1] << 16;
+        }
+        __syncthreads();
+    }
 }
 
-__global__ __launch_bounds__(kTreeBlock) void k_tree_segof(int *__restrict__ segof, const int2 *__restrict__ seg,
-                                                         const int *__restrict__ np0, const int2 *__restrict__ kid,
-                                                         long long n)
-{
-    const long long i = gid();
-    if (i >= n)
-        return;
-    const int s = segof[i];
-    if (s < 0)
-        return;
-    const int k = i >= seg[s].x + np0[s] ? kid[s].y : kid[s].x;
-    segof[i] = k >= 0 ? k : -1;
-}
-
+// ------------------------------------------------------------- placement
 // below[s] = (nodes, leaves) in the subtree of segment s.
-__global__ __launch_bounds__(kTreeBlock) void k_tree_below(const int2 *__restrict__ kid, int nseg,
+__global__ __launch_bounds__(kTreeBlock) void k_tree_below(TreeLevelView lv, int nseg,
                                                          const int2 *__restrict__ below_next,
-                                                         int2 *__restrict__ below)
+                                                         const TreeSub *__restrict__ sub)
 {
     const long long s = gid();
     if (s >= nseg)
         return;
-    const int k[2] = {kid[s].x, kid[s].y};
+    const int k[2] = {lv.kid[s].x, lv.kid[s].y};
     int nb = 1, lb = 0;
     for (int c = 0; c < 2; ++c) {
-        if (k[c] >= 0) {
+        if (k[c] >= kSubKid) {
+            nb += sub[k[c] - kSubKid].nnode;
+            lb += sub[k[c] - kSubKid].nleaf;
+        } else if (k[c] >= 0) {
             nb += below_next[k[c]].x;
             lb += below_next[k[c]].y;
         } else {
             lb += 1;
         }
     }
-    below[s] = make_int2(nb, lb);
+    lv.below[s] = make_int2(nb, lb);
 }
 
 __device__ __forceinline__ void set_dim(float4 &v, int dir, float x)
@@ -307,63 +914,129 @@ __device__ __forceinline__ void set_dim(float4 &v, int dir, float x)
         v.z = x;
 }
 
+__device__ __forceinline__ float get_dim(const float4 &v, int dir) { return dir == 0 ? v.x : dir == 1 ? v.y : v.z; }
+
+__device__ __forceinline__ float4 box_width(const float4 &lo, const float4 &hi)
+{
+    return make_float4(hi.x - lo.x, hi.y - lo.y, hi.z - lo.z, 0.f);
+}
+
+__device__ __forceinline__ float4 box_center(const float4 &lo, const float4 &hi)
+{
+    return make_float4((float)(0.5 * (double)(hi.x + lo.x)), (float)(0.5 * (double)(hi.y + lo.y)),
+                       (float)(0.5 * (double)(hi.z + lo.z)), 0.f);
+}
+
+// Leaf l, son c of a node with box [lo, hi] split at sp along dir.
+__device__ __forceinline__ void place_leaf(const TreeOut &out, int l, int2 rg, int c, float4 lo, float4 hi, int dir,
+                                           float sp)
+{
+    float4 lw = box_width(lo, hi), lc = box_center(lo, hi);
+    const float lod = get_dim(lo, dir), hid = get_dim(hi, dir);
+    if (c == 0) {
+        set_dim(lw, dir, sp - lod);
+        set_dim(lc, dir, (float)(0.5 * (double)(lod + sp)));
+    } else {
+        set_dim(lw, dir, hid - sp);
+        set_dim(lc, dir, (float)(0.5 * (double)(hid + sp)));
+    }
+    out.leaf_rng[l] = rg;
+    out.leaf_width[l] = lw;
+    out.leaf_center[l] = lc;
+}
+
 // Depth-first ids and boxes: node s of this level has id idb[s].x, its
 // subtree's leaves start at idb[s].y, its box is [lo, hi].  Writes the node,
-// its leaf sons, and the ids and boxes of its node sons.
-__global__ __launch_bounds__(kTreeBlock) void k_tree_place(TreeLevelView lv, TreeLevelView nx, int dir,
-                                                         TreeOut out)
+// its leaf sons, and the ids and boxes of its node and subtree sons.
+__global__ __launch_bounds__(kTreeBlock) void k_tree_place(TreeLevelView lv, int nseg, TreeLevelView nx, int dir,
+                                                         TreeSub *__restrict__ sub, TreeOut out)
 {
     const long long s = gid();
-    if (s >= lv.nseg)
+    if (s >= nseg)
         return;
-    const int I = lv.idb[s].x, B = lv.idb[s].y;
+    int id = lv.idb[s].x, lf = lv.idb[s].y;
     const float4 lo = lv.lo[s], hi = lv.hi[s];
-    const float w[3] = {hi.x - lo.x, hi.y - lo.y, hi.z - lo.z};
-    const float cc[3] = {(float)(0.5 * (double)(hi.x + lo.x)), (float)(0.5 * (double)(hi.y + lo.y)),
-                         (float)(0.5 * (double)(hi.z + lo.z))};
-    out.node_width[I] = make_float4(w[0], w[1], w[2], 0.f);
-    out.node_center[I] = make_float4(cc[0], cc[1], cc[2], 0.f);
+    const int I = id;
+    out.node_width[I] = box_width(lo, hi);
+    out.node_center[I] = box_center(lo, hi);
     const int k[2] = {lv.kid[s].x, lv.kid[s].y};
     const float sp = lv.split[s];
-    int id[2], base[2];
-    id[0] = I + 1;
-    base[0] = B;
-    if (k[0] >= 0) {
-        id[1] = I + 1 + nx.below[k[0]].x;
-        base[1] = B + nx.below[k[0]].y;
-    } else {
-        id[1] = I + 1;
-        base[1] = B + 1;
-    }
-    const float lod = dir == 0 ? lo.x : dir == 1 ? lo.y : lo.z;
-    const float hid = dir == 0 ? hi.x : dir == 1 ? hi.y : hi.z;
     int son[2];
+    ++id;
     for (int c = 0; c < 2; ++c) {
-        if (k[c] >= 0) {
-            float4 clo = lo, chi = hi;
-            set_dim(c == 0 ? chi : clo, dir, sp);
-            nx.idb[k[c]] = make_int2(id[c], base[c]);
+        if (k[c] < 0) {
+            place_leaf(out, lf, lv.leaf[-k[c] - 1], c, lo, hi, dir, sp);
+            son[c] = -lf - 1;
+            ++lf;
+            continue;
+        }
+        float4 clo = lo, chi = hi;
+        set_dim(c == 0 ? chi : clo, dir, sp);
+        son[c] = id;
+        if (k[c] >= kSubKid) {
+            TreeSub &t = sub[k[c] - kSubKid];
+            t.id = id;
+            t.leaf0 = lf;
+            t.lo = clo;
+            t.hi = chi;
+            id += t.nnode;
+            lf += t.nleaf;
+        } else {
+            nx.idb[k[c]] = make_int2(id, lf);
             nx.lo[k[c]] = clo;
             nx.hi[k[c]] = chi;
-            son[c] = id[c];
-        } else {
-            const int l = base[c];
-            const int2 rg = lv.leaf[-k[c] - 1];
-            float4 lw = make_float4(w[0], w[1], w[2], 0.f), lc = make_float4(cc[0], cc[1], cc[2], 0.f);
-            if (c == 0) {
-                set_dim(lw, dir, sp - lod);
-                set_dim(lc, dir, (float)(0.5 * (double)(lod + sp)));
-            } else {
-                set_dim(lw, dir, hid - sp);
-                set_dim(lc, dir, (float)(0.5 * (double)(hid + sp)));
-            }
-            out.leaf_rng[l] = rg;
-            out.leaf_width[l] = lw;
-            out.leaf_center[l] = lc;
-            son[c] = -l - 1;
+            id += nx.below[k[c]].x;
+            lf += nx.below[k[c]].y;
         }
     }
     out.son[I] = make_int2(son[0], son[1]);
+}
+
+// The nodes and leaves of the subtrees, one block per subtree and one thread
+// per node: its box is the root's, cut by the nearest split on the way up
+// that bounds each side.
+__global__ __launch_bounds__(kTreeBlock) void k_tree_place_sub(TreeScratch w, const TreeSub *__restrict__ sub,
+                                                             TreeOut out)
+{
+    const TreeSub &t = sub[blockIdx.x];
+    const int start = t.start, nnode = t.nnode;
+    for (int i = threadIdx.x; i < nnode; i += kTreeBlock) {
+        const unsigned a = (unsigned)w.la[start + i];
+        const int lb = w.lb[start + i];
+        // levels above node i in the subtree
+        int lev = 0;
+        for (int p = i; p > 0; p = (int)((unsigned)w.la[start + p] >> 13))
+            ++lev;
+        float4 lo = t.lo, hi = t.hi;
+        unsigned have = 0;                           // bits 0-2: lo set, 3-5: hi set
+        int p = i, dir = (t.depth + lev) % 3;
+        const int mine = dir;
+        while (p > 0 && have != 63u) {
+            const unsigned up = (unsigned)w.la[start + p] >> 12;
+            p = (int)(up >> 1);
+            dir = dir == 0 ? 2 : dir - 1;
+            const unsigned bit = (up & 1u) ? 1u << dir : 8u << dir;     // right son: its lower side
+            if (!(have & bit)) {
+                have |= bit;
+                set_dim((up & 1u) ? lo : hi, dir, __int_as_float(w.lc[start + p]));
+            }
+        }
+        const int I = t.id + (int)(a & 0xfffu);
+        const float sp = __int_as_float(w.lc[start + i]);
+        out.node_width[I] = box_width(lo, hi);
+        out.node_center[I] = box_center(lo, hi);
+        int son[2] = {(int)(short)(lb & 0xffff), lb >> 16};
+        for (int c = 0; c < 2; ++c) {
+            if (son[c] >= 0) {
+                son[c] += t.id;
+            } else {
+                const int q = -son[c] - 1, r = w.ld[start + q], l = t.leaf0 + q;
+                place_leaf(out, l, make_int2(start + (r & 0xffff), (int)((unsigned)r >> 16)), c, lo, hi, mine, sp);
+                son[c] = -l - 1;
+            }
+        }
+        out.son[I] = make_int2(son[0], son[1]);
+    }
 }
 
 // Target marking (src/fmm.c:1226-1236): 0 when the leaf holds a particle
@@ -398,70 +1071,77 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_x3(const int *__restrict__ 
     x3[3 * i + 2] = int2pos * (double)x2[i];
 }
 
+__global__ void k_tree_root(TreeLevelView root, TreeSub *sub, float4 lo, float4 hi)
+{
+    if (threadIdx.x != 0)
+        return;
+    if (sub) {
+        sub->id = sub->leaf0 = 0;
+        sub->lo = lo;
+        sub->hi = hi;
+    } else {
+        root.idb[0] = make_int2(0, 0);
+        root.lo[0] = lo;
+        root.hi[0] = hi;
+    }
+}
+
 }  // namespace
 
-hipError_t tree_init(const int *posi, long long n, int *const x[3], int *idx, int *segof, hipStream_t st)
+hipError_t tree_root(const TreeLevelView *root, TreeSub *sub, float4 lo, float4 hi, hipStream_t st)
 {
-    k_tree_init<<<grid_of(n), kTreeBlock, 0, st>>>(posi, n, x[0], x[1], x[2], idx, segof);
+    k_tree_root<<<1, 64, 0, st>>>(root ? *root : TreeLevelView{}, root ? nullptr : sub, lo, hi);
     return hipGetLastError();
 }
 
-hipError_t tree_split(const TreeScratch &w, const int2 *seg, int nseg, int dir, double int2pos, long long n,
-                      double *mean, float *split, int *np0, int *kk, void *temp, size_t *temp_bytes, hipStream_t st)
+hipError_t tree_init(const int *posi, long long n, const TreeScratch &w, TreeCounts *counts, const TreeLevelView *root,
+                     TreeSub *sub, hipStream_t st)
 {
-    if (!temp)
-        return rocprim::exclusive_scan(nullptr, *temp_bytes, w.small, w.sx, 0, (size_t)n, rocprim::plus<int>(), st);
-    const int *x = w.x[dir];
-    k_tree_mean<<<(unsigned)((nseg + kTreeBlock / 64 - 1) / (kTreeBlock / 64)), kTreeBlock, 0, st>>>(
-        seg, nseg, x, int2pos, mean, split);
-    k_tree_flags<<<grid_of(n), kTreeBlock, 0, st>>>(x, w.segof, seg, mean, int2pos, n, w.small);
-    hipError_t e = rocprim::exclusive_scan(temp, *temp_bytes, w.small, w.sx, 0, (size_t)n, rocprim::plus<int>(), st);
-    if (e != hipSuccess)
-        return e;
-    k_tree_scan_end<<<1, 64, 0, st>>>(w.sx, w.small, n);
-    k_tree_count<<<grid_of(nseg), kTreeBlock, 0, st>>>(seg, nseg, w.sx, np0, kk);
-    k_tree_table<<<grid_of(n), kTreeBlock, 0, st>>>(w.segof, seg, kk, w.small, w.sx, n, w.tbl);
-    k_tree_swap<<<grid_of(n), kTreeBlock, 0, st>>>(w.x[0], w.x[1], w.x[2], w.idx, dir, w.segof, seg, kk, w.small,
-                                                   w.sx, w.tbl, n);
+    k_tree_init<<<grid_of(n), kTreeBlock, 0, st>>>(posi, n, w, counts, root ? *root : TreeLevelView{},
+                                                   root ? nullptr : sub);
     return hipGetLastError();
 }
 
-hipError_t tree_children(const int2 *seg, int nseg, const int *np0, int maxleaf, int *nodef, int *leaff, int *noff,
-                         int *loff, void *temp, size_t *temp_bytes, hipStream_t st)
+hipError_t tree_level(const TreeScratch &w, const TreeLevelView &lv, const TreeLevelView &nx, int level, int cap,
+                      long long tiles, double int2pos, int maxleaf, int gmax, unsigned long long *mask, int *tcnt,
+                      int *tmap, TreeCounts *counts, TreeSub *sub, int subcap, hipStream_t st)
 {
-    if (!temp) {
-        size_t a = 0;
-        hipError_t e = rocprim::exclusive_scan(nullptr, a, nodef, noff, 0, (size_t)2 * nseg + 1,
-                                               rocprim::plus<int>(), st);
-        *temp_bytes = a;
-        return e;
-    }
-    k_tree_kidflags<<<grid_of(nseg), kTreeBlock, 0, st>>>(seg, nseg, np0, maxleaf, nodef, leaff);
-    hipError_t e = rocprim::exclusive_scan(temp, *temp_bytes, nodef, noff, 0, (size_t)2 * nseg + 1,
-                                           rocprim::plus<int>(), st);
-    if (e == hipSuccess)
-        e = rocprim::exclusive_scan(temp, *temp_bytes, leaff, loff, 0, (size_t)2 * nseg + 1, rocprim::plus<int>(),
-                                    st);
-    return e;
-}
-
-hipError_t tree_next(const TreeScratch &w, const int2 *seg, int nseg, const int *np0, const int *nodef,
-                     const int *noff, const int *loff, int2 *next, int2 *leaf, int2 *kid, long long n, hipStream_t st)
-{
-    k_tree_next<<<grid_of(nseg), kTreeBlock, 0, st>>>(seg, nseg, np0, nodef, noff, loff, next, leaf, kid);
-    k_tree_segof<<<grid_of(n), kTreeBlock, 0, st>>>(w.segof, seg, np0, kid, n);
+    const int *ns = &counts->nseg[level];
+    const int *x = w.x[level % 3];
+    const unsigned nt = (unsigned)tiles;
+    k_tree_mean<<<(unsigned)cap, kMeanThreads, 0, st>>>(lv, ns, x, int2pos);
+    k_tree_flags<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, mask, tcnt, tmap);
+    k_tree_lists<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, mask, tcnt, tmap, w.la, w.lb);
+    k_tree_swap<<<nt, kTreeBlock, 0, st>>>(lv, ns, tmap, w);
+    k_tree_next<<<1, kNextBlock, 0, st>>>(lv, nx, level, maxleaf, gmax, counts, sub, subcap);
     return hipGetLastError();
 }
 
-hipError_t tree_below(const int2 *kid, int nseg, const int2 *below_next, int2 *below, hipStream_t st)
+hipError_t tree_subs(const TreeScratch &w, TreeSub *sub, int nsub, double int2pos, int maxleaf, unsigned short *off,
+                     TreeCounts *counts, hipStream_t st)
 {
-    k_tree_below<<<grid_of(nseg), kTreeBlock, 0, st>>>(kid, nseg, below_next, below);
+    if (nsub > 0)
+        k_tree_sub<<<(unsigned)nsub, kSubBlock, 0, st>>>(w, sub, int2pos, maxleaf, off, counts);
     return hipGetLastError();
 }
 
-hipError_t tree_place(const TreeLevelView &lv, const TreeLevelView &nx, int dir, const TreeOut &out, hipStream_t st)
+hipError_t tree_below(const TreeLevelView &lv, int nseg, const int2 *below_next, const TreeSub *sub, hipStream_t st)
 {
-    k_tree_place<<<grid_of(lv.nseg), kTreeBlock, 0, st>>>(lv, nx, dir, out);
+    k_tree_below<<<grid_of(nseg), kTreeBlock, 0, st>>>(lv, nseg, below_next, sub);
+    return hipGetLastError();
+}
+
+hipError_t tree_place(const TreeLevelView &lv, int nseg, const TreeLevelView &nx, int dir, TreeSub *sub,
+                      const TreeOut &out, hipStream_t st)
+{
+    k_tree_place<<<grid_of(nseg), kTreeBlock, 0, st>>>(lv, nseg, nx, dir, sub, out);
+    return hipGetLastError();
+}
+
+hipError_t tree_place_subs(const TreeScratch &w, const TreeSub *sub, int nsub, const TreeOut &out, hipStream_t st)
+{
+    if (nsub > 0)
+        k_tree_place_sub<<<(unsigned)nsub, kTreeBlock, 0, st>>>(w, sub, out);
     return hipGetLastError();
 }
 
