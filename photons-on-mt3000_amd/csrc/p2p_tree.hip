@@ -78,9 +78,9 @@ __device__ __forceinline__ double lane_value(double v, int k)
 }
 
 // Inclusive prefix sum over the wave by DPP (rows of 16, then the rows' totals
-// handed on): six steps of two moves and an addition.  The same by
-// __shfl_up (two LDS permutes per step) made the sums of the means three times
-// as long.
+// handed on): six steps of two moves and an addition.  With __shfl_up (two LDS
+// permutes per step) the subtrees of the 256^3 clustered tree took 3.9 ms
+// instead of 3.3.
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp_or_zero(double v)
 {
@@ -205,10 +205,11 @@ __device__ double add_run(double s, const double (&v)[kV], int lane)
 // more than two particles, the midpoint of two, 0 for fewer.  One block per
 // segment; the samples come 4096 at a time, the next ones loading meanwhile.
 // Each wave turns its 512 values into integers and round-ups, which every thread
-// then adds in wave order.  What bounds it: a chain of batches, each the latency of 4096 scattered
-// samples (stride up to n / 10^5).  Adding the samples one after the other, as
-// before, was a chain of dependent FP64 additions of about 19 cycles: 433 us
-// per level on the 256^3 clustered tree (1.9 10^7 particles).
+// then adds in wave order.  Bound by latency: 25 batches in a row above 10^5
+// particles, and about one more pass per binade.  256^3 clustered tree (1.9 10^7
+// particles, 16 levels): 140 us per level; one wave per segment adding its
+// samples one after the other (about 19 cycles each) took 433 us per level
+// over 23 levels.
 constexpr int kMeanThreads = 512;
 constexpr int kMeanValues = 8;
 constexpr int kMeanBatch = kMeanThreads * kMeanValues;
@@ -583,10 +584,12 @@ __global__ __launch_bounds__(kNextBlock) void k_tree_next(TreeLevelView lv, Tree
 // per segment when there are many, one wave per segment with the parallel sums
 // otherwise), the masks, the partners, the swaps, the sons.  The nodes are
 // numbered breadth first while they are made and depth first at the end.
-// Bound by the barriers and LDS latencies of about eight levels; it takes the
-// place of as many passes over all particles in HBM.  4096 particles with the
-// records fill one CU's LDS; the next level up costs the device passes less
-// than a second resident workgroup would gain.
+// Bound by the latencies of about eight levels (the means first, then seven
+// barriers each); it takes the place of as many passes over all particles in
+// HBM: 3.0 ms for 1.9 10^7 particles (256^3 clustered) where ten levels of
+// device-wide passes took about 8.  4096 particles with the records fill one
+// CU's LDS.  The whole build, uploads included, went from 28.2 to 15.7 ms
+// there, from 4.6 to 1.5 ms at 64^3 and from 1.5 to 0.58 ms at 16^3.
 constexpr int kSubBlock = 1024;
 
 struct SubLds {
