@@ -182,22 +182,18 @@ struct pp2p_ctx {
     DevBuf<unsigned long long> pair_count;
     DevBuf<unsigned char> temp;
 
-    // device walk: the tree, and per round its frames, codes, child offsets
-    // and task offsets (kept for the backward and position passes)
-    struct WalkRound {
-        DevBuf<int2> f;
-        DevBuf<unsigned char> code;
-        DevBuf<unsigned> off;
-        DevBuf<int> x;
-        DevBuf<int> bs, bso;            // well-separated frames per block, their scan
-        long long n = 0;
-    };
+    // device walk: the tree, its cells as the walk reads them, the opened
+    // frames of all rounds (codes, child offsets, task counts) and their tiles
     DevBuf<int2> wson;
     DevBuf<float4> wnc, wnw, wlc, wlw;
     DevBuf<int> wact;
-    std::vector<WalkRound> wr;
-    DevBuf<int> wcnt, wpos_a, wpos_b;
-    DevBuf<unsigned long long> wemit, wsep;
+    DevBuf<WalkCell> wcell;
+    DevBuf<WalkRound> wround;
+    DevBuf<int2> wf;
+    DevBuf<unsigned char> wcode;
+    DevBuf<unsigned> woff;
+    DevBuf<int> wcnt, wsep;
+    DevBuf<unsigned long long> wlook;
     // the walk's well-separated pairs as cells (leaf id, or nleaf + node id)
     DevBuf<int> wm2l_t, wm2l_s;
     long long walk_m2l_n = -1;      // -1: none since the last walk
@@ -321,11 +317,8 @@ void pp2p_destroy(pp2p_ctx *c)
     c->total.release(); c->item_count.release(); c->item_off.release(); c->items_rows.release();
     c->items_q.release(); c->cost.release(); c->cost_sorted.release();
     c->wson.release(); c->wnc.release(); c->wnw.release(); c->wlc.release(); c->wlw.release(); c->wact.release();
-    for (auto &r : c->wr) {
-        r.f.release(); r.code.release(); r.off.release(); r.x.release(); r.bs.release(); r.bso.release();
-    }
-    c->wcnt.release(); c->wpos_a.release(); c->wpos_b.release(); c->wemit.release();
-    c->wsep.release(); c->wm2l_t.release(); c->wm2l_s.release();
+    c->wcell.release(); c->wround.release(); c->wf.release(); c->wcode.release(); c->woff.release();
+    c->wcnt.release(); c->wsep.release(); c->wlook.release(); c->wm2l_t.release(); c->wm2l_s.release();
     for (auto &l : c->tl)
         l.mem.release();
     c->tx0.release(); c->tx1.release(); c->tx2.release(); c->tidx.release(); c->tla.release();
@@ -706,136 +699,151 @@ static int upload_boxes(pp2p_ctx *c, DevBuf<float4> &dst, int n, const float *xy
     return PP2P_OK;
 }
 
+// b with room for n elements, its first `used` (of what it holds) kept.
+extern "C++" {
+template <typename T>
+static hipError_t grow_keep(DevBuf<T> &b, size_t n, size_t used, hipStream_t st)
+{
+    if (n <= b.cap)
+        return hipSuccess;
+    DevBuf<T> nb;
+    hipError_t e = nb.reserve(n);
+    used = std::min(used, b.cap);
+    if (e == hipSuccess && used)
+        e = hipMemcpyAsync(nb.p, b.p, sizeof(T) * used, hipMemcpyDeviceToDevice, st);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+        nb.release();
+        return e;
+    }
+    b.release();
+    b = nb;
+    return hipSuccess;
+}
+}  // extern "C++"
+
+// Room for `frames` frames and `tiles` tiles, the first ones of each kept.
+static int walk_room(pp2p_ctx *c, long long frames, long long keep, long long tiles, long long tkeep, WalkFrames *w)
+{
+    HIPCHK(grow_keep(c->wf, (size_t)frames, (size_t)keep, c->stream));
+    HIPCHK(grow_keep(c->wcode, (size_t)frames, (size_t)keep, c->stream));
+    HIPCHK(grow_keep(c->woff, (size_t)frames, (size_t)keep, c->stream));
+    HIPCHK(grow_keep(c->wcnt, (size_t)frames, 0, c->stream));
+    HIPCHK(grow_keep(c->wlook, (size_t)tiles, 0, c->stream));
+    HIPCHK(grow_keep(c->wsep, (size_t)tiles, (size_t)tkeep, c->stream));
+    const size_t cap = std::min(std::min(c->wf.cap, c->wcode.cap), std::min(c->woff.cap, c->wcnt.cap));
+    *w = WalkFrames{c->wf.p, c->wcode.p, c->woff.p, c->wcnt.p, (long long)cap, c->wlook.p, c->wsep.p,
+                    (long long)std::min(c->wlook.cap, c->wsep.cap)};
+    return PP2P_OK;
+}
+
 // The walk over the tree in the walk arrays (c->walk_nnode nodes, c->nleaf
 // leaves): replaces the context's list.
 static int run_walk(pp2p_ctx *c, float open_angle, float cutoff_radius, long long *ntask)
 {
-    const int nnode = c->walk_nnode;
+    const int nnode = c->walk_nnode, nleaf = c->nleaf;
+    const hipStream_t sm = c->stream;
     int st = PP2P_OK;
-    WalkTree t{c->wson.p, c->wnc.p, c->wnw.p, c->wlc.p, c->wlw.p, c->wact.p, open_angle, cutoff_radius};
+    const WalkTree t{c->wson.p, c->wnc.p, c->wnw.p, c->wlc.p, c->wlw.p, c->wact.p, nnode, nleaf, open_angle,
+                     cutoff_radius};
 
     c->ntask = 0;
     c->csr_ready = c->items_ready = false;
-    auto &wr = c->wr;
-    // forward: the frames of each round
-    if (wr.empty())
-        wr.resize(1);
-    HIPCHK(wr[0].f.reserve(1));
-    const int2 root = nnode > 0 ? make_int2(0, 0) : make_int2(-1, -1);
-    HIPCHK(hipMemcpyAsync(wr[0].f.p, &root, sizeof(int2), hipMemcpyHostToDevice, c->stream));
-    wr[0].n = 1;
-    // per round: frames that emit a task (the list length is their sum) and
-    // well-separated frames (the M2L pairs)
-    HIPCHK(c->wemit.reserve(2 * (size_t)nnode + 4));
-    HIPCHK(c->wsep.reserve(2 * (size_t)nnode + 4));
     c->walk_m2l_n = -1;
-    int last = 0;
-    for (int r = 0;; ++r) {
-        if (r > 2 * nnode + 2)
-            return fail(PP2P_ERR_ARG, "tree walk did not end");
-        const long long n = wr[r].n;
-        // child offsets are 32-bit: a round holds at most 2^29 frames
-        if (n > (1ll << 29))
-            return fail(PP2P_ERR_ARG, "tree walk round larger than 2^29 frames");
-        size_t tb = 0;
-        HIPCHK(walk_code(t, wr[r].f.p, n, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &tb, c->stream));
-        if ((st = ensure_temp(c, tb)))
-            return st;
-        tb = c->temp.cap;
-        HIPCHK(wr[r].code.reserve(n));
-        HIPCHK(wr[r].off.reserve(n + 1));
-        HIPCHK(wr[r].bs.reserve(walk_blocks(n)));
-        HIPCHK(walk_code(t, wr[r].f.p, n, wr[r].code.p, wr[r].off.p, wr[r].bs.p, c->wemit.p + r, c->wsep.p + r,
-                         c->temp.p, &tb, c->stream));
-        unsigned nn = 0;
-        HIPCHK(hipMemcpyAsync(&nn, wr[r].off.p + n, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        if (nn == 0) {
-            last = r;
-            break;
-        }
-        if ((int)wr.size() < r + 2)
-            wr.resize(r + 2);
-        HIPCHK(wr[r + 1].f.reserve(nn));
-        HIPCHK(walk_children(t, wr[r].f.p, n, wr[r].off.p, wr[r + 1].f.p, c->stream));
-        wr[r + 1].n = nn;
-    }
-    std::vector<unsigned long long> em(last + 1), sep(last + 1);
-    HIPCHK(hipMemcpyAsync(em.data(), c->wemit.p, sizeof(unsigned long long) * (last + 1), hipMemcpyDeviceToHost,
-                          c->stream));
-    HIPCHK(hipMemcpyAsync(sep.data(), c->wsep.p, sizeof(unsigned long long) * (last + 1), hipMemcpyDeviceToHost,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    std::vector<WalkRound> rounds;                 // every round with frames
     unsigned long long emitted = 0, nsep = 0;
-    for (int r = 0; r <= last; ++r) {
-        emitted += em[r];
-        nsep += sep[r];
+    WalkFrames w{};
+    if (nnode == 0) {
+        // one leaf: its self pair
+        int act = -1;
+        HIPCHK(hipMemcpyAsync(&act, c->wact.p, sizeof(int), hipMemcpyDeviceToHost, sm));
+        HIPCHK(hipStreamSynchronize(sm));
+        emitted = act >= 0 ? 1 : 0;
+        HIPCHK(c->task_t.reserve(1));
+        HIPCHK(c->task_s.reserve(1));
+        HIPCHK(launch_fill_i32(c->task_t.p, 1, 0, sm));
+        HIPCHK(launch_fill_i32(c->task_s.p, 1, 0, sm));
+    } else {
+        const long long ncell = (long long)nnode + nleaf;
+        HIPCHK(c->wcell.reserve(ncell));
+        HIPCHK(walk_cells(t, c->wcell.p, sm));
+        // Rounds are launched a group at a time (two per level of a balanced
+        // tree first, then a few) and the host reads a group's sizes at once.
+        // A round whose frames outgrow the arrays stops the group; the round
+        // before it runs again with larger ones.
+        int group = 4;
+        for (int l = nleaf; l > 1; l >>= 1)
+            group += 2;
+        WalkRound cur{};                           // the next round to run
+        cur.n = 1;
+        long long need = 256ll * nleaf + 4096;     // frames: about 250 per leaf on the clustered configurations
+        std::vector<WalkRound> h;
+        for (bool more = true; more;) {
+            const long long tiles = std::max(need, (long long)c->wf.cap) / kWalkTile + (long long)rounds.size() + group + 2;
+            if ((st = walk_room(c, need, cur.fbase + cur.n, tiles, cur.tbase, &w)))
+                return st;
+            HIPCHK(c->wround.reserve((size_t)group + 1));
+            HIPCHK(walk_begin(w, c->wround.p, group + 1, cur, sm));
+            for (int k = 0; k < group; ++k) {
+                // a grid for as many frames as the round may hold: 4^r at
+                // most, and a few dozen per cell
+                const int r = (int)rounds.size() + k;
+                const long long most = std::min(r < 16 ? 1ll << (2 * r) : 64 * ncell, 64 * ncell);
+                const int blocks = (int)std::min<long long>((most + kWalkTile - 1) / kWalkTile, 8ll * c->num_cu);
+                HIPCHK(walk_open(t, c->wcell.p, w, c->wround.p + k, blocks, sm));
+            }
+            h.resize((size_t)group + 1);
+            HIPCHK(hipMemcpyAsync(h.data(), c->wround.p, sizeof(WalkRound) * h.size(), hipMemcpyDeviceToHost, sm));
+            HIPCHK(hipStreamSynchronize(sm));
+            for (int k = 0; k <= group; ++k) {
+                if (h[k].n > (1u << 29))
+                    return fail(PP2P_ERR_ARG, "tree walk round larger than 2^29 frames");
+                if (h[k].n == 0) {
+                    more = false;
+                    break;
+                }
+                if (h[k].over) {                   // never the first: round 0 of a group has room
+                    need = std::max(2 * w.cap, h[k].fbase + (long long)h[k].n);
+                    cur = rounds.back();
+                    rounds.pop_back();
+                    break;
+                }
+                cur = h[k];
+                if (k < group)
+                    rounds.push_back(h[k]);
+            }
+            if ((long long)rounds.size() > 2ll * nnode + 2)
+                return fail(PP2P_ERR_ARG, "tree walk did not end");
+            group = 6;
+        }
+        for (const WalkRound &r : rounds) {
+            emitted += r.ntask;
+            nsep += r.nsep;
+        }
     }
-    // the well-separated pairs, round by round in frame order, as cells
     if (nsep > (1ull << 31) - 1)
         return fail(PP2P_ERR_ARG, "more than 2^31-1 well-separated pairs");
-    {
-        size_t tsel = 0;
-        for (int r = 0; r <= last; ++r) {
-            size_t tb = 0;
-            HIPCHK(walk_m2l(nullptr, nullptr, wr[r].n, nullptr, nullptr, 0, nullptr, nullptr, nullptr, &tb,
-                            c->stream));
-            tsel = std::max(tsel, tb);
-            HIPCHK(wr[r].bso.reserve(walk_blocks(wr[r].n)));
-        }
-        if ((st = ensure_temp(c, tsel)))
-            return st;
-        HIPCHK(c->wm2l_t.reserve(std::max<unsigned long long>(nsep, 1)));
-        HIPCHK(c->wm2l_s.reserve(std::max<unsigned long long>(nsep, 1)));
-        unsigned long long o = 0;
-        for (int r = 0; r <= last; ++r) {
-            if (!sep[r])
-                continue;
-            size_t tb = c->temp.cap;
-            HIPCHK(walk_m2l(wr[r].f.p, wr[r].code.p, wr[r].n, wr[r].bs.p, wr[r].bso.p, c->nleaf, c->wm2l_t.p + o,
-                            c->wm2l_s.p + o, c->temp.p, &tb, c->stream));
-            o += sep[r];
-        }
-        c->walk_m2l_n = (long long)nsep;
-    }
     if (emitted > (1ull << 31) - 1)
         return fail(PP2P_ERR_ARG, "more than 2^31-1 tasks in one list");
-    // backward: tasks at and below each frame, last round first (every
-    // buffer the passes share is sized before the first launch)
-    long long nmax = 1;
-    size_t tmax = 0;
-    for (int r = 0; r <= last; ++r) {
-        size_t tb = 0;
-        HIPCHK(walk_below(nullptr, nullptr, nullptr, wr[r].n, nullptr, nullptr, nullptr, &tb, c->stream));
-        tmax = std::max(tmax, tb);
-        nmax = std::max(nmax, wr[r].n);
-        HIPCHK(wr[r].x.reserve(wr[r].n + 1));
+    HIPCHK(c->wm2l_t.reserve(std::max<unsigned long long>(nsep, 1)));
+    HIPCHK(c->wm2l_s.reserve(std::max<unsigned long long>(nsep, 1)));
+    HIPCHK(c->task_t.reserve(std::max<unsigned long long>(emitted, 1)));
+    HIPCHK(c->task_s.reserve(std::max<unsigned long long>(emitted, 1)));
+    if (!rounds.empty()) {
+        for (size_t r = rounds.size(); r-- > 0;)
+            HIPCHK(walk_below(w, rounds[r].fbase, rounds[r].n, sm));
+        HIPCHK(launch_fill_i32(w.cnt, 1, 0, sm));              // the root's first task
+        unsigned long long o = 0;
+        for (const WalkRound &r : rounds) {
+            HIPCHK(walk_emit(t, c->wcell.p, w, r.fbase, r.tbase, r.n, r.nsep, c->task_t.p, c->task_s.p,
+                             c->wm2l_t.p + o, c->wm2l_s.p + o, sm));
+            o += r.nsep;
+        }
     }
-    if ((st = ensure_temp(c, tmax)))
-        return st;
-    HIPCHK(c->wcnt.reserve(nmax));
-    HIPCHK(c->wpos_a.reserve(nmax));
-    HIPCHK(c->wpos_b.reserve(nmax));
-    for (int r = last; r >= 0; --r) {
-        const int *xn = r < last ? wr[r + 1].x.p : nullptr;
-        size_t tb = c->temp.cap;
-        HIPCHK(walk_below(wr[r].code.p, wr[r].off.p, xn, wr[r].n, c->wcnt.p, wr[r].x.p, c->temp.p, &tb, c->stream));
-    }
-    const long long total = (long long)emitted;
-    // positions: first task of each frame, round by round; emitting frames write
-    HIPCHK(c->task_t.reserve(std::max(total, 1ll)));
-    HIPCHK(c->task_s.reserve(std::max(total, 1ll)));
-    const int zero = 0;
-    HIPCHK(hipMemcpyAsync(c->wpos_a.p, &zero, sizeof(int), hipMemcpyHostToDevice, c->stream));
-    DevBuf<int> *pc = &c->wpos_a, *pn = &c->wpos_b;
-    for (int r = 0; r <= last; ++r) {
-        const int *xn = r < last ? wr[r + 1].x.p : nullptr;
-        HIPCHK(walk_emit(wr[r].f.p, wr[r].code.p, wr[r].off.p, xn, wr[r].n, pc->p, r < last ? pn->p : nullptr,
-                         c->task_t.p, c->task_s.p, c->stream));
-        std::swap(pc, pn);
-    }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    c->ntask = total;
+    HIPCHK(hipStreamSynchronize(sm));
+    c->walk_m2l_n = (long long)nsep;
+    c->ntask = (long long)emitted;
     if (ntask)
         *ntask = c->ntask;
     return PP2P_OK;

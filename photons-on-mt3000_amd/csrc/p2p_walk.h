@@ -4,6 +4,9 @@
 
 namespace pp2p {
 
+constexpr int kWalkTile = 256;      // fewest frames per tile of a round
+constexpr int kWalkSmall = 1024;    // most tiles of that size; larger rounds have tiles of 1024 frames
+
 // The kd-tree as the walk reads it.  son[k] = the two children of node k
 // (>= 0: node id, < 0: leaf -(id + 1)); centres and widths of the node and
 // leaf boxes (w unused); leaf_active >= 0 marks a leaf holding a local
@@ -13,38 +16,57 @@ struct WalkTree {
     const float4 *node_center, *node_width;
     const float4 *leaf_center, *leaf_width;
     const int *leaf_active;
+    int nnode, nleaf;
     float open_angle, cutoff;
 };
 
-// Forward pass, round of n frames f: code[i] = children (0, 2, 4) | task << 3
-// | well-separated << 4,
-// off[0..n] = exclusive scan of the children (off[n] = next round's size),
-// bs[b] = well-separated frames in block b (walk_blocks(n) blocks),
-// *emitted = frames of the round that emit a task, *separated = its
-// well-separated frames.
-// rocPRIM convention: temp == nullptr only queries *temp_bytes.
-hipError_t walk_code(const WalkTree &t, const int2 *f, long long n, unsigned char *code, unsigned *off, int *bs,
-                     unsigned long long *emitted, unsigned long long *separated, void *temp, size_t *temp_bytes,
-                     hipStream_t st);
-// Blocks of a round of n frames (the length of walk_code's bs).
-long long walk_blocks(long long n);
-// The children of round f at their offsets in next.
-hipError_t walk_children(const WalkTree &t, const int2 *f, long long n, const unsigned *off, int2 *next,
-                         hipStream_t st);
-// Backward pass: cnt[i] = tasks at and below frame i (xn: the next round's x,
-// null for the last round), x[0..n] = exclusive scan of cnt.  32-bit: the
-// caller checks that the list length (the emitted count) fits.
-hipError_t walk_below(const unsigned char *code, const unsigned *off, const int *xn, long long n, int *cnt, int *x,
-                      void *temp, size_t *temp_bytes, hipStream_t st);
-// Position pass: pos[i] = first task position of frame i; fills pos_next for
-// the next round and writes the tasks of the emitting frames.
-hipError_t walk_emit(const int2 *f, const unsigned char *code, const unsigned *off, const int *xn, long long n,
-                     const int *pos, int *pos_next, int *task_t, int *task_s, hipStream_t st);
+// One cell in 32 bytes: node k at k, leaf l at nnode + l.
+struct WalkCell {
+    float cx, cy, cz;
+    int a;                          // node: first son; leaf: active
+    float wx, wy, wz;
+    int b;                          // node: second son
+};
 
-// The round's well-separated frames (code bit 4), in frame order, written as
-// cells (leaf id, or nleaf + node id) to ct/cs: bso = exclusive scan of
-// walk_code's bs (walk_blocks(n) entries).  rocPRIM convention for temp.
-hipError_t walk_m2l(const int2 *f, const unsigned char *code, long long n, const int *bs, int *bso, int nleaf,
-                    int *ct, int *cs, void *temp, size_t *temp_bytes, hipStream_t st);
+// One round as the device keeps it: n opened frames at frame index fbase, its
+// tiles at tbase; what their children are.
+struct WalkRound {
+    unsigned n;
+    unsigned over;                  // 1: its frames did not fit the arrays (n is right)
+    unsigned ticket;
+    unsigned nsep;                  // well-separated children
+    unsigned long long ntask;       // leaf-leaf children that are tasks
+    long long fbase, tbase;
+};
+
+// The frames of all rounds, and per tile the look-back word and the
+// exclusive count of well-separated children before it in its round.
+struct WalkFrames {
+    int2 *f;                        // (target, source) cells: >= 0 node, < 0 leaf -(id + 1)
+    unsigned char *code;            // two bits per child: 0 none, 1 opened, 2 task, 3 well separated; bit 4 of a
+                                    // frame with two children: the target cell was split
+    unsigned *off;                  // first opened child in the next round
+    int *cnt;                       // tasks at and below; then the first task's position
+    long long cap;
+    unsigned long long *look;
+    int *sep;
+    long long tcap;
+};
+
+hipError_t walk_cells(const WalkTree &t, WalkCell *cells, hipStream_t st);
+// rounds[0] = cur (n frames at fbase, its tiles at tbase) with its counters
+// cleared, rounds[1 .. count) cleared, and the tiles' look-back words from tbase
+// on.  The frame of a first round (fbase 0) is set to the root's self pair.
+hipError_t walk_begin(const WalkFrames &w, WalkRound *rounds, int count, const WalkRound &cur, hipStream_t st);
+// Children of the round's frames: codes, offsets, the next round's frames and
+// both rounds' counters, by up to `blocks` blocks.
+hipError_t walk_open(const WalkTree &t, const WalkCell *cells, const WalkFrames &w, WalkRound *round, int blocks,
+                     hipStream_t st);
+// Backward: tasks at and below each of the n frames at fbase (children at fbase + n).
+hipError_t walk_below(const WalkFrames &w, long long fbase, unsigned n, hipStream_t st);
+// Positions: the first task of each opened child, the tasks of the round, and
+// (nsep > 0) its well-separated pairs from ct / cs on, as cells (leaf id, or nleaf + node id).
+hipError_t walk_emit(const WalkTree &t, const WalkCell *cells, const WalkFrames &w, long long fbase, long long tbase,
+                     unsigned n, unsigned nsep, int *task_t, int *task_s, int *ct, int *cs, hipStream_t st);
 
 }  // namespace pp2p
