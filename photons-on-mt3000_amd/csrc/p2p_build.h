@@ -31,6 +31,13 @@ hipError_t launch_i32_to_f64(const int *posi, long long n3, double int2pos, bool
 hipError_t launch_round_f32(double *x3, long long n3, hipStream_t st);
 hipError_t launch_fill_f64(double *p, long long n, double v, hipStream_t st);
 hipError_t launch_f64_to_f32(const double *a, long long n, float *b, hipStream_t st);
+// three planes of n to n rows of three
+hipError_t launch_planes_to_rows(const double *a, long long n, double *out, hipStream_t st);
+// n packed triples to float4 (w = 0), and back
+hipError_t launch_pack_xyz(const float *a, int n, float4 *out, hipStream_t st);
+hipError_t launch_unpack_xyz(const float4 *a, int n, float *out, hipStream_t st);
+// n pairs to two planes
+hipError_t launch_split_pairs(const int2 *a, int n, int *x, int *y, hipStream_t st);
 hipError_t launch_fill_i32(int *p, long long n, int v, hipStream_t st);
 
 // The functions below follow the rocPRIM convention: temp == nullptr only

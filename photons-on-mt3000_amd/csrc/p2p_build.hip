@@ -474,6 +474,71 @@ hipError_t launch_f64_to_f32(const double *a, long long n, float *b, hipStream_t
     return hipGetLastError();
 }
 
+__global__ void k_planes_to_rows(const double *__restrict__ a, long long n, double *__restrict__ out)
+{
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n)
+        return;
+    out[3 * k] = a[k];
+    out[3 * k + 1] = a[n + k];
+    out[3 * k + 2] = a[2 * n + k];
+}
+
+hipError_t launch_planes_to_rows(const double *a, long long n, double *out, hipStream_t st)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_planes_to_rows, dim3(grid_of(n)), dim3(256), 0, st, a, n, out);
+    return hipGetLastError();
+}
+
+__global__ void k_pack_xyz(const float *__restrict__ a, int n, float4 *__restrict__ out)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n)
+        out[k] = make_float4(a[3 * (size_t)k], a[3 * (size_t)k + 1], a[3 * (size_t)k + 2], 0.f);
+}
+
+hipError_t launch_pack_xyz(const float *a, int n, float4 *out, hipStream_t st)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_pack_xyz, dim3(grid_of(n)), dim3(256), 0, st, a, n, out);
+    return hipGetLastError();
+}
+
+__global__ void k_unpack_xyz(const float4 *__restrict__ a, int n, float *__restrict__ out)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n)
+        return;
+    const float4 v = a[k];
+    out[3 * (size_t)k] = v.x;
+    out[3 * (size_t)k + 1] = v.y;
+    out[3 * (size_t)k + 2] = v.z;
+}
+
+hipError_t launch_unpack_xyz(const float4 *a, int n, float *out, hipStream_t st)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_unpack_xyz, dim3(grid_of(n)), dim3(256), 0, st, a, n, out);
+    return hipGetLastError();
+}
+
+__global__ void k_split_pairs(const int2 *__restrict__ a, int n, int *__restrict__ x, int *__restrict__ y)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n)
+        return;
+    x[k] = a[k].x;
+    y[k] = a[k].y;
+}
+
+hipError_t launch_split_pairs(const int2 *a, int n, int *x, int *y, hipStream_t st)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_split_pairs, dim3(grid_of(n)), dim3(256), 0, st, a, n, x, y);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill_f64(double *p, long long n, double v, hipStream_t st)
 {
     if (n <= 0)

@@ -9,11 +9,12 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <thread>
+#include <atomic>
 #include <vector>
 
 #include "../../include/photons_p2p.h"
 #include "forcelaw.h"
+#include "host_pipe.h"
 #include "p2p_build.h"
 #include "p2p_launch.h"
 #include "p2p_m2l.h"
@@ -40,6 +41,9 @@ int fail(int code, const std::string &msg)
         if (e_ != hipSuccess)                                                              \
             return fail(PP2P_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
+
+// small results: sizes read between launches, the arrays of a small tree
+constexpr size_t kMailBytes = 128 << 10;
 
 // grow-only device buffer
 template <typename T>
@@ -69,7 +73,7 @@ struct DevBuf {
     }
 };
 
-// grow-only pinned host buffer (staging of host-side repacking)
+// pinned host buffer (small results that the host waits for)
 struct PinnedBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -94,28 +98,16 @@ struct PinnedBuf {
     }
 };
 
-// fn(b, e) over [0, n) in up to 16 threads when n is large
-template <typename Fn>
-void parallel_ranges(long long n, Fn fn)
+// whether every value lies in [0, n)
+bool all_below(const int *v, size_t count, unsigned n)
 {
-    const unsigned hw = std::thread::hardware_concurrency();
-    const long long nth = n < (1ll << 20) ? 1 : std::min<long long>(hw ? hw : 1, 16);
-    if (nth <= 1) {
-        fn(0ll, n);
-        return;
-    }
-    std::vector<std::thread> th;
-    for (long long k = 0; k < nth; ++k)
-        th.emplace_back(fn, n * k / nth, n * (k + 1) / nth);
-    for (auto &t : th)
-        t.join();
+    unsigned over = 0;
+    for (size_t k = 0; k < count; ++k)
+        over |= (unsigned)v[k] >= n;
+    return !over;
 }
 
 }  // namespace
-
-struct pp2p_ctx;
-template <typename Fill>
-static hipError_t staged_h2d(pp2p_ctx *c, void *dst, size_t units, size_t unit, size_t at, Fill fill);
 
 struct pp2p_ctx {
     int device = 0;
@@ -143,7 +135,11 @@ struct pp2p_ctx {
     DevBuf<float> acc32;        // FP32 copy of acc for pp2p_get_acc_f32_soa
     DevBuf<double> x3;          // FP64 staging of positions
     DevBuf<int> posi;           // int32 staging
-    PinnedBuf h_stage;          // host packing of strided records
+    HostPipe pipe;              // large host copies
+    PinnedBuf mail;             // small ones back, allocated with the context
+    DevBuf<double> acc3;        // AoS copy of acc for pp2p_get_acc_f64
+    DevBuf<float> xyz;          // packed triples on their way in or out
+    DevBuf<int> pair_a, pair_b; // planes of int2 arrays on their way out
     std::vector<int2> h_rng;
 
     // active subset
@@ -255,6 +251,64 @@ static int ensure_temp(pp2p_ctx *c, size_t bytes)
     return PP2P_OK;
 }
 
+// Waits for the stream with `bytes` from src in dst: through the pinned mailbox
+// when they fit (a copy to pageable memory is staged and waited for by the
+// runtime first).
+static int fetch(pp2p_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    if (bytes > c->mail.cap) {
+        HIPCHK(c->pipe.to_host(dst, src, bytes, c->stream));
+        return PP2P_OK;
+    }
+    HIPCHK(hipMemcpyAsync(c->mail.p, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(dst, c->mail.p, bytes);
+    return PP2P_OK;
+}
+
+// Several device arrays to the host with one wait where they fit the mailbox.
+class Gather {
+public:
+    explicit Gather(pp2p_ctx *c) : c_(c) {}
+    int add(void *dst, const void *src, size_t bytes)
+    {
+        if (!dst || !bytes)
+            return PP2P_OK;
+        if (bytes > c_->mail.cap - used_) {
+            int st = finish();
+            if (st)
+                return st;
+            if (bytes > c_->mail.cap) {
+                HIPCHK(c_->pipe.to_host(dst, src, bytes, c_->stream));
+                return PP2P_OK;
+            }
+        }
+        HIPCHK(hipMemcpyAsync(static_cast<char *>(c_->mail.p) + used_, src, bytes, hipMemcpyDeviceToHost, c_->stream));
+        parts_.push_back({dst, used_, bytes});
+        used_ += (bytes + 15) & ~(size_t)15;
+        used_ = std::min(used_, c_->mail.cap);
+        return PP2P_OK;
+    }
+    int finish()
+    {
+        HIPCHK(hipStreamSynchronize(c_->stream));
+        for (const Part &p : parts_)
+            std::memcpy(p.dst, static_cast<const char *>(c_->mail.p) + p.at, p.bytes);
+        parts_.clear();
+        used_ = 0;
+        return PP2P_OK;
+    }
+
+private:
+    struct Part {
+        void *dst;
+        size_t at, bytes;
+    };
+    pp2p_ctx *c_;
+    std::vector<Part> parts_;
+    size_t used_ = 0;
+};
+
 extern "C" {
 
 const char *pp2p_version(void) { return "photons_p2p 0.1 (gfx950)"; }
@@ -286,7 +340,7 @@ pp2p_ctx *pp2p_create(int device, int *status)
             hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreate(&c->ev_k0) != hipSuccess || hipEventCreate(&c->ev_k1) != hipSuccess ||
             hipEventCreate(&c->ev_p0) != hipSuccess || hipEventCreate(&c->ev_p1) != hipSuccess ||
-            c->counter.reserve(1) != hipSuccess) {
+            c->counter.reserve(1) != hipSuccess || c->mail.reserve(kMailBytes) != hipSuccess) {
             st = fail(PP2P_ERR_DEVICE, "context creation failed");
             pp2p_destroy(c);
             c = nullptr;
@@ -339,7 +393,12 @@ void pp2p_destroy(pp2p_ctx *c)
     c->idx.release(); c->idx_sorted.release(); c->counter.release(); c->temp.release();
     c->pair_count.release();
     c->acc32.release();
-    c->h_stage.release();
+    c->pipe.release();
+    c->mail.release();
+    c->acc3.release();
+    c->xyz.release();
+    c->pair_a.release();
+    c->pair_b.release();
     if (c->ev_k0) (void)hipEventDestroy(c->ev_k0);
     if (c->ev_k1) (void)hipEventDestroy(c->ev_k1);
     if (c->ev_p0) (void)hipEventDestroy(c->ev_p0);
@@ -430,16 +489,22 @@ static int upload_leaves(pp2p_ctx *c, long long npart, int nleaf, const int *lea
     if (nleaf < 0 || (nleaf > 0 && (!leaf_ip || !leaf_np)))
         return fail(PP2P_ERR_ARG, "invalid leaf arrays");
     c->h_rng.resize(nleaf);
+    bool ascending = true;                      // non-empty ranges in order and disjoint
+    long long end = 0;
     for (int l = 0; l < nleaf; ++l) {
         if (leaf_np[l] < 0 || leaf_ip[l] < 0 || (long long)leaf_ip[l] + leaf_np[l] > npart)
             return fail(PP2P_ERR_ARG, "leaf " + std::to_string(l) + " outside the particle range");
         c->h_rng[l] = make_int2(leaf_ip[l], leaf_np[l]);
+        if (leaf_np[l] > 0) {
+            ascending &= leaf_ip[l] >= end;
+            end = (long long)leaf_ip[l] + leaf_np[l];
+        }
     }
     // Every leaf owns its particles: the leaf frames and the i-order lists are
     // written per particle, so two leaves sharing a particle would overwrite
     // each other's entries.  Non-empty ranges must be disjoint (the kd-tree
-    // leaves of the reference are).
-    {
+    // leaves of the reference are, in order).
+    if (!ascending) {
         std::vector<int> ord;
         ord.reserve(nleaf);
         for (int l = 0; l < nleaf; ++l)
@@ -455,7 +520,7 @@ static int upload_leaves(pp2p_ctx *c, long long npart, int nleaf, const int *lea
     }
     HIPCHK(c->rng.reserve(std::max(nleaf, 1)));
     if (nleaf)
-        HIPCHK(hipMemcpyAsync(c->rng.p, c->h_rng.data(), sizeof(int2) * nleaf, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c->pipe.to_device(c->rng.p, c->h_rng.data(), sizeof(int2) * nleaf, c->stream));
     return PP2P_OK;
 }
 
@@ -500,38 +565,9 @@ int pp2p_set_particles_f64(pp2p_ctx *c, long long npart, const double *pos, int 
         return st;
     HIPCHK(c->x3.reserve(std::max<long long>(3 * npart, 1)));
     if (npart)
-        HIPCHK(hipMemcpyAsync(c->x3.p, pos, sizeof(double) * 3 * npart, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c->pipe.to_device(c->x3.p, pos, sizeof(double) * 3 * npart, c->stream));
     return finish_particles(c, npart, nleaf);
 }
-
-// Host-to-device copy of `units` records of `unit` bytes through the
-// context's pinned buffer (from byte `at`, reserved by the caller) in four
-// pieces: fill(stage, u0, u1) writes records [u0, u1) to stage + u0 * unit
-// (called on up to 16 threads, each with its own sub-range), and the DMA of a
-// piece overlaps the filling of the next.  Copies straight from pageable
-// memory ran at about half the rate.  The buffer stays in use until the
-// stream has passed the copies.
-extern "C++" {
-template <typename Fill>
-static hipError_t staged_h2d(pp2p_ctx *c, void *dst, size_t units, size_t unit, size_t at, Fill fill)
-{
-    char *stage = static_cast<char *>(c->h_stage.p) + at;
-    constexpr int kPieces = 4;
-    for (int k = 0; k < kPieces; ++k) {
-        const size_t u0 = units * k / kPieces, u1 = units * (k + 1) / kPieces;
-        if (u1 <= u0)
-            continue;
-        parallel_ranges((long long)(u1 - u0), [&](long long i0, long long i1) {
-            fill(stage, u0 + (size_t)i0, u0 + (size_t)i1);
-        });
-        hipError_t e = hipMemcpyAsync(static_cast<char *>(dst) + u0 * unit, stage + u0 * unit, (u1 - u0) * unit,
-                                      hipMemcpyHostToDevice, c->stream);
-        if (e != hipSuccess)
-            return e;
-    }
-    return hipSuccess;
-}
-}  // extern "C++"
 
 int pp2p_set_particles_i32(pp2p_ctx *c, long long npart, const void *posi, size_t stride, double int2pos, int nleaf,
                            const int *leaf_ip, const int *leaf_np)
@@ -548,23 +584,20 @@ int pp2p_set_particles_i32(pp2p_ctx *c, long long npart, const void *posi, size_
     HIPCHK(c->posi.reserve(std::max<long long>(3 * npart, 1)));
     HIPCHK(c->x3.reserve(std::max<long long>(3 * npart, 1)));
     if (npart) {
-        // contiguous 12-byte rows through a pinned buffer kept by the context:
-        // records wider than the three coordinates are packed on the way (as
-        // the reference repacks part[i].posi, src/gpu_entry.cu:85-105); a
-        // pitched copy of npart 12-byte rows from pageable memory is orders of
-        // magnitude slower
-        HIPCHK(c->h_stage.reserve(12 * (size_t)npart));
+        // contiguous 12-byte rows: records wider than the three coordinates are
+        // packed on the way through the pinned slots (as the reference repacks
+        // part[i].posi, src/gpu_entry.cu:85-105); a pitched copy of npart 12-byte
+        // rows from pageable memory is orders of magnitude slower
         const unsigned char *b = static_cast<const unsigned char *>(posi);
-        HIPCHK(staged_h2d(c, c->posi.p, (size_t)npart, 12, 0, [&](char *stage, size_t u0, size_t u1) {
-            if (stride == 12) {
-                std::memcpy(stage + 12 * u0, b + 12 * u0, 12 * (u1 - u0));
-                return;
-            }
-            for (size_t i = u0; i < u1; ++i)
-                std::memcpy(stage + 12 * i, b + i * stride, 12);
-        }));
+        if (stride == 12)
+            HIPCHK(c->pipe.to_device(c->posi.p, b, 12 * (size_t)npart, c->stream));
+        else
+            HIPCHK(c->pipe.to_device_filled(c->posi.p, 12 * (size_t)npart, 12, c->stream,
+                                            [=](char *at, size_t o, size_t n) {
+                                                for (size_t i = 0; i < n / 12; ++i)
+                                                    std::memcpy(at + 12 * i, b + (o / 12 + i) * stride, 12);
+                                            }));
         HIPCHK(launch_i32_to_f64(c->posi.p, 3 * npart, int2pos, false, c->x3.p, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));      // before the staging buffer is reused
     }
     return finish_particles(c, npart, nleaf);
 }
@@ -588,7 +621,7 @@ int pp2p_set_active(pp2p_ctx *c, const unsigned char *a, int level)
     HIPCHK(c->act_off.reserve(c->nleaf + 1));
     HIPCHK(c->ilist.reserve(std::max<long long>(c->npart, 1)));
     if (c->npart)
-        HIPCHK(hipMemcpyAsync(c->act.p, a, c->npart, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c->pipe.to_device(c->act.p, a, c->npart, c->stream));
     size_t tb = 0;
     HIPCHK(active_lists(c->act.p, level, c->rng.p, c->nleaf, c->act_cnt.p, c->act_off.p, c->ilist.p, nullptr, &tb,
                         c->stream));
@@ -610,37 +643,6 @@ static int append_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
         return fail(PP2P_ERR_ARG, "invalid task arrays");
     if (c->ntask + n > (1ll << 31) - 1)
         return fail(PP2P_ERR_ARG, "more than 2^31-1 tasks in one list");
-    {
-        // the first task naming a leaf outside [0, nleaf), in parallel over
-        // ranges of a long list
-        const unsigned nl = (unsigned)c->nleaf;
-        auto first_bad = [&](long long b, long long e) {
-            for (long long k = b; k < e; ++k)
-                if ((unsigned)tt[k] >= nl || (unsigned)ts[k] >= nl)
-                    return k;
-            return e;
-        };
-        long long bad = n;
-        const unsigned hw = std::thread::hardware_concurrency();
-        const int nth = n < (1ll << 20) ? 1 : (int)std::min<unsigned>(hw ? hw : 1, 16);
-        if (nth <= 1) {
-            bad = first_bad(0, n);
-        } else {
-            std::vector<long long> found(nth, n);
-            std::vector<std::thread> th;
-            for (int k = 0; k < nth; ++k)
-                th.emplace_back([&, k] {
-                    const long long b = n * k / nth, e = n * (k + 1) / nth;
-                    const long long f = first_bad(b, e);
-                    found[k] = f < e ? f : n;
-                });
-            for (auto &t : th)
-                t.join();
-            bad = *std::min_element(found.begin(), found.end());
-        }
-        if (bad < n)
-            return fail(PP2P_ERR_ARG, "task " + std::to_string(bad) + " names a leaf outside [0, nleaf)");
-    }
     const size_t need = (size_t)(c->ntask + n);
     if (need > c->task_t.cap) {
         // keep the existing tasks across the grow
@@ -658,9 +660,31 @@ static int append_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
         c->task_s = ns;
     }
     if (n) {
-        HIPCHK(hipMemcpyAsync(c->task_t.p + c->ntask, tt, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipMemcpyAsync(c->task_s.p + c->ntask, ts, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+        // the leaf ids are checked while they are copied; a bad list leaves the
+        // context's as it is
+        const unsigned nl = (unsigned)c->nleaf;
+        std::atomic<bool> good{true};
+        auto upload = [&](int *dst, const int *v) {
+            const size_t bytes = sizeof(int) * (size_t)n;
+            if (bytes < HostPipe::kLeast) {
+                if (!all_below(v, (size_t)n, nl))
+                    good = false;
+                return c->pipe.to_device(dst, v, bytes, c->stream);
+            }
+            return c->pipe.to_device_filled(dst, bytes, sizeof(int), c->stream, [&](char *at, size_t b, size_t m) {
+                const int *p = v + b / sizeof(int);
+                std::memcpy(at, p, m);
+                if (!all_below(p, m / sizeof(int), nl))
+                    good = false;
+            });
+        };
+        HIPCHK(upload(c->task_t.p + c->ntask, tt));
+        HIPCHK(upload(c->task_s.p + c->ntask, ts));
         HIPCHK(hipStreamSynchronize(c->stream));   // the caller may reuse its buffers on return
+        if (!good)
+            for (long long k = 0; k < n; ++k)
+                if ((unsigned)tt[k] >= nl || (unsigned)ts[k] >= nl)
+                    return fail(PP2P_ERR_ARG, "task " + std::to_string(k) + " names a leaf outside [0, nleaf)");
     }
     c->ntask += n;
     c->csr_ready = c->items_ready = false;
@@ -690,12 +714,10 @@ int pp2p_add_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
 
 static int upload_boxes(pp2p_ctx *c, DevBuf<float4> &dst, int n, const float *xyz)
 {
-    std::vector<float4> h((size_t)std::max(n, 1));
-    for (int k = 0; k < n; ++k)
-        h[k] = make_float4(xyz[3 * k], xyz[3 * k + 1], xyz[3 * k + 2], 0.f);
-    HIPCHK(dst.reserve(h.size()));
-    HIPCHK(hipMemcpyAsync(dst.p, h.data(), sizeof(float4) * h.size(), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(dst.reserve(std::max(n, 1)));
+    HIPCHK(c->xyz.reserve(3 * (size_t)std::max(n, 1)));
+    HIPCHK(c->pipe.to_device(c->xyz.p, xyz, sizeof(float) * 3 * (size_t)n, c->stream));
+    HIPCHK(launch_pack_xyz(c->xyz.p, n, dst.p, c->stream));
     return PP2P_OK;
 }
 
@@ -757,8 +779,8 @@ static int run_walk(pp2p_ctx *c, float open_angle, float cutoff_radius, long lon
     if (nnode == 0) {
         // one leaf: its self pair
         int act = -1;
-        HIPCHK(hipMemcpyAsync(&act, c->wact.p, sizeof(int), hipMemcpyDeviceToHost, sm));
-        HIPCHK(hipStreamSynchronize(sm));
+        if ((st = fetch(c, &act, c->wact.p, sizeof(int))))
+            return st;
         emitted = act >= 0 ? 1 : 0;
         HIPCHK(c->task_t.reserve(1));
         HIPCHK(c->task_s.reserve(1));
@@ -794,8 +816,8 @@ static int run_walk(pp2p_ctx *c, float open_angle, float cutoff_radius, long lon
                 HIPCHK(walk_open(t, c->wcell.p, w, c->wround.p + k, blocks, sm));
             }
             h.resize((size_t)group + 1);
-            HIPCHK(hipMemcpyAsync(h.data(), c->wround.p, sizeof(WalkRound) * h.size(), hipMemcpyDeviceToHost, sm));
-            HIPCHK(hipStreamSynchronize(sm));
+            if ((st = fetch(c, h.data(), c->wround.p, sizeof(WalkRound) * h.size())))
+                return st;
             for (int k = 0; k <= group; ++k) {
                 if (h[k].n > (1u << 29))
                     return fail(PP2P_ERR_ARG, "tree walk round larger than 2^29 frames");
@@ -877,9 +899,9 @@ int pp2p_walk_tasks(pp2p_ctx *c, int nnode, const int *node_son, const float *no
         }
     HIPCHK(c->wson.reserve(std::max(nnode, 1)));
     if (nnode)
-        HIPCHK(hipMemcpyAsync(c->wson.p, node_son, sizeof(int2) * nnode, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c->pipe.to_device(c->wson.p, node_son, sizeof(int2) * nnode, c->stream));
     HIPCHK(c->wact.reserve(nleaf));
-    HIPCHK(hipMemcpyAsync(c->wact.p, leaf_active, sizeof(int) * nleaf, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c->pipe.to_device(c->wact.p, leaf_active, sizeof(int) * nleaf, c->stream));
     if ((st = upload_boxes(c, c->wnc, nnode, node_center)) || (st = upload_boxes(c, c->wnw, nnode, node_width)) ||
         (st = upload_boxes(c, c->wlc, nleaf, leaf_center)) || (st = upload_boxes(c, c->wlw, nleaf, leaf_width)))
         return st;
@@ -964,9 +986,8 @@ static int tree_split_all(pp2p_ctx *c, const TreeScratch &w, long long n, double
                 HIPCHK(tree_level(w, tl[k].v, tl[k + 1].v, k, (int)cap(k), tiles(k), int2pos, maxleaf, gmax,
                                   c->tmask.p, c->ttcnt.p, c->ttmap.p, c->tcounts.p, c->tsub.p,
                                   subs ? (int)subcap : 0, sm));
-            HIPCHK(hipMemcpyAsync(&h, c->tcounts.p, sizeof(int) * (size_t)(2 + l + group + 1), hipMemcpyDeviceToHost,
-                                  sm));
-            HIPCHK(hipStreamSynchronize(sm));
+            if ((st = fetch(c, &h, c->tcounts.p, sizeof(int) * (size_t)(2 + l + group + 1))))
+                return st;
             if (h.misfit)
                 return PP2P_OK;
             for (int k = l; k < l + group && last < 0; ++k) {
@@ -986,12 +1007,13 @@ static int tree_split_all(pp2p_ctx *c, const TreeScratch &w, long long n, double
     HIPCHK(tree_subs(w, c->tsub.p, *nsub, int2pos, maxleaf, c->tsuboff.p, c->tcounts.p, sm));
     for (int l = last; l >= 0; --l)
         HIPCHK(tree_below(tl[l].v, tl[l].nseg, l < last ? tl[l + 1].v.below : nullptr, c->tsub.p, sm));
-    HIPCHK(hipMemcpyAsync(&h, c->tcounts.p, 2 * sizeof(int), hipMemcpyDeviceToHost, sm));
-    if (root_sub)
-        HIPCHK(hipMemcpyAsync(counts, &c->tsub.p->nnode, sizeof(int2), hipMemcpyDeviceToHost, sm));
-    else
-        HIPCHK(hipMemcpyAsync(counts, tl[0].v.below, sizeof(int2), hipMemcpyDeviceToHost, sm));
+    int *mail = static_cast<int *>(c->mail.p);
+    HIPCHK(hipMemcpyAsync(mail, &c->tcounts.p->misfit, sizeof(int), hipMemcpyDeviceToHost, sm));
+    HIPCHK(hipMemcpyAsync(mail + 2, root_sub ? (const void *)&c->tsub.p->nnode : (const void *)tl[0].v.below,
+                          sizeof(int2), hipMemcpyDeviceToHost, sm));
     HIPCHK(hipStreamSynchronize(sm));
+    *counts = make_int2(mail[2], mail[3]);
+    h.misfit = mail[0];
     *fits = h.misfit == 0;
     return PP2P_OK;
 }
@@ -1014,16 +1036,8 @@ int pp2p_build_tree(pp2p_ctx *c, long long n, const int *posi, const int *tag, d
     HIPCHK(c->ttag.reserve(n));
     for (DevBuf<int> *b : {&c->tx0, &c->tx1, &c->tx2, &c->tidx, &c->tla, &c->tlb, &c->tlc, &c->tld})
         HIPCHK(b->reserve(n));
-    {
-        const size_t np3 = 3 * (size_t)n;
-        HIPCHK(c->h_stage.reserve(sizeof(int) * (np3 + (size_t)n)));
-        HIPCHK(staged_h2d(c, c->tposi.p, np3, sizeof(int), 0, [&](char *stage, size_t u0, size_t u1) {
-            std::memcpy(stage + sizeof(int) * u0, posi + u0, sizeof(int) * (u1 - u0));
-        }));
-        HIPCHK(staged_h2d(c, c->ttag.p, (size_t)n, sizeof(int), sizeof(int) * np3, [&](char *stage, size_t u0, size_t u1) {
-            std::memcpy(stage + sizeof(int) * u0, tag + u0, sizeof(int) * (u1 - u0));
-        }));
-    }
+    HIPCHK(c->pipe.to_device(c->tposi.p, posi, sizeof(int) * 3 * (size_t)n, sm));
+    HIPCHK(c->pipe.to_device(c->ttag.p, tag, sizeof(int) * (size_t)n, sm));
     const TreeScratch w{{c->tx0.p, c->tx1.p, c->tx2.p}, c->tidx.p, c->tla.p, c->tlb.p, c->tlc.p, c->tld.p};
     int levels = 0, nsub = 0;
     int2 counts = make_int2(0, 0);
@@ -1083,20 +1097,6 @@ int pp2p_walk_tree(pp2p_ctx *c, float open_angle, float cutoff_radius, long long
     return run_walk(c, open_angle, cutoff_radius, ntask);
 }
 
-static int copy_xyz(pp2p_ctx *c, const float4 *src, int n, float *dst)
-{
-    std::vector<float4> h((size_t)n);
-    if (n)
-        HIPCHK(hipMemcpyAsync(h.data(), src, sizeof(float4) * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (int k = 0; k < n; ++k) {
-        dst[3 * k] = h[k].x;
-        dst[3 * k + 1] = h[k].y;
-        dst[3 * k + 2] = h[k].z;
-    }
-    return PP2P_OK;
-}
-
 int pp2p_get_tree(pp2p_ctx *c, int *perm, int *leaf_ip, int *leaf_np, int *leaf_active, float *leaf_center,
                   float *leaf_width, int *node_son, float *node_center, float *node_width)
 {
@@ -1106,30 +1106,34 @@ int pp2p_get_tree(pp2p_ctx *c, int *perm, int *leaf_ip, int *leaf_np, int *leaf_
     if (!c->tree_ready)
         return fail(PP2P_ERR_STATE, "no tree built on the device");
     const int nleaf = c->nleaf, nnode = c->walk_nnode;
-    if (perm)
-        HIPCHK(hipMemcpyAsync(perm, c->tidx.p, sizeof(int) * c->npart, hipMemcpyDeviceToHost, c->stream));
-    if (leaf_active)
-        HIPCHK(hipMemcpyAsync(leaf_active, c->wact.p, sizeof(int) * nleaf, hipMemcpyDeviceToHost, c->stream));
-    if (node_son)
-        HIPCHK(hipMemcpyAsync(node_son, c->wson.p, sizeof(int2) * nnode, hipMemcpyDeviceToHost, c->stream));
-    if (leaf_ip || leaf_np) {
-        std::vector<int2> r((size_t)nleaf);
-        HIPCHK(hipMemcpyAsync(r.data(), c->rng.p, sizeof(int2) * nleaf, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        for (int l = 0; l < nleaf; ++l) {
-            if (leaf_ip)
-                leaf_ip[l] = r[l].x;
-            if (leaf_np)
-                leaf_np[l] = r[l].y;
-        }
-    }
-    if ((leaf_center && (st = copy_xyz(c, c->wlc.p, nleaf, leaf_center))) ||
-        (leaf_width && (st = copy_xyz(c, c->wlw.p, nleaf, leaf_width))) ||
-        (node_center && (st = copy_xyz(c, c->wnc.p, nnode, node_center))) ||
-        (node_width && (st = copy_xyz(c, c->wnw.p, nnode, node_width))))
+    // the boxes and leaf ranges are unpacked on the device, each into its own
+    // part of the buffers
+    const size_t nl = (size_t)nleaf, nn = (size_t)nnode;
+    HIPCHK(c->xyz.reserve(6 * (nl + nn)));
+    HIPCHK(c->pair_a.reserve(nl));
+    HIPCHK(c->pair_b.reserve(nl));
+    const float4 *boxes[4] = {c->wlc.p, c->wlw.p, c->wnc.p, c->wnw.p};
+    float *const box_out[4] = {leaf_center, leaf_width, node_center, node_width};
+    Gather g(c);
+    if ((st = g.add(perm, c->tidx.p, sizeof(int) * (size_t)c->npart)) ||
+        (st = g.add(leaf_active, c->wact.p, sizeof(int) * nl)) || (st = g.add(node_son, c->wson.p, sizeof(int2) * nn)))
         return st;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return PP2P_OK;
+    if (leaf_ip || leaf_np) {
+        HIPCHK(launch_split_pairs(c->rng.p, nleaf, c->pair_a.p, c->pair_b.p, c->stream));
+        if ((st = g.add(leaf_ip, c->pair_a.p, sizeof(int) * nl)) || (st = g.add(leaf_np, c->pair_b.p, sizeof(int) * nl)))
+            return st;
+    }
+    float *at = c->xyz.p;
+    for (int k = 0; k < 4; ++k) {
+        const size_t n = k < 2 ? nl : nn;
+        if (box_out[k]) {
+            HIPCHK(launch_unpack_xyz(boxes[k], (int)n, at, c->stream));
+            if ((st = g.add(box_out[k], at, sizeof(float) * 3 * n)))
+                return st;
+        }
+        at += 3 * n;
+    }
+    return g.finish();
 }
 
 static int upload_centers(pp2p_ctx *c, int n, const float *xyz)
@@ -1139,6 +1143,14 @@ static int upload_centers(pp2p_ctx *c, int n, const float *xyz)
 
 static int m2l_core(pp2p_ctx *c, int ncell, long long ntask, const int *task_t, const int *task_s, float rs,
                     double *ms_out);
+static int check_m2l_tasks(long long ntask, const int *task_t, const int *task_s, long long ncell)
+{
+    if (ntask > 0 && !(all_below(task_t, (size_t)ntask, (unsigned)ncell) && all_below(task_s, (size_t)ntask, (unsigned)ncell)))
+        for (long long k = 0; k < ntask; ++k)
+            if ((unsigned)task_t[k] >= (unsigned)ncell || (unsigned)task_s[k] >= (unsigned)ncell)
+                return fail(PP2P_ERR_ARG, "m2l task " + std::to_string(k) + " names a cell outside [0, ncell)");
+    return PP2P_OK;
+}
 // host task arrays to the device copies mtt / mts
 static int upload_m2l_tasks(pp2p_ctx *c, long long ntask, const int *task_t, const int *task_s)
 {
@@ -1146,8 +1158,8 @@ static int upload_m2l_tasks(pp2p_ctx *c, long long ntask, const int *task_t, con
         return PP2P_OK;
     HIPCHK(c->mtt.reserve(ntask));
     HIPCHK(c->mts.reserve(ntask));
-    HIPCHK(hipMemcpyAsync(c->mtt.p, task_t, sizeof(int) * ntask, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->mts.p, task_s, sizeof(int) * ntask, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c->pipe.to_device(c->mtt.p, task_t, sizeof(int) * (size_t)ntask, c->stream));
+    HIPCHK(c->pipe.to_device(c->mts.p, task_s, sizeof(int) * (size_t)ntask, c->stream));
     return PP2P_OK;
 }
 
@@ -1163,23 +1175,21 @@ int pp2p_m2l(pp2p_ctx *c, int ncell, const float *center, const float *M, long l
         return fail(PP2P_ERR_ARG, "invalid split radius");
     if (ntask > (1ll << 31) - 1 || (long long)ncell * 20 > (1ll << 31) - 1)
         return fail(PP2P_ERR_ARG, "more than 2^31-1 tasks or coefficients");
-    for (long long k = 0; k < ntask; ++k)
-        if (task_t[k] < 0 || task_t[k] >= ncell || task_s[k] < 0 || task_s[k] >= ncell)
-            return fail(PP2P_ERR_ARG, "m2l task " + std::to_string(k) + " names a cell outside [0, ncell)");
+    if ((st = check_m2l_tasks(ntask, task_t, task_s, ncell)))
+        return st;
     const hipStream_t sm = c->stream;
     if ((st = upload_centers(c, ncell, center)))
         return st;
     const size_t nco = (size_t)20 * ncell;
     HIPCHK(c->mM.reserve(nco));
     HIPCHK(c->mL.reserve(nco));
-    HIPCHK(hipMemcpyAsync(c->mM.p, M, sizeof(float) * nco, hipMemcpyHostToDevice, sm));
-    HIPCHK(hipMemcpyAsync(c->mL.p, L, sizeof(float) * nco, hipMemcpyHostToDevice, sm));
+    HIPCHK(c->pipe.to_device(c->mM.p, M, sizeof(float) * nco, sm));
+    HIPCHK(c->pipe.to_device(c->mL.p, L, sizeof(float) * nco, sm));
     c->fmm_ready = false;
     double ms = 0.0;
     if ((st = upload_m2l_tasks(c, ntask, task_t, task_s)) || (st = m2l_core(c, ncell, ntask, c->mtt.p, c->mts.p, rs, &ms)))
         return st;
-    HIPCHK(hipMemcpyAsync(L, c->mL.p, sizeof(float) * nco, hipMemcpyDeviceToHost, sm));
-    HIPCHK(hipStreamSynchronize(sm));
+    HIPCHK(c->pipe.to_host(L, c->mL.p, sizeof(float) * nco, sm));
     if (kernel_ms)
         *kernel_ms = ms;
     return PP2P_OK;
@@ -1210,8 +1220,8 @@ static int m2l_core(pp2p_ctx *c, int ncell, long long ntask, const int *task_t, 
         HIPCHK(csr_sort(task_t, task_s, c->mkey.p, c->msrc.p, n, bits, c->temp.p, &tb1, sm));
         HIPCHK(csr_rows(c->mkey.p, n, c->mflag.p, c->mrowidx.p, c->mrow_tgt.p, c->mrow_off.p, c->temp.p, &tb2,
                         sm));
-        HIPCHK(hipMemcpyAsync(&nrows, c->mrowidx.p + n - 1, sizeof(int), hipMemcpyDeviceToHost, sm));
-        HIPCHK(hipStreamSynchronize(sm));
+        if ((st = fetch(c, &nrows, c->mrowidx.p + n - 1, sizeof(int))))
+            return st;
     }
     if (!c->ev_m0) {
         HIPCHK(hipEventCreate(&c->ev_m0));
@@ -1243,7 +1253,7 @@ int pp2p_l2p(pp2p_ctx *c, const float *L, const float *center)
         return st;
     const size_t nco = (size_t)20 * c->nleaf;
     HIPCHK(c->mL.reserve(nco));
-    HIPCHK(hipMemcpyAsync(c->mL.p, L, sizeof(float) * nco, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c->pipe.to_device(c->mL.p, L, sizeof(float) * nco, c->stream));
     c->fmm_ready = false;
     const L2PArgs a{c->rng.p, c->mcenter.p, c->mL.p, c->x3.p, c->nleaf, c->npart, c->acc.p};
     HIPCHK(launch_l2p(a, c->stream));
@@ -1269,9 +1279,8 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
         return fail(PP2P_ERR_STATE, "no well-separated pairs from pp2p_walk_tree on this tree");
     if (!walked && nm2l > 0 && (!m2l_t || !m2l_s))
         return fail(PP2P_ERR_ARG, "invalid m2l task arrays");
-    for (long long k = 0; k < nm2l; ++k)
-        if (m2l_t[k] < 0 || m2l_t[k] >= ncell || m2l_s[k] < 0 || m2l_s[k] >= ncell)
-            return fail(PP2P_ERR_ARG, "m2l task " + std::to_string(k) + " names a cell outside [0, ncell)");
+    if ((st = check_m2l_tasks(nm2l, m2l_t, m2l_s, ncell)))
+        return st;
     const hipStream_t sm = c->stream;
     HIPCHK(c->mcenter.reserve(ncell));
     HIPCHK(c->mM.reserve(20 * ncell));
@@ -1336,9 +1345,9 @@ int pp2p_get_expansions(pp2p_ctx *c, float *M, float *L)
         return fail(PP2P_ERR_STATE, "no fmm_short since the last tree or m2l call");
     const size_t n = (size_t)20 * ((size_t)c->nleaf + c->walk_nnode);
     if (M)
-        HIPCHK(hipMemcpyAsync(M, c->mM.p, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(M, c->mM.p, sizeof(float) * n, c->stream));
     if (L)
-        HIPCHK(hipMemcpyAsync(L, c->mL.p, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(L, c->mL.p, sizeof(float) * n, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return PP2P_OK;
 }
@@ -1353,9 +1362,9 @@ int pp2p_get_m2l_tasks(pp2p_ctx *c, long long *n, int *m2l_t, int *m2l_s)
     if (n)
         *n = c->walk_m2l_n;
     if (c->walk_m2l_n && m2l_t)
-        HIPCHK(hipMemcpyAsync(m2l_t, c->wm2l_t.p, sizeof(int) * c->walk_m2l_n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(m2l_t, c->wm2l_t.p, sizeof(int) * (size_t)c->walk_m2l_n, c->stream));
     if (c->walk_m2l_n && m2l_s)
-        HIPCHK(hipMemcpyAsync(m2l_s, c->wm2l_s.p, sizeof(int) * c->walk_m2l_n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(m2l_s, c->wm2l_s.p, sizeof(int) * (size_t)c->walk_m2l_n, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return PP2P_OK;
 }
@@ -1367,12 +1376,11 @@ int pp2p_get_tasks(pp2p_ctx *c, long long *ntask, int *task_t, int *task_s)
         return st;
     if (ntask)
         *ntask = c->ntask;
-    if (c->ntask && task_t)
-        HIPCHK(hipMemcpyAsync(task_t, c->task_t.p, sizeof(int) * c->ntask, hipMemcpyDeviceToHost, c->stream));
-    if (c->ntask && task_s)
-        HIPCHK(hipMemcpyAsync(task_s, c->task_s.p, sizeof(int) * c->ntask, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return PP2P_OK;
+    Gather g(c);
+    if ((st = g.add(task_t, c->task_t.p, sizeof(int) * (size_t)c->ntask)) ||
+        (st = g.add(task_s, c->task_s.p, sizeof(int) * (size_t)c->ntask)))
+        return st;
+    return g.finish();
 }
 
 // Device storage of one list's CSR and work items: the context's grow-only
@@ -1495,8 +1503,8 @@ static int csr_build(pp2p_ctx *c, Space &sp, const int *tt, const int *ts, int n
     HIPCHK(csr_sort(tt, ts, L.key_sorted, L.src, n, bits, tmp, &tb1, c->stream));
     HIPCHK(csr_rows(L.key_sorted, n, flag, rowidx, L.row_tgt, L.row_off, tmp, &tb2, c->stream));
     int rows = 0;
-    HIPCHK(hipMemcpyAsync(&rows, rowidx + n - 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((st = fetch(c, &rows, rowidx + n - 1, sizeof(int))))
+        return st;
     L.nrows = rows;
     return PP2P_OK;
 }
@@ -1563,10 +1571,9 @@ static int queue_waves(pp2p_ctx *c)
 
 // Work items of a list: every CSR row cut into i-chunks and source ranges of
 // about `split` pair-interactions.  Two copies: row order (GRID and
-// PER_TARGET forms; h_item_off, when given, receives the items per row) and
-// sorted by cost, largest first (QUEUE form).  Two host synchronisations
+// PER_TARGET forms) and sorted by cost, largest first (QUEUE form).  Two host synchronisations
 // (the pair total, the item count).
-static int items_build(pp2p_ctx *c, Space &sp, ListView &L, std::vector<int> *h_item_off)
+static int items_build(pp2p_ctx *c, Space &sp, ListView &L)
 {
     const int nr = L.nrows;
     unsigned long long *row_cost = nullptr, *total = nullptr;
@@ -1578,8 +1585,6 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L, std::vector<int> *h_
         return st;
     L.nitems = 0;
     L.pairs = 0;
-    if (h_item_off)
-        h_item_off->assign(1, 0);
     if (nr == 0)
         return PP2P_OK;
     if ((st = sp.get(c->nsx, (size_t)L.ntask + 1, &L.nsx)))
@@ -1597,8 +1602,8 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L, std::vector<int> *h_
     HIPCHK(src_prefix(L.src, c->rng.p, L.ntask, L.nsx, tmp, &tb0, c->stream));
     HIPCHK(rows_cost(ra, row_cost, total, tmp, &tb1, c->stream));
     unsigned long long tot[2] = {0, 0};              // pairs, staged source particles
-    HIPCHK(hipMemcpyAsync(tot, total, sizeof(tot), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((st = fetch(c, tot, total, sizeof(tot))))
+        return st;
     L.pairs = tot[0];
 
     long long split;
@@ -1616,8 +1621,8 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L, std::vector<int> *h_
     HIPCHK(launch_fill_i32(item_count + nr, 1, 0, c->stream));
     HIPCHK(items_count(ra, split, item_count, item_off, tmp, &tb2, c->stream));
     int nitems = 0;
-    HIPCHK(hipMemcpyAsync(&nitems, item_off + nr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((st = fetch(c, &nitems, item_off + nr, sizeof(int))))
+        return st;
     unsigned *cost = nullptr, *cost_sorted = nullptr;
     int *idx = nullptr, *idx_sorted = nullptr;
     if ((st = sp.get(c->items_rows, nitems, &L.items_rows)) || (st = sp.get(c->items_q, nitems, &L.items_q)) ||
@@ -1631,12 +1636,6 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L, std::vector<int> *h_
     if ((st = sp.temp(tb3, &tmp, &tb3)))
         return st;
     HIPCHK(items_sort(cost, cost_sorted, idx, idx_sorted, L.items_rows, L.items_q, nitems, tmp, &tb3, c->stream));
-    if (h_item_off) {
-        h_item_off->resize(nr + 1);
-        HIPCHK(hipMemcpyAsync(h_item_off->data(), item_off, sizeof(int) * (nr + 1), hipMemcpyDeviceToHost,
-                              c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
     L.nitems = nitems;
     L.split = split;
     return PP2P_OK;
@@ -1646,16 +1645,19 @@ static int build_items(pp2p_ctx *c)
 {
     Space sp(c);
     ListView L = ctx_view(c);
-    int st = items_build(c, sp, L, &c->h_item_off);
+    int st = items_build(c, sp, L);
     if (st)
         return st;
+    c->h_item_off.clear();
     c->list_pairs = L.pairs;
     c->nitems = L.nitems;
     c->split = L.split;
     return PP2P_OK;
 }
 
-static int prepare_form(pp2p_ctx *c, bool)
+// CSR and items of the current list, and for the PER_TARGET form the items of
+// each row on the host.
+static int prepare_form(pp2p_ctx *c, int exec)
 {
     int st;
     if (!c->csr_ready && (st = build_csr(c)))
@@ -1664,6 +1666,13 @@ static int prepare_form(pp2p_ctx *c, bool)
         if ((st = build_items(c)))
             return st;
         c->items_ready = true;
+    }
+    if (exec == PP2P_EXEC_PER_TARGET && c->nrows > 0 && c->h_item_off.empty()) {
+        c->h_item_off.resize((size_t)c->nrows + 1);
+        if ((st = fetch(c, c->h_item_off.data(), c->item_off.p, sizeof(int) * c->h_item_off.size()))) {
+            c->h_item_off.clear();
+            return st;
+        }
     }
     return PP2P_OK;
 }
@@ -1677,7 +1686,7 @@ int pp2p_prepare(pp2p_ctx *c)
         return fail(PP2P_ERR_STATE, "set_particles before prepare");
     HIPCHK(hipEventRecord(c->ev_p0, c->stream));
     c->csr_ready = c->items_ready = false;
-    if ((st = prepare_form(c, true)))
+    if ((st = prepare_form(c, PP2P_EXEC_QUEUE)))
         return st;
     HIPCHK(hipEventRecord(c->ev_p1, c->stream));
     HIPCHK(hipEventSynchronize(c->ev_p1));
@@ -1758,7 +1767,7 @@ int pp2p_compute(pp2p_ctx *c, int exec)
         return fail(PP2P_ERR_STATE, "set_particles before compute");
     if (exec != PP2P_EXEC_QUEUE && exec != PP2P_EXEC_GRID && exec != PP2P_EXEC_PER_TARGET)
         return fail(PP2P_ERR_ARG, "unknown execution form");
-    if ((st = prepare_form(c, exec == PP2P_EXEC_QUEUE)))
+    if ((st = prepare_form(c, exec)))
         return st;
     HIPCHK(hipEventRecord(c->ev_k0, c->stream));
     if ((st = enqueue_compute(c, exec)))
@@ -1789,12 +1798,12 @@ int pp2p_compute_noalloc(pp2p_ctx *c, long long ntask, const int *task_t, const 
     HIPCHK(launch_fill_i32(flag, 1, 0, c->stream));
     HIPCHK(launch_check_tasks(task_t, task_s, ntask, c->nleaf, flag, c->stream));
     int bad = 0;
-    HIPCHK(hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if ((st = fetch(c, &bad, flag, sizeof(int))))
+        return st;
     if (bad)
         return fail(PP2P_ERR_ARG, "compute_noalloc: a task names a leaf outside [0, nleaf)");
     ListView L;
-    if ((st = csr_build(c, sp, task_t, task_s, (int)ntask, L)) || (st = items_build(c, sp, L, nullptr)))
+    if ((st = csr_build(c, sp, task_t, task_s, (int)ntask, L)) || (st = items_build(c, sp, L)))
         return st;
     ForceArgs a = force_args(c, true);
     a.items = L.items_q;
@@ -1836,7 +1845,7 @@ int pp2p_run_graph(pp2p_ctx *c, int exec, int nsteps, int nreplay)
         return fail(PP2P_ERR_ARG, "nsteps and nreplay must be >= 1");
     if (exec != PP2P_EXEC_QUEUE && exec != PP2P_EXEC_GRID && exec != PP2P_EXEC_PER_TARGET)
         return fail(PP2P_ERR_ARG, "unknown execution form");
-    if ((st = prepare_form(c, exec == PP2P_EXEC_QUEUE)))
+    if ((st = prepare_form(c, exec)))
         return st;
     // occupancy queries are not capturable: resolve them before capture
     (void)queue_groups(c);
@@ -1893,15 +1902,15 @@ int pp2p_get_acc_f64(pp2p_ctx *c, double *out)
         return st;
     if (!out && c->npart)
         return fail(PP2P_ERR_ARG, "null output");
-    std::vector<double> planes((size_t)3 * c->npart);
-    if (c->npart)
-        HIPCHK(hipMemcpyAsync(planes.data(), c->acc.p, sizeof(double) * 3 * c->npart, hipMemcpyDeviceToHost,
-                              c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    for (long long i = 0; i < c->npart; ++i)
-        for (int d = 0; d < 3; ++d)
-            out[3 * i + d] = planes[(size_t)d * c->npart + i];
-    return PP2P_OK;
+    // transposed on the device; a copy of the planes and a host pass over them
+    // took ten times as long
+    if (c->npart) {
+        HIPCHK(c->acc3.reserve((size_t)3 * c->npart));
+        HIPCHK(launch_planes_to_rows(c->acc.p, c->npart, c->acc3.p, c->stream));
+    }
+    Gather g(c);
+    st = g.add(out, c->acc3.p, sizeof(double) * 3 * (size_t)c->npart);
+    return st ? st : g.finish();
 }
 
 int pp2p_get_acc_f32_soa(pp2p_ctx *c, float *out)
@@ -1915,10 +1924,10 @@ int pp2p_get_acc_f32_soa(pp2p_ctx *c, float *out)
     if (c->npart) {
         HIPCHK(c->acc32.reserve((size_t)3 * c->npart));
         HIPCHK(launch_f64_to_f32(c->acc.p, 3 * c->npart, c->acc32.p, c->stream));
-        HIPCHK(hipMemcpyAsync(out, c->acc32.p, sizeof(float) * 3 * c->npart, hipMemcpyDeviceToHost, c->stream));
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return PP2P_OK;
+    Gather g(c);
+    st = g.add(out, c->acc32.p, sizeof(float) * 3 * (size_t)c->npart);
+    return st ? st : g.finish();
 }
 
 int pp2p_list_stats(pp2p_ctx *c, long long *ntask, long long *nrows, long long *nitems, long long *npairs)
@@ -1928,7 +1937,7 @@ int pp2p_list_stats(pp2p_ctx *c, long long *ntask, long long *nrows, long long *
         return st;
     if (!c->have_particles)
         return fail(PP2P_ERR_STATE, "set_particles before list_stats");
-    if ((st = prepare_form(c, true)))
+    if ((st = prepare_form(c, PP2P_EXEC_QUEUE)))
         return st;
     if (ntask) *ntask = c->ntask;
     if (nrows) *nrows = c->nrows;
@@ -1948,14 +1957,14 @@ int pp2p_get_csr(pp2p_ctx *c, long long *nrows, int *key_sorted, int *src, int *
         return st;
     const size_t n = (size_t)c->ntask, r = (size_t)c->nrows;
     if (n && key_sorted)
-        HIPCHK(hipMemcpyAsync(key_sorted, c->key_sorted.p, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(key_sorted, c->key_sorted.p, sizeof(int) * n, c->stream));
     if (n && src)
-        HIPCHK(hipMemcpyAsync(src, c->src.p, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(src, c->src.p, sizeof(int) * n, c->stream));
     if (r && row_tgt)
-        HIPCHK(hipMemcpyAsync(row_tgt, c->row_tgt.p, sizeof(int) * r, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c->pipe.to_host(row_tgt, c->row_tgt.p, sizeof(int) * r, c->stream));
     if (row_off) {
         if (r)
-            HIPCHK(hipMemcpyAsync(row_off, c->row_off.p, sizeof(int) * (r + 1), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c->pipe.to_host(row_off, c->row_off.p, sizeof(int) * (r + 1), c->stream));
         else
             row_off[0] = 0;
     }
@@ -1974,7 +1983,7 @@ int pp2p_count_inside(pp2p_ctx *c, long long *n_inside)
         return fail(PP2P_ERR_STATE, "set_particles before count_inside");
     if (!n_inside)
         return fail(PP2P_ERR_ARG, "null output");
-    if ((st = prepare_form(c, true)))
+    if ((st = prepare_form(c, PP2P_EXEC_QUEUE)))
         return st;
     HIPCHK(c->pair_count.reserve(1));
     unsigned long long zero = 0, total = 0;
@@ -2007,7 +2016,7 @@ int pp2p_time_steps(pp2p_ctx *c, int exec, int nsteps, double *total_ms, double 
         return fail(PP2P_ERR_ARG, "nsteps >= 1 and a result pointer are required");
     if (exec != PP2P_EXEC_QUEUE && exec != PP2P_EXEC_GRID && exec != PP2P_EXEC_PER_TARGET)
         return fail(PP2P_ERR_ARG, "unknown execution form");
-    if ((st = prepare_form(c, exec == PP2P_EXEC_QUEUE)))
+    if ((st = prepare_form(c, exec)))
         return st;
     (void)queue_groups(c);
     std::vector<hipEvent_t> ev(2 * (size_t)nsteps, nullptr);
@@ -2195,17 +2204,16 @@ int pp2p_pm_forces(pp2p_ctx *c, long long npart, const int *posi, const int *tag
     HIPCHK(c->pm_tag.reserve(std::max(npart, 1ll)));
     HIPCHK(c->pm_acc.reserve(std::max(3 * npart, 1ll)));
     if (npart > 0) {
-        HIPCHK(hipMemcpyAsync(c->pm_posi.p, posi, sizeof(int) * 3 * npart, hipMemcpyHostToDevice, sm));
+        HIPCHK(c->pipe.to_device(c->pm_posi.p, posi, sizeof(int) * 3 * (size_t)npart, sm));
         if (tag)
-            HIPCHK(hipMemcpyAsync(c->pm_tag.p, tag, sizeof(int) * npart, hipMemcpyHostToDevice, sm));
+            HIPCHK(c->pipe.to_device(c->pm_tag.p, tag, sizeof(int) * (size_t)npart, sm));
     }
     const int *p = c->pm_posi.p;
     PmArgs a{p, p + 1, p + 2, 3, tag ? c->pm_tag.p : nullptr, nullptr, npart, int2pos, box, mass, nside};
     if ((st = pm_run(c, a, split_radius, c->pm_acc.p, nullptr, device_ms)))
         return st;
     if (npart > 0) {
-        HIPCHK(hipMemcpyAsync(acc, c->pm_acc.p, sizeof(float) * 3 * npart, hipMemcpyDeviceToHost, sm));
-        HIPCHK(hipStreamSynchronize(sm));
+        HIPCHK(c->pipe.to_host(acc, c->pm_acc.p, sizeof(float) * 3 * (size_t)npart, sm));
     }
     return PP2P_OK;
 }
@@ -2235,8 +2243,6 @@ int pp2p_pm_get_mesh(pp2p_ctx *c, int which, double *out)
     if ((which != 0 && which != 1) || !out)
         return fail(PP2P_ERR_ARG, "which must be 0 (mass) or 1 (potential), with an output array");
     const long long ncell = (long long)c->pm_nside * c->pm_nside * c->pm_nside;
-    HIPCHK(hipMemcpyAsync(out, which == 0 ? c->pm_rho.p : c->pm_pot.p, sizeof(double) * ncell,
-                          hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(c->pipe.to_host(out, which == 0 ? c->pm_rho.p : c->pm_pot.p, sizeof(double) * (size_t)ncell, c->stream));
     return PP2P_OK;
 }
