@@ -87,7 +87,7 @@ typedef struct {
 typedef struct {
     int waves_per_cu;     /* persistent waves per CU (0 = occupancy maximum) */
     int split_pairs;      /* queue items of about this many pair-interactions
-                             (0 = automatic: ~8 items per persistent wave) */
+                             (0 = automatic, from the list's work per wave) */
     int segs_per_octave;  /* table law: 16 or 32 segments per octave of s (0 = 32) */
     int no_cull;          /* 1 disables the per-item j-culling (for measurement) */
     int chunk_model;      /* largest i-chunk of a target per work item: <= 0 the

@@ -264,7 +264,8 @@ __global__ void k_row_cost(RowView v, int nrows, unsigned long long *__restrict_
     if (r < nrows) {
         int ibeg, ni;
         row_i(v, v.row_tgt[r], ibeg, ni);
-        ns = v.nsx[v.row_off[r + 1]] - v.nsx[v.row_off[r]];
+        if (ni > 0)                                  // a row without active targets is no work
+            ns = v.nsx[v.row_off[r + 1]] - v.nsx[v.row_off[r]];
         cost[r] = ns * (unsigned long long)ni;
     }
     for (int o = 32; o > 0; o >>= 1)

@@ -1610,11 +1610,18 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L)
     if (c->tuning.split_pairs > 0) {
         split = c->tuning.split_pairs;
     } else {
-        // about 8 items per persistent wave of the modelled work (pairs and
-        // staging, as the cut counts it), within [2^14, 2^22]
-        const long long waves = (long long)queue_waves(c);
-        const unsigned long long work = tot[0] + (unsigned long long)kStagePairs * tot[1];
-        split = (long long)(work / (unsigned long long)std::max(1ll, 8 * waves));
+        // Items of s = sqrt(1e5 x), x the modelled work (pairs and staging, as
+        // the cut counts it) per persistent wave, within [2^14, 2^22].  An item
+        // costs its wave about 8.5 us (15 000 pair evaluations) beside its work,
+        // a share 15 000 / s of the launch, and the waves end up to an item
+        // apart, a share near 0.15 s / x; the sum is least at this s.  Measured
+        // optima: x = 7.8e4 (32^3 plain) 2^17, 9.5e4 (1e5 uneven pairs) 2^16, 3.8e5
+        // (5% of 96^3) 2^17, 7.4e5 (64^3 plain) from 2^18 on, 8.8e5 (1e6 uneven
+        // pairs) 2^17 to 2^18, 2.1e6 (half of 96^3) 2^19, 1.3e7 (144^3 clustered)
+        // 2^20 on.  Eight items per wave, the rule before, took 159 against 98 us on
+        // the first of them, 199 against 106 on the second.
+        const double x = ((double)tot[0] + (double)kStagePairs * (double)tot[1]) / (double)std::max(1, queue_waves(c));
+        split = (long long)std::sqrt(1e5 * x);
         split = std::max(split, 1ll << 14);
         split = std::min(split, 1ll << 22);
     }
@@ -1623,6 +1630,8 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L)
     int nitems = 0;
     if ((st = fetch(c, &nitems, item_off + nr, sizeof(int))))
         return st;
+    if (nitems == 0)                                 // no target holds an active particle
+        return PP2P_OK;
     unsigned *cost = nullptr, *cost_sorted = nullptr;
     int *idx = nullptr, *idx_sorted = nullptr;
     if ((st = sp.get(c->items_rows, nitems, &L.items_rows)) || (st = sp.get(c->items_q, nitems, &L.items_q)) ||

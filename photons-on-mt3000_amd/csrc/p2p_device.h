@@ -13,6 +13,7 @@ constexpr int kTileCap = 128;        // j-tile capacity per wave (particles)
 
 // LDS of one force-kernel workgroup: one 64 KiB array at LDS address 0.
 //   [0, 16K)       j-tiles, kTileCap float4 per wave
+//   [16K, +16)     the workgroup's share of the item queue
 //   [24K, 32K)     LOGTAB table, 16 segments per octave
 //   [32K, 48K)     source directories, 2 KiB per wave
 //   [48K, 64K)     LOGTAB table, 32 segments per octave
@@ -24,10 +25,13 @@ constexpr int kTileCap = 128;        // j-tile capacity per wave (particles)
 // 160 KiB, 16 waves per CU.
 constexpr int kLdsBytes = 65536;
 constexpr int kLdsTileOff = 0;
+constexpr int kLdsQueueOff = 16384;  // the workgroup's share of the item queue
+constexpr int kQueueBytes = 16;
 constexpr int kLdsDirOff = 32768;
 constexpr int kLdsDirBytes = 2048;   // sizeof(SrcDir)
 __host__ __device__ constexpr int lds_table_off(int seg_shift) { return 96 << (27 - seg_shift); }
-static_assert(kLdsTileOff + kWavesPerGroup * kTileCap * 16 <= 24576, "tiles overlap the 16-segment table");
+static_assert(kLdsTileOff + kWavesPerGroup * kTileCap * 16 <= kLdsQueueOff && kLdsQueueOff + kQueueBytes <= 24576,
+              "tiles or the queue overlap the 16-segment table");
 static_assert(kLdsDirOff + kWavesPerGroup * kLdsDirBytes <= 49152, "directories overlap the 32-segment table");
 // LINEAR law: F(s) = a + b s on 512 segments per binary octave of s, one
 // float2 (a, b) per segment.  Its table outgrows half a CU's LDS, so the
@@ -37,6 +41,7 @@ static_assert(kLdsDirOff + kWavesPerGroup * kLdsDirBytes <= 49152, "directories 
 //                  is at byte (bits(s) >> 11) & 0x1fff8, i.e. 8 x ((biased
 //                  exponent mod 32) * 512 + top 9 mantissa bits); lo = 4 KiB x
 //                  (biased exponent of smin mod 32), and the last entry is s = 1
+//   [127K, +16)    the workgroup's share of the item queue
 //   [128K, 160K)   j-tiles, kTileCap float4 per wave
 // The used octaves must neither wrap (biased exponent of smin >= 96) nor
 // reach the directories (lo >= 24K): smin >= 2^-25, eps / rc >= 2^-12.5.
@@ -47,9 +52,11 @@ constexpr int kLinDirOff = 0;
 constexpr int kLinDirStride = 1536;  // 3 x 64 doubles
 constexpr int kLinTableLo = 24576;   // lowest byte the table may start at
 constexpr int kLinTableEnd = 31 * 4096 + 8;
+constexpr int kLinQueueOff = 130048;
 constexpr int kLinTileOff = 131072;
 static_assert(kLinDirOff + kLinWaves * kLinDirStride <= kLinTableLo, "directories overlap the linear table");
-static_assert(kLinTableEnd <= kLinTileOff, "the linear table overlaps the tiles");
+static_assert(kLinTableEnd <= kLinQueueOff && kLinQueueOff + kQueueBytes <= kLinTileOff,
+              "the linear table overlaps the queue or the tiles");
 static_assert(kLinTileOff + kLinWaves * kTileCap * 16 <= kLinLdsBytes, "tiles outgrow the LDS");
 constexpr int kLogOctaves = 32;      // LOGTAB: cyclic table spans 32 binary octaves of s
 constexpr int kLogSegsMax = 32;      // LOGTAB: segments per octave (16 or 32)

@@ -615,6 +615,34 @@ __device__ __forceinline__ void process_item(const ForceArgs &a, const LawConst 
     }
 }
 
+// The workgroup's share of the item queue: items [next, end) are its waves'.
+struct Queue {
+    unsigned lock;
+    int next, end;
+};
+static_assert(sizeof(Queue) <= kQueueBytes, "queue size");
+
+// The next item for one wave (called by one lane).  The workgroup takes several
+// items from the global counter at a time: every atomic on it takes 12 ns
+// whichever wave asks, which alone was 0.48 of the 0.58 ms of a list of 39 000
+// items (64^3 plain).  A share is a quarter of an even part of what is left, at
+// most one item per wave, so that the last items still go out singly.
+__device__ __forceinline__ int next_item(Queue &q, unsigned *counter, int deal, int nitems, int waves, int groups)
+{
+    while (__hip_atomic_exchange(&q.lock, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP))
+        __builtin_amdgcn_s_sleep(1);
+    int n = __hip_atomic_load(&q.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    const int end = __hip_atomic_load(&q.end, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (n >= end) {
+        const int share = min(max((nitems - end) / (4 * groups), 1), waves);
+        n = deal + (int)atomicAdd(counter, (unsigned)share);
+        __hip_atomic_store(&q.end, n + share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __hip_atomic_store(&q.next, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(&q.lock, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return n;
+}
+
 // Persistent (QUEUE) or one-wave-per-item kernel.  The item's IPL selects
 // one of three specialisations; the branch is uniform per wave.
 template <int LAW, int SOFT, bool FOLD64, bool INDIRECT, bool QUEUE, bool COUNT = false>
@@ -641,6 +669,13 @@ void p2p_force(ForceArgs a, LawConst lc)
     float4 *tile = reinterpret_cast<float4 *>(lds + (kLin ? kLinTileOff : kLdsTileOff)) + wv * kTileCap;
     SrcDir &dir = *reinterpret_cast<SrcDir *>(lds + (kLin ? kLinDirOff + wv * kLinDirStride
                                                          : kLdsDirOff + wv * kLdsDirBytes));
+    Queue *queue = reinterpret_cast<Queue *>(lds + (kLin ? kLinQueueOff : kLdsQueueOff));
+    if (QUEUE) {
+        if (threadIdx.x == 0)
+            *queue = Queue{0u, 0, 0};
+        __syncthreads();
+    }
+
     // QUEUE with deal > 0 (the grid's wave count): the grid's first items are
     // dealt out without the counter, wave v of workgroup b taking item
     // v * gridDim.x + b (a workgroup's waves share a CU, which so starts on
@@ -658,10 +693,10 @@ void p2p_force(ForceArgs a, LawConst lc)
 
     for (;;) {
         if (QUEUE && (!first || !deal)) {
-            unsigned k = 0;
+            int next = 0;
             if (lane == 0)
-                k = atomicAdd(a.counter, 1u);
-            item_id = deal + __builtin_amdgcn_readfirstlane((int)k);
+                next = next_item(*queue, a.counter, deal, a.nitems, kWpg, (int)gridDim.x);
+            item_id = __builtin_amdgcn_readfirstlane(next);
         }
         first = false;
         if (item_id >= a.nitems)

@@ -1,0 +1,60 @@
+"""The item queue at the sizes where its shares change: fewer items than
+waves, a few per wave (the first ones dealt out), tens per wave (shares of
+several items), a grid of one wave per CU; each equals the form with one wave
+per item.  And the automatic item size with targets that hold no active
+particle: as many items as the list of the active targets alone gives."""
+import numpy as np
+import pytest
+
+import photons_p2p as pp
+from photons_p2p import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def work():
+    return W.uneven_pairs(seed=11, lattice=16, n_pool=900, max_src=60, reach=3, total_pairs=20000)
+
+
+def _forces(ctx, w, law, exec_form, **tuning):
+    ctx.set_tuning(**tuning)
+    ctx.set_law(pp.ForceLaw(eps=w.eps, rs=w.rs, softening=w.softening, box=w.box, law=law))
+    ctx.set_particles(w.pos, w.leaf_ip, w.leaf_np)
+    ctx.set_tasks(w.task_t, w.task_s)
+    ctx.compute(exec_form)
+    ctx.compute(exec_form)                           # the queue starts over
+    return ctx.acc(), ctx.list_stats()["nitems"]
+
+
+@pytest.mark.parametrize("law", [pp.LAW_TABLE, pp.LAW_LINEAR, pp.LAW_POLY])
+@pytest.mark.parametrize("waves,split", [(0, 1 << 22), (0, 1 << 15), (0, 1 << 12), (0, 1), (1, 1 << 12), (1, 1), (8, 1)])
+def test_every_item_once(gpu_ctx, work, law, waves, split):
+    print(f"case: law={law} waves_per_cu={waves} split={split}", flush=True)
+    a, n = _forces(gpu_ctx, work, law, pp.EXEC_QUEUE, waves_per_cu=waves, split_pairs=split)
+    b, m = _forces(gpu_ctx, work, law, pp.EXEC_GRID, waves_per_cu=waves, split_pairs=split)
+    assert n == m
+    mag = np.linalg.norm(b, axis=1)
+    assert np.all(np.linalg.norm(a - b, axis=1) <= 1e-12 * np.maximum(mag, 1e-30))
+
+
+@pytest.mark.parametrize("fraction", [0.5, 0.02, 0.0])
+def test_automatic_size_counts_active_targets_only(gpu_ctx, work, fraction):
+    g = np.random.default_rng(5)
+    leaf = g.random(work.nleaf) < fraction
+    act = np.repeat(leaf, work.leaf_np).astype(np.uint8)
+    gpu_ctx.set_tuning()
+    gpu_ctx.set_law(pp.ForceLaw(eps=work.eps, rs=work.rs, softening=work.softening, box=work.box))
+    gpu_ctx.set_particles(work.pos, work.leaf_ip, work.leaf_np)
+    gpu_ctx.set_active(act, 1)
+    gpu_ctx.set_tasks(work.task_t, work.task_s)
+    whole = gpu_ctx.list_stats()["nitems"]
+    gpu_ctx.compute()
+    a = gpu_ctx.acc()
+    gpu_ctx.zero_acc()
+    keep = leaf[work.task_t]
+    gpu_ctx.set_tasks(work.task_t[keep], work.task_s[keep])
+    assert gpu_ctx.list_stats()["nitems"] == whole
+    gpu_ctx.compute()
+    b = gpu_ctx.acc()
+    assert np.all(np.abs(a - b) <= 1e-12 * np.abs(b).max(initial=1e-30))
