@@ -210,6 +210,8 @@ struct pp2p_ctx {
     DevBuf<int> tx0, tx1, tx2, tidx, tla, tlb, tlc, tld, ttag, tposi;
     DevBuf<unsigned long long> tmask;
     DevBuf<int> ttcnt, ttmap;
+    DevBuf<double> tcsum;
+    DevBuf<char> tunits;
     double tree_int2pos = 0.0;  // grid step of the last pp2p_build_tree
     bool tree_ready = false;    // walk arrays, tidx and rng hold the last pp2p_build_tree
     int tree_levels = 0;        // device-wide levels of that tree (tl[0 .. tree_levels))
@@ -378,7 +380,7 @@ void pp2p_destroy(pp2p_ctx *c)
     c->tx0.release(); c->tx1.release(); c->tx2.release(); c->tidx.release(); c->tla.release();
     c->tlb.release(); c->tlc.release(); c->tld.release(); c->ttag.release(); c->tposi.release();
     c->tsub.release(); c->tsuboff.release(); c->tcounts.release();
-    c->tmask.release(); c->ttcnt.release(); c->ttmap.release();
+    c->tmask.release(); c->ttcnt.release(); c->ttmap.release(); c->tcsum.release(); c->tunits.release();
     c->mcenter.release(); c->mM.release(); c->mL.release();
     for (DevBuf<int> *b : {&c->mtt, &c->mts, &c->mkey, &c->msrc, &c->mflag, &c->mrowidx, &c->mrow_tgt, &c->mrow_off})
         b->release();
@@ -982,9 +984,11 @@ static int tree_split_all(pp2p_ctx *c, const TreeScratch &w, long long n, double
             HIPCHK(c->tmask.reserve(nt * (kTreeTile / 64)));
             HIPCHK(c->ttcnt.reserve(nt));
             HIPCHK(c->ttmap.reserve(nt));
+            HIPCHK(c->tcsum.reserve(nt));
+            HIPCHK(c->tunits.reserve(nt * kTreeUnitBytes));
             for (int k = l; k < l + group; ++k)
                 HIPCHK(tree_level(w, tl[k].v, tl[k + 1].v, k, (int)cap(k), tiles(k), int2pos, maxleaf, gmax,
-                                  c->tmask.p, c->ttcnt.p, c->ttmap.p, c->tcounts.p, c->tsub.p,
+                                  c->tcsum.p, c->tunits.p, c->tmask.p, c->ttcnt.p, c->ttmap.p, c->tcounts.p, c->tsub.p,
                                   subs ? (int)subcap : 0, sm));
             if ((st = fetch(c, &h, c->tcounts.p, sizeof(int) * (size_t)(2 + l + group + 1))))
                 return st;

@@ -7,6 +7,7 @@ namespace pp2p {
 constexpr int kSubMax = 4096;       // particles of a subtree built in one workgroup's LDS
 constexpr int kSubLevels = 1024;    // levels of one subtree (the depth limit of a tree)
 constexpr int kTreeTile = 4096;     // positions per block of the level passes
+constexpr int kTreeUnitBytes = 64 * 24; // sums of a tile's samples, per group of 64
 constexpr int kSubKid = 1 << 30;    // son codes from here on name subtrees
 
 // Per-particle arrays of the build (n entries each, n + 1 where a caller
@@ -67,11 +68,12 @@ hipError_t tree_init(const int *posi, long long n, const TreeScratch &w, TreeCou
 // One level (level < 1024): split values, partition (particles permuted in
 // place), and the next level's segments, this level's leaves and the new
 // subtrees.  cap: most segments the level can hold, tiles: most tiles.
-// mask: 64 words per tile, tcnt and tmap: one int per tile.  More than subcap
-// subtrees in all count as a misfit.
+// Per tile: csum one double, units kTreeUnitBytes, mask 64 words, tcnt and tmap one
+// int.  More than subcap subtrees in all count as a misfit.
 hipError_t tree_level(const TreeScratch &w, const TreeLevelView &lv, const TreeLevelView &nx, int level, int cap,
-                      long long tiles, double int2pos, int maxleaf, int gmax, unsigned long long *mask, int *tcnt,
-                      int *tmap, TreeCounts *counts, TreeSub *sub, int subcap, hipStream_t st);
+                      long long tiles, double int2pos, int maxleaf, int gmax, double *csum, void *units,
+                      unsigned long long *mask, int *tcnt, int *tmap, TreeCounts *counts, TreeSub *sub, int subcap,
+                      hipStream_t st);
 // The subtrees: particles permuted in place, records and sizes; level
 // offsets of subtree s at off[s * kSubLevels].
 hipError_t tree_subs(const TreeScratch &w, TreeSub *sub, int nsub, double int2pos, int maxleaf, unsigned short *off,

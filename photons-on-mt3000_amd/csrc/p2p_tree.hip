@@ -199,118 +199,87 @@ __device__ double add_run(double s, const double (&v)[kV], int lane)
     return s;
 }
 
-// ------------------------------------------------------------- level passes
+// Sums of long segments take three steps, so that all but the last run in
+// parallel: plain sums of groups of 64 values say in which binade each group
+// starts (nearly always; a wrong guess only costs time), every group is turned
+// into units of that binade, and one wave composes the groups in order, 64 at a
+// time by a prefix sum.  A group that leaves its binade or was guessed wrong is
+// added by itself from its values.
+constexpr int kGroup = 64;
 
-// Split value of each segment (src/fmm.c:168-197): the sampled FP64 mean for
-// more than two particles, the midpoint of two, 0 for fewer.  One block per
-// segment; the samples come 4096 at a time, the next ones loading meanwhile.
-// Each wave turns its 512 values into integers and round-ups, which every thread
-// then adds in wave order.  Bound by latency: 25 batches in a row above 10^5
-// particles, and about one more pass per binade.  256^3 clustered tree (1.9 10^7
-// particles, 16 levels): 140 us per level; one wave per segment adding its
-// samples one after the other (about 19 cycles each) took 433 us per level
-// over 23 levels.
-constexpr int kMeanThreads = 512;
-constexpr int kMeanValues = 8;
-constexpr int kMeanBatch = kMeanThreads * kMeanValues;
+// info: 0 where the rule does not apply, else the start's sign and exponent
+// (bits 11 to 22) and the SeqTies of the group (any, first, out, rest)
+struct GroupUnits {
+    double up, down;
+    int info;
+};
 
-__global__ __launch_bounds__(kMeanThreads) void k_tree_mean(TreeLevelView lv, const int *__restrict__ nseg,
-                                                          const int *__restrict__ x, double int2pos)
+__device__ __forceinline__ int binade_of(double s)
 {
-    constexpr int kWaves = kMeanThreads / 64;
-    __shared__ double2 sums[kWaves];
-    __shared__ int4 runs[kWaves];                    // SeqTies of each wave
-    __shared__ double s_sum;
-    const int s = blockIdx.x;
-    if (s >= *nseg)
-        return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int a = lv.seg[s].x, len = lv.seg[s].y;
-    double m = 0.0;
-    float sp = 0.0f;
-    if (len > 2) {
-        const long long mul = len > 100000 ? len / 100000 : 1;
-        const int ns = (int)((len + mul - 1) / mul);
-        int r[kMeanValues];
-        // a thread's values are consecutive
-        auto at = [&](int u) { return (int)threadIdx.x * kMeanValues + u; };
-        auto load = [&](int b) {
-#pragma unroll
-            for (int u = 0; u < kMeanValues; ++u) {
-                const int k = b + at(u);
-                r[u] = x[a + (k < ns ? k : ns - 1) * mul];
-            }
-        };
-        load(0);
-        for (int b = 0; b < ns; b += kMeanBatch) {
-            double v[kMeanValues];
-#pragma unroll
-            for (int u = 0; u < kMeanValues; ++u)
-                v[u] = b + at(u) < ns ? int2pos * (double)r[u] : 0.0;
-            if (b + kMeanBatch < ns)
-                load(b + kMeanBatch);
-            // the waves' values in turn: all that keep the sum in its binade at
-            // once, then the wave that does not by itself, then on with the rest
-            int next = 0;
-            while (next < kWaves) {
-                const double scale = seq_scale(m);
-                __syncthreads();                     // the previous pass's reads
-                if (scale != 0.0 && wave >= next) {
-                    double up, down;
-                    const SeqTies run = lane_units(v, m < 0.0 ? -scale : scale, up, down);
-                    SeqTies all;
-                    if (__ballot(run.any)) {
-                        lanes_parity(run, 0, lane, all);
-                        for (int o = 32; o > 0; o >>= 1)
-                            all.rest += __shfl_xor(all.rest, o, 64);
-                    } else {
-                        all.out = __popcll(__ballot(run.out)) & 1;
-                    }
-                    up = wave_sum(up);
-                    down = wave_sum(down);
-                    if (lane == 0) {
-                        sums[wave] = make_double2(up, down);
-                        runs[wave] = make_int4(all.any, all.first, all.rest, all.out);
-                    }
-                }
-                __syncthreads();
-                if (scale != 0.0) {
-                    double S = fabs(m) * scale;
-                    int p = seq_parity(m);
-                    for (; next < kWaves; ++next) {
-                        const double2 ud = sums[next];
-                        const int4 q = runs[next];
-                        const double up = ud.x + (double)seq_roundups(SeqTies{q.x, q.y, q.z, q.w}, p);
-                        if (!seq_inside(S, up, ud.y))
-                            break;
-                        S = S + up - ud.y;
-                    }
-                    const double t = S * seq_unit(scale);
-                    m = m < 0.0 ? -t : t;
-                }
-                if (next < kWaves) {
-                    if (wave == next) {
-                        const double t = add_run(m, v, lane);
-                        if (lane == 0)
-                            s_sum = t;
-                    }
-                    __syncthreads();
-                    m = s_sum;
-                    ++next;
-                }
-            }
-        }
-        m /= (double)len;
-        m *= (double)mul;
-        sp = (float)m;
-    } else if (len == 2) {
-        sp = (float)(0.5 * (int2pos * (double)(x[a] + x[a + 1])));
-    }
-    if (threadIdx.x == 0) {
-        lv.mean[s] = m;
-        lv.split[s] = sp;
-    }
+    return seq_scale(s) == 0.0 ? 0 : (int)((unsigned long long)__double_as_longlong(s) >> 52) << 11;
 }
+
+// The wave's 64 values (+0.0 past the end) as units of the binade of `start`.
+__device__ __forceinline__ GroupUnits group_units(double v, double start, int lane)
+{
+    GroupUnits g{0.0, 0.0, binade_of(start)};
+    if (!g.info)
+        return g;
+    const double scale = seq_scale(start), one[1] = {v};
+    const SeqTies run = lane_units(one, start < 0.0 ? -scale : scale, g.up, g.down);
+    SeqTies all;
+    if (__ballot(run.any)) {
+        lanes_parity(run, 0, lane, all);
+        all.rest = __popcll(__ballot(all.rest));
+    } else {
+        all.out = __popcll(__ballot(run.out)) & 1;
+    }
+    g.up = wave_sum(g.up);
+    g.down = wave_sum(g.down);
+    g.info |= all.any | all.first << 1 | all.out << 2 | all.rest << 3;
+    return g;
+}
+
+// s + the cnt <= 64 groups from `base` on, the same in every lane: u is the
+// lane's group, value(g) the lane's value of group g.
+template <class Value>
+__device__ __forceinline__ double add_groups(double s, const GroupUnits &u, int base, int cnt, int lane, Value value)
+{
+    int next = 0;
+    while (next < cnt) {
+        const double scale = seq_scale(s), S = fabs(s) * scale;
+        const int at = binade_of(s);
+        const bool mine = lane >= next && lane < cnt && at && (u.info >> 11) == (at >> 11);
+        SeqTies run, all;
+        double up = 0.0, down = 0.0;
+        if (mine) {
+            run.any = u.info & 1;
+            run.first = u.info >> 1 & 1;
+            run.out = u.info >> 2 & 1;
+            run.rest = u.info >> 3 & 0xff;
+            up = u.up;
+            down = u.down;
+        }
+        int p = lanes_parity(run, seq_parity(s), lane, all);
+        up += (double)seq_roundups(run, p);
+        const double inc = up - down, t = wave_prefix(inc);
+        const unsigned long long bad =
+            __ballot(!mine || !seq_inside(S + (t - inc), up, down)) & (~0ull << next) & (~0ull >> (64 - cnt));
+        const int first = bad ? __builtin_ctzll(bad) : cnt;
+        if (first > next) {
+            const double m = (S + lane_value(t, first - 1)) * seq_unit(scale);
+            s = s < 0.0 ? -m : m;
+        }
+        if (first < cnt) {
+            const double one[1] = {value(base + first)};
+            s = add_run(s, one, lane);
+        }
+        next = first + 1;
+    }
+    return s;
+}
+
+// ------------------------------------------------------------- level passes
 
 // the segment holding a tile: the last s with toff[s] <= tile
 __device__ __forceinline__ int seg_of_tile(const int *__restrict__ toff, int nseg, int tile)
@@ -326,18 +295,161 @@ __device__ __forceinline__ int seg_of_tile(const int *__restrict__ toff, int nse
     return lo;
 }
 
+// Split values (src/fmm.c:168-197): the sampled FP64 mean for more than two
+// particles, the midpoint of two, 0 for fewer.  A segment's samples (all
+// particles, or every (len / 10^5)-th) in chunks of 4096: sums of the chunks, the
+// groups of each chunk in units, and one wave per segment that composes them.
+// The first two are bound by HBM, the last by the chain of about ten groups that
+// change the binade, 2 us each with the load of their samples.  One workgroup
+// per segment doing all of it, one 4096 values after the other, was bound by
+// the loads and the rounding of a single CU where the segments are few: 9 levels of
+// 64^3 took 625 us and take 390, 16 of 256^3 (clustered) 2500 and take 1950.
+struct Samples {
+    const int *x;                                    // the segment's coordinates
+    long long mul;
+    int ns, chunks;
+    double int2pos;
+    __device__ Samples(const int *coord, int2 seg, double step) : x(coord + seg.x), mul(1), int2pos(step)
+    {
+        if (seg.y > 100000)
+            mul = seg.y / 100000;
+        ns = seg.y > 2 ? (int)((seg.y + mul - 1) / mul) : 0;
+        chunks = (ns + kTreeTile - 1) / kTreeTile;   // at most 49, and at most the segment's tiles
+    }
+    // sample k, +0.0 past the end
+    __device__ double operator()(int k) const
+    {
+        const int r = x[(k < ns ? k : ns - 1) * mul];
+        return k < ns ? int2pos * (double)r : 0.0;
+    }
+};
+
+// plain sums of the chunks; tmap[tile] = the tile's segment
+__global__ __launch_bounds__(kTreeBlock) void k_tree_sums(TreeLevelView lv, const int *__restrict__ nseg,
+                                                        const int *__restrict__ x, double int2pos,
+                                                        double *__restrict__ csum, int *__restrict__ tmap)
+{
+    __shared__ double part[kTreeBlock / 64];
+    const int n = *nseg, tile = blockIdx.x;
+    if (n == 0 || tile >= lv.toff[n])
+        return;
+    const int s = seg_of_tile(lv.toff, n, tile);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0)
+        tmap[tile] = s;
+    const Samples v(x, lv.seg[s], int2pos);
+    const int c = tile - lv.toff[s];
+    if (c >= v.chunks)
+        return;
+    double sum = 0.0;
+#pragma unroll
+    for (int u = 0; u < kTreeTile / kTreeBlock; ++u)
+        sum += v(c * kTreeTile + u * kTreeBlock + (int)threadIdx.x);
+    sum = wave_sum(sum);
+    if (lane == 0)
+        part[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kTreeBlock / 64; ++q)
+            sum += part[q];
+        csum[tile] = sum;
+    }
+}
+
+// the groups of each chunk in units
+__global__ __launch_bounds__(kTreeBlock) void k_tree_units(TreeLevelView lv, const int *__restrict__ nseg,
+                                                         const int *__restrict__ x, double int2pos,
+                                                         const double *__restrict__ csum,
+                                                         const int *__restrict__ tmap,
+                                                         GroupUnits *__restrict__ units)
+{
+    constexpr int kGroups = kTreeTile / kGroup, kPerWave = kGroups / (kTreeBlock / 64);
+    __shared__ double start[kGroups];
+    const int n = *nseg, tile = blockIdx.x;
+    if (n == 0 || tile >= lv.toff[n])
+        return;
+    const int s = tmap[tile];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const Samples v(x, lv.seg[s], int2pos);
+    const int t0 = lv.toff[s], c = tile - t0;
+    if (c >= v.chunks)
+        return;
+    double mine[kPerWave];
+#pragma unroll
+    for (int u = 0; u < kPerWave; ++u)
+        mine[u] = v(c * kTreeTile + (wave * kPerWave + u) * kGroup + lane);
+#pragma unroll
+    for (int u = 0; u < kPerWave; ++u) {
+        const double g = wave_sum(mine[u]);
+        if (lane == 0)
+            start[wave * kPerWave + u] = g;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const double before = wave_sum(lane < c ? csum[t0 + lane] : 0.0);
+        const double g = start[lane];
+        start[lane] = before + (wave_prefix(g) - g);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPerWave; ++u) {
+        const int g = wave * kPerWave + u;
+        const GroupUnits r = group_units(mine[u], start[g], lane);
+        if (lane == 0)
+            units[(long long)tile * kGroups + g] = r;
+    }
+}
+
+constexpr int kAhead = 4;                            // batches of groups loaded together
+
+__global__ __launch_bounds__(64) void k_tree_mean(TreeLevelView lv, const int *__restrict__ nseg,
+                                                const int *__restrict__ x, double int2pos,
+                                                const GroupUnits *__restrict__ units)
+{
+    const int s = blockIdx.x, lane = threadIdx.x;
+    if (s >= *nseg)
+        return;
+    const int2 sg = lv.seg[s];
+    const Samples v(x, sg, int2pos);
+    double m = 0.0;
+    float sp = 0.0f;
+    if (sg.y > 2) {
+        const GroupUnits *u = units + (long long)lv.toff[s] * (kTreeTile / kGroup);
+        const int ng = (v.ns + kGroup - 1) / kGroup;
+        for (int base = 0; base < ng; base += kAhead * 64) {
+            GroupUnits r[kAhead];                    // loads in flight together
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q)
+                r[q] = u[min(base + q * 64 + lane, ng - 1)];
+#pragma unroll
+            for (int q = 0; q < kAhead; ++q)
+                m = add_groups(m, r[q], base + q * 64, min(64, ng - base - q * 64), lane,
+                               [&](int g) { return v(g * kGroup + lane); });
+        }
+        m /= (double)sg.y;
+        m *= (double)v.mul;
+        sp = (float)m;
+    } else if (sg.y == 2) {
+        sp = (float)(0.5 * (int2pos * (double)(x[sg.x] + x[sg.x + 1])));
+    }
+    if (lane == 0) {
+        lv.mean[s] = m;
+        lv.split[s] = sp;
+    }
+}
+
 // Masks of the particles at or below the mean, 64 words and their total per
-// tile of kTreeTile positions of one segment; tmap[tile] = the segment.
+// tile of kTreeTile positions of one segment.
 __global__ __launch_bounds__(kTreeBlock) void k_tree_flags(TreeLevelView lv, const int *__restrict__ nseg,
                                                          const int *__restrict__ x, double int2pos,
                                                          unsigned long long *__restrict__ mask,
-                                                         int *__restrict__ tcnt, int *__restrict__ tmap)
+                                                         int *__restrict__ tcnt, const int *__restrict__ tmap)
 {
     __shared__ int part[kTreeBlock / 64];
     const int ns = *nseg, tile = blockIdx.x;
     if (ns == 0 || tile >= lv.toff[ns])
         return;
-    const int s = seg_of_tile(lv.toff, ns, tile);
+    const int s = tmap[tile];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int2 sg = lv.seg[s];
     const double mean = lv.mean[s];
@@ -369,7 +481,6 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_flags(TreeLevelView lv, con
         for (int q = 0; q < kTreeBlock / 64; ++q)
             t += part[q];
         tcnt[tile] = t;
-        tmap[tile] = s;
     }
 }
 
@@ -612,6 +723,7 @@ struct SubNumber {
     unsigned short id[kSubMax], leaf0[kSubMax];
     unsigned short up[kSubMax];                      // parent << 1 | side
 };
+static_assert(sizeof(GroupUnits) * (kTreeTile / kGroup) == kTreeUnitBytes, "tile record");
 static_assert(sizeof(SubNumber) <= sizeof(SubLds::x), "numbering overlaps more than the coordinates");
 
 __device__ __forceinline__ int sub_small_before(const SubLds &m, int p)
@@ -1106,13 +1218,17 @@ hipError_t tree_init(const int *posi, long long n, const TreeScratch &w, TreeCou
 }
 
 hipError_t tree_level(const TreeScratch &w, const TreeLevelView &lv, const TreeLevelView &nx, int level, int cap,
-                      long long tiles, double int2pos, int maxleaf, int gmax, unsigned long long *mask, int *tcnt,
-                      int *tmap, TreeCounts *counts, TreeSub *sub, int subcap, hipStream_t st)
+                      long long tiles, double int2pos, int maxleaf, int gmax, double *csum, void *units,
+                      unsigned long long *mask, int *tcnt, int *tmap, TreeCounts *counts, TreeSub *sub, int subcap,
+                      hipStream_t st)
 {
     const int *ns = &counts->nseg[level];
     const int *x = w.x[level % 3];
     const unsigned nt = (unsigned)tiles;
-    k_tree_mean<<<(unsigned)cap, kMeanThreads, 0, st>>>(lv, ns, x, int2pos);
+    GroupUnits *u = reinterpret_cast<GroupUnits *>(units);
+    k_tree_sums<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap);
+    k_tree_units<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap, u);
+    k_tree_mean<<<(unsigned)cap, 64, 0, st>>>(lv, ns, x, int2pos, u);
     k_tree_flags<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, mask, tcnt, tmap);
     k_tree_lists<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, mask, tcnt, tmap, w.la, w.lb);
     k_tree_swap<<<nt, kTreeBlock, 0, st>>>(lv, ns, tmap, w);

@@ -116,3 +116,15 @@ def test_multipoles_of_levels_and_subtrees(gpu_ctx, kind, n, maxleaf):
                                       Lf[nl + k], Lf[cell(sn)])
     scale = np.abs(Lf).max(0) + 1e-30
     assert np.all(np.abs(L - Lf) <= 5e-5 * scale)
+
+
+# means over several tiles: about the sampled strides (1, then 2) and a whole tile,
+# with coordinates of both signs (sums that cross zero) or far from it
+@pytest.mark.parametrize("n", [8191, 8192, 12289, 199999, 200000, 200001])
+@pytest.mark.parametrize("offset", [0, 1 << 29])
+def test_means_over_tiles(gpu_ctx, n, offset):
+    print(f"case: n={n} offset={offset}", flush=True)
+    g = np.random.default_rng(n)
+    posi = g.integers(-(1 << 27), 1 << 27, (n, 3)) + offset
+    for k, step in enumerate(STEPS):
+        _same(gpu_ctx, posi, step, 1000, n + k)
