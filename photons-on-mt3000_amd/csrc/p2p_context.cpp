@@ -2177,7 +2177,7 @@ static int pm_run(pp2p_ctx *c, const PmArgs &a, float split_radius, float *acc32
         return st;
     HIPCHK(c->pm_rho.reserve(ncell));
     HIPCHK(c->pm_pot.reserve(ncell));
-    HIPCHK(c->pm_grad.reserve(3 * ncell));
+    HIPCHK(c->pm_grad.reserve(3 * (ncell + (long long)nside * nside)));
     HIPCHK(c->pm_spec.reserve(nspec));
     if (!c->ev_m0) {
         HIPCHK(hipEventCreate(&c->ev_m0));

@@ -21,7 +21,7 @@ hipError_t pm_deposit(const PmArgs &a, double *rho, hipStream_t st);
 // spec[N][N][N/2+1] *= G(k) (the long-range Green's function with the CIC
 // deconvolution and the mass-per-cell-to-density factor (N / box)^3; spec[0] = 0).
 hipError_t pm_green(int nside, float split_radius, float box, double2 *spec, hipStream_t st);
-// grad[3][N^3] = 4-point gradient of pot[N^3] per cell, interpolated with the
+// grad[N][N][N + 1][3] = 4-point gradient of pot[N^3] per cell, interpolated with the
 // CIC weights: acc32 != null stores acc32[3][n] (SoA, zero for particles that
 // are not local); else acc64[3][n] += the local particles' accelerations.
 hipError_t pm_interp(const PmArgs &a, const double *pot, double *grad, float *acc32, double *acc64,
