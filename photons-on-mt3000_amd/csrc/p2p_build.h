@@ -36,6 +36,20 @@ hipError_t launch_planes_to_rows(const double *a, long long n, double *out, hipS
 // n packed triples to float4 (w = 0), and back
 hipError_t launch_pack_xyz(const float *a, int n, float4 *out, hipStream_t st);
 hipError_t launch_unpack_xyz(const float4 *a, int n, float *out, hipStream_t st);
+// Small arrays to pinned host memory by one kernel, which then writes `ticket`
+// into the host word `flag`.
+constexpr int kMailParts = 12;
+struct MailPart {
+    const void *src;            // 4-byte aligned
+    unsigned at;                // byte offset in the mailbox, a multiple of 16
+    unsigned words;             // 4-byte words written
+    bool round;                 // src holds doubles, written as floats
+};
+struct MailList {
+    MailPart part[kMailParts];
+    int n;
+};
+hipError_t launch_mail(const MailList &list, void *box, unsigned *flag, unsigned ticket, hipStream_t st);
 // n pairs to two planes
 hipError_t launch_split_pairs(const int2 *a, int n, int *x, int *y, hipStream_t st);
 hipError_t launch_fill_i32(int *p, long long n, int v, hipStream_t st);

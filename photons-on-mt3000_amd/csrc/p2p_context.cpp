@@ -5,6 +5,7 @@
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -43,7 +44,7 @@ int fail(int code, const std::string &msg)
     } while (0)
 
 // small results: sizes read between launches, the arrays of a small tree
-constexpr size_t kMailBytes = 128 << 10;
+constexpr size_t kMailBytes = 512 << 10;
 
 // grow-only device buffer
 template <typename T>
@@ -73,7 +74,7 @@ struct DevBuf {
     }
 };
 
-// pinned host buffer (small results that the host waits for)
+// pinned host buffer that kernels write (small results that the host waits for)
 struct PinnedBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -82,7 +83,7 @@ struct PinnedBuf {
         if (bytes <= cap)
             return hipSuccess;
         release();
-        hipError_t e = hipHostMalloc(&p, std::max<size_t>(bytes, 1), hipHostMallocDefault);
+        hipError_t e = hipHostMalloc(&p, std::max<size_t>(bytes, 1), hipHostMallocMapped | hipHostMallocCoherent);
         if (e == hipSuccess)
             cap = bytes;
         else
@@ -136,7 +137,8 @@ struct pp2p_ctx {
     DevBuf<double> x3;          // FP64 staging of positions
     DevBuf<int> posi;           // int32 staging
     HostPipe pipe;              // large host copies
-    PinnedBuf mail;             // small ones back, allocated with the context
+    PinnedBuf mail;             // small ones back (the flag, then kMailBytes), allocated with the context
+    unsigned ticket = 0;        // of the last mail
     DevBuf<double> acc3;        // AoS copy of acc for pp2p_get_acc_f64
     DevBuf<float> xyz;          // packed triples on their way in or out
     DevBuf<int> pair_a, pair_b; // planes of int2 arrays on their way out
@@ -253,63 +255,74 @@ static int ensure_temp(pp2p_ctx *c, size_t bytes)
     return PP2P_OK;
 }
 
-// Waits for the stream with `bytes` from src in dst: through the pinned mailbox
-// when they fit (a copy to pageable memory is staged and waited for by the
-// runtime first).
-static int fetch(pp2p_ctx *c, void *dst, const void *src, size_t bytes)
-{
-    if (bytes > c->mail.cap) {
-        HIPCHK(c->pipe.to_host(dst, src, bytes, c->stream));
-        return PP2P_OK;
-    }
-    HIPCHK(hipMemcpyAsync(c->mail.p, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    std::memcpy(dst, c->mail.p, bytes);
-    return PP2P_OK;
-}
+// Several device arrays to the host with one wait: what fits the pinned mailbox
+// is put there by one kernel, whose flag the host polls.  After kMailSpin without
+// it the host waits for the stream, which also reports errors.
+constexpr auto kMailSpin = std::chrono::microseconds(200);
 
-// Several device arrays to the host with one wait where they fit the mailbox.
 class Gather {
 public:
-    explicit Gather(pp2p_ctx *c) : c_(c) {}
-    int add(void *dst, const void *src, size_t bytes)
-    {
-        if (!dst || !bytes)
-            return PP2P_OK;
-        if (bytes > c_->mail.cap - used_) {
-            int st = finish();
-            if (st)
-                return st;
-            if (bytes > c_->mail.cap) {
-                HIPCHK(c_->pipe.to_host(dst, src, bytes, c_->stream));
-                return PP2P_OK;
-            }
-        }
-        HIPCHK(hipMemcpyAsync(static_cast<char *>(c_->mail.p) + used_, src, bytes, hipMemcpyDeviceToHost, c_->stream));
-        parts_.push_back({dst, used_, bytes});
-        used_ += (bytes + 15) & ~(size_t)15;
-        used_ = std::min(used_, c_->mail.cap);
-        return PP2P_OK;
-    }
+    explicit Gather(pp2p_ctx *c) : c_(c) { list_.n = 0; }
+    int add(void *dst, const void *src, size_t bytes) { return put(dst, src, bytes, false); }
+    // n doubles of src as floats; 4 n bytes must fit the mailbox
+    int add_round(float *dst, const double *src, size_t n) { return put(dst, src, sizeof(float) * n, true); }
     int finish()
     {
-        HIPCHK(hipStreamSynchronize(c_->stream));
-        for (const Part &p : parts_)
-            std::memcpy(p.dst, static_cast<const char *>(c_->mail.p) + p.at, p.bytes);
-        parts_.clear();
+        if (!list_.n) {
+            HIPCHK(hipStreamSynchronize(c_->stream));
+            return PP2P_OK;
+        }
+        unsigned *flag = static_cast<unsigned *>(c_->mail.p);
+        char *box = static_cast<char *>(c_->mail.p) + 64;
+        const unsigned ticket = ++c_->ticket;
+        HIPCHK(launch_mail(list_, box, flag, ticket, c_->stream));
+        const auto end = std::chrono::steady_clock::now() + kMailSpin;
+        while (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != ticket) {
+            if (std::chrono::steady_clock::now() < end)
+                continue;
+            HIPCHK(hipStreamSynchronize(c_->stream));
+            break;
+        }
+        for (int q = 0; q < list_.n; ++q)
+            std::memcpy(dst_[q], box + list_.part[q].at, sizeof(int) * (size_t)list_.part[q].words);
+        list_.n = 0;
         used_ = 0;
         return PP2P_OK;
     }
 
 private:
-    struct Part {
-        void *dst;
-        size_t at, bytes;
-    };
+    int put(void *dst, const void *src, size_t bytes, bool round)
+    {
+        if (!dst || !bytes)
+            return PP2P_OK;
+        if (list_.n && (bytes > kMailBytes - used_ || list_.n == kMailParts)) {
+            int st = finish();
+            if (st)
+                return st;
+        }
+        if (bytes > kMailBytes) {
+            HIPCHK(c_->pipe.to_host(dst, src, bytes, c_->stream));
+            return PP2P_OK;
+        }
+        dst_[list_.n] = dst;
+        list_.part[list_.n++] = MailPart{src, (unsigned)used_, (unsigned)(bytes / sizeof(int)), round};
+        used_ = std::min(kMailBytes, (used_ + bytes + 15) & ~(size_t)15);
+        return PP2P_OK;
+    }
+
     pp2p_ctx *c_;
-    std::vector<Part> parts_;
+    MailList list_;
+    void *dst_[kMailParts];
     size_t used_ = 0;
 };
+
+// Waits for `bytes` (a multiple of 4) from src in dst.
+static int fetch(pp2p_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    Gather g(c);
+    const int st = g.add(dst, src, bytes);
+    return st ? st : g.finish();
+}
 
 extern "C" {
 
@@ -342,12 +355,13 @@ pp2p_ctx *pp2p_create(int device, int *status)
             hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreate(&c->ev_k0) != hipSuccess || hipEventCreate(&c->ev_k1) != hipSuccess ||
             hipEventCreate(&c->ev_p0) != hipSuccess || hipEventCreate(&c->ev_p1) != hipSuccess ||
-            c->counter.reserve(1) != hipSuccess || c->mail.reserve(kMailBytes) != hipSuccess) {
+            c->counter.reserve(1) != hipSuccess || c->mail.reserve(64 + kMailBytes) != hipSuccess) {
             st = fail(PP2P_ERR_DEVICE, "context creation failed");
             pp2p_destroy(c);
             c = nullptr;
         } else {
             c->num_cu = prop.multiProcessorCount;
+            std::memset(c->mail.p, 0, c->mail.cap);      // no ticket yet; the pages are there
             // once per device, with the device current; a failure only
             // disables pp2p_compute_noalloc
             if (scratch_address(device, &c->scratch) != hipSuccess)
@@ -1011,13 +1025,11 @@ static int tree_split_all(pp2p_ctx *c, const TreeScratch &w, long long n, double
     HIPCHK(tree_subs(w, c->tsub.p, *nsub, int2pos, maxleaf, c->tsuboff.p, c->tcounts.p, sm));
     for (int l = last; l >= 0; --l)
         HIPCHK(tree_below(tl[l].v, tl[l].nseg, l < last ? tl[l + 1].v.below : nullptr, c->tsub.p, sm));
-    int *mail = static_cast<int *>(c->mail.p);
-    HIPCHK(hipMemcpyAsync(mail, &c->tcounts.p->misfit, sizeof(int), hipMemcpyDeviceToHost, sm));
-    HIPCHK(hipMemcpyAsync(mail + 2, root_sub ? (const void *)&c->tsub.p->nnode : (const void *)tl[0].v.below,
-                          sizeof(int2), hipMemcpyDeviceToHost, sm));
-    HIPCHK(hipStreamSynchronize(sm));
-    *counts = make_int2(mail[2], mail[3]);
-    h.misfit = mail[0];
+    Gather g(c);
+    if ((st = g.add(&h.misfit, &c->tcounts.p->misfit, sizeof(int))) ||
+        (st = g.add(counts, root_sub ? (const void *)&c->tsub.p->nnode : (const void *)tl[0].v.below, sizeof(int2))) ||
+        (st = g.finish()))
+        return st;
     *fits = h.misfit == 0;
     return PP2P_OK;
 }
@@ -1934,12 +1946,15 @@ int pp2p_get_acc_f32_soa(pp2p_ctx *c, float *out)
     if (!out && c->npart)
         return fail(PP2P_ERR_ARG, "null output");
     // rounded to FP32 on the device: half the bytes over the bus, no host pass
-    if (c->npart) {
-        HIPCHK(c->acc32.reserve((size_t)3 * c->npart));
-        HIPCHK(launch_f64_to_f32(c->acc.p, 3 * c->npart, c->acc32.p, c->stream));
-    }
+    const size_t n = (size_t)3 * c->npart;
     Gather g(c);
-    st = g.add(out, c->acc32.p, sizeof(float) * 3 * (size_t)c->npart);
+    if (sizeof(float) * n <= kMailBytes) {
+        st = g.add_round(out, c->acc.p, n);
+    } else {
+        HIPCHK(c->acc32.reserve(n));
+        HIPCHK(launch_f64_to_f32(c->acc.p, n, c->acc32.p, c->stream));
+        st = g.add(out, c->acc32.p, sizeof(float) * n);
+    }
     return st ? st : g.finish();
 }
 
