@@ -645,15 +645,17 @@ static_assert(sizeof(Queue) <= kQueueBytes, "queue size");
 // items from the global counter at a time: every atomic on it takes 12 ns
 // whichever wave asks, which alone was 0.48 of the 0.58 ms of a list of 39 000
 // items (64^3 plain).  A share is a quarter of an even part of what is left, at
-// most one item per wave, so that the last items still go out singly.
+// most one item per wave, so that the last items still go out singly.  Once the
+// counter has run out the workgroup does not ask again: with an atomic of each
+// of 4096 waves at the end a launch of 5900 items took 81 us, now 57.
 __device__ __forceinline__ int next_item(Queue &q, unsigned *counter, int deal, int nitems, int waves, int groups)
 {
     while (__hip_atomic_exchange(&q.lock, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP))
         __builtin_amdgcn_s_sleep(1);
     int n = __hip_atomic_load(&q.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     const int end = __hip_atomic_load(&q.end, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (n >= end) {
-        const int share = min(max((nitems - end) / (4 * groups), 1), waves);
+    if (n >= end && end < nitems) {                  // end >= nitems: the counter has run out
+        const int share = min(max((nitems - max(end, deal)) / (4 * groups), 1), waves);
         n = deal + (int)atomicAdd(counter, (unsigned)share);
         __hip_atomic_store(&q.end, n + share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -726,7 +728,8 @@ void p2p_force(ForceArgs a, LawConst lc)
         case 2: process_item<2, LAW, SOFT, FOLD64, INDIRECT, COUNT>(a, lc, it, lds, tile, dir, lane, n_in); break;
         default: process_item<3, LAW, SOFT, FOLD64, INDIRECT, COUNT>(a, lc, it, lds, tile, dir, lane, n_in); break;
         }
-        if (!QUEUE)
+        // a grid with a wave for every item is dealt all of them
+        if (!QUEUE || deal >= a.nitems)
             break;
     }
     if (COUNT) {

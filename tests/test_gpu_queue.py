@@ -58,3 +58,28 @@ def test_automatic_size_counts_active_targets_only(gpu_ctx, work, fraction):
     gpu_ctx.compute()
     b = gpu_ctx.acc()
     assert np.all(np.abs(a - b) <= 1e-12 * np.abs(b).max(initial=1e-30))
+
+
+# a list of `items` rows of one item each: fewer than workgroups, than waves (every item
+# dealt, no counter), one more than either, for grids of 16 waves per CU and of one
+@pytest.mark.parametrize("items", [1, 2, 255, 256, 257, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4097, 5000])
+@pytest.mark.parametrize("waves", [0, 1])
+@pytest.mark.parametrize("law", [pp.LAW_TABLE, pp.LAW_LINEAR])
+def test_small_lists(gpu_ctx, items, waves, law):
+    print(f"case: {items} items waves_per_cu={waves} law={law}", flush=True)
+    g = np.random.default_rng(items)
+    nleaf = 5000
+    pos = g.random((3 * nleaf, 3)) * 2.0
+    gpu_ctx.set_tuning(waves_per_cu=waves)
+    gpu_ctx.set_law(pp.ForceLaw(eps=0.05, rs=1.0, law=law))
+    gpu_ctx.set_particles(pos, (3 * np.arange(nleaf)).astype(np.int32), np.full(nleaf, 3, np.int32))
+    t = g.permutation(nleaf)[:items].astype(np.int32)
+    gpu_ctx.set_tasks(t, g.integers(0, nleaf, items).astype(np.int32))
+    out = []
+    for form in (pp.EXEC_QUEUE, pp.EXEC_QUEUE, pp.EXEC_GRID):
+        gpu_ctx.zero_acc()
+        gpu_ctx.compute(form)
+        out.append(gpu_ctx.acc())
+    assert gpu_ctx.list_stats()["nitems"] == items
+    # the same items, each by one wave: equal to the bit
+    assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[2])
