@@ -287,23 +287,38 @@ __global__ void k_zero_u64(unsigned long long *p)
 // i-particles per lane (more independent pairs per step: 1% on the 256^3
 // clustered list).  48 -> L 16 (G 4) x IPL 3, 40 -> L 20 (G 3) x IPL 2,
 // 64 -> L 32 (G 2) x IPL 2, 1 -> L 1 (G 64) x 1.
-__device__ __forceinline__ void item_shape(int c, int ipl_max, int &lanes, int &ipl)
+// One table for all sizes and limits: the search divides in a loop of up to 63
+// steps, and took most of the item kernels' time.
+struct ItemShapes {
+    unsigned char lanes[kIplMax + 1][kWave * kIplMax + 1], ipl[kIplMax + 1][kWave * kIplMax + 1];
+};
+
+constexpr ItemShapes item_shapes()
 {
-    lanes = kWave;
-    ipl = (c + kWave - 1) / kWave;
-    float best = (float)ipl;
-    for (int l = kWave - 1; l >= 1; --l) {
-        const int p = (c + l - 1) / l;
-        if (p > ipl_max)
-            break;                                   // fewer lanes only need more slots
-        const float t = (float)p / (float)(kWave / l);
-        if (t < best * 0.999f || (t < best * 1.001f && p > ipl)) {
-            best = t;
-            lanes = l;
-            ipl = p;
+    ItemShapes s{};
+    for (int ipl_max = 1; ipl_max <= kIplMax; ++ipl_max) {
+        for (int c = 1; c <= kWave * ipl_max; ++c) {
+            int lanes = kWave, ipl = (c + kWave - 1) / kWave;
+            float best = (float)ipl;
+            for (int l = kWave - 1; l >= 1; --l) {
+                const int p = (c + l - 1) / l;
+                if (p > ipl_max)
+                    break;                           // fewer lanes only need more slots
+                const float t = (float)p / (float)(kWave / l);
+                if (t < best * 0.999f || (t < best * 1.001f && p > ipl)) {
+                    best = t;
+                    lanes = l;
+                    ipl = p;
+                }
+            }
+            s.lanes[ipl_max][c] = (unsigned char)lanes;
+            s.ipl[ipl_max][c] = (unsigned char)ipl;
         }
     }
+    return s;
 }
+
+__device__ constexpr ItemShapes kItemShapes = item_shapes();
 
 // i-chunks of a target with ni particles: k = ceil(ni / 256) near-equal chunks
 // (chunk_model > 0 asks for chunks of at most that many particles instead)
@@ -328,74 +343,71 @@ __device__ __forceinline__ void chunk_of(int ni, int k, int q, int &beg, int &si
 // long source list from becoming one long item (it would run last in the
 // cost order and hold the launch open).  Every (range, chunk) pair is one
 // item; its cost is the modelled work (IPL * 64 / G + kStagePairs) * sum n_s.
+// kCutLanes lanes per row, which search its cuts together.  One thread per
+// row, halving, took 29 us to emit and 14 to count at 1300 rows (20 000
+// particles), 11 and 9 now: bound by the trips to memory, two per cut.
 template <bool EMIT>
 __device__ int row_ranges(const RowView &v, int r, long long split, int tgt, int ibeg, int ni,
                           Item *items, unsigned *cost, int out0)
 {
     if (ni == 0)
         return 0;
+    const int lane = threadIdx.x & (kCutLanes - 1), group = threadIdx.x & (kWave - kCutLanes);
     const int k = n_chunks(ni, v.stage_ops, v.ipl_max);
     const long long wi = (ni + k - 1) / k;
     const int k0 = v.row_off[r], k1 = v.row_off[r + 1];
     int nr = 0, out = out0;
+    const PrefixArray P{v.nsx};
     int beg = k0;
-    // the row's chunks have two sizes at most (ni / k and one more): their
-    // shapes once per row, not once per item (the shape search divides in a
-    // loop of up to 63 steps)
-    int lanes_lo = 0, ipl_lo = 0, lanes_hi = 0, ipl_hi = 0;
-    if (EMIT) {
-        const int base = ni / k;
-        if (base > 0)
-            item_shape(base, v.ipl_max, lanes_lo, ipl_lo);
-        if (ni % k)
-            item_shape(base + 1, v.ipl_max, lanes_hi, ipl_hi);
-    }
-    auto emit = [&](int s_beg, int s_end, long long ns) {
-        for (int q = 0; q < k; ++q) {
-            int cb, cs;
-            chunk_of(ni, k, q, cb, cs);
-            const bool hi = cs > ni / k;
-            const int lanes = hi ? lanes_hi : lanes_lo, ipl = hi ? ipl_hi : ipl_lo;
-            items[out] = Item{tgt, ibeg + cb, cs, r, s_beg, s_end, lanes, ipl};
-            if (cost)
-                cost[out] = (unsigned)min(ns * ((long long)(kWave * ipl / (kWave / lanes)) + kStagePairs),
-                                          0xffffffffll);
-            ++out;
-        }
-    };
-    // the cut after `beg`: a binary search on the prefix of the source sizes
-    const unsigned *P = v.nsx;
+    unsigned pb = P(beg);
     for (;;) {
-        const int cut = split > 0 ? range_cut(PrefixArray{P}, beg, k1, wi + kStagePairs, split) : k1;
+        int cut = k1;
+        if (split > 0)
+            cut = cut_search(beg, k1, [&](long long lo, long long step, int n) {
+                const bool over = lane < n && cut_over(P, pb, lo + (lane + 1) * step - 1, wi + kStagePairs, split);
+                const unsigned m = (unsigned)(__ballot(over) >> group) & ((1u << kCutLanes) - 1u);
+                return m ? __builtin_ctz(m) : n;
+            });
         ++nr;
-        if (cut >= k1) {
-            if (EMIT)
-                emit(beg, k1, (long long)(P[k1] - P[beg]));
-            break;
+        const unsigned pc = P(cut);
+        if (EMIT) {
+            const long long ns = (long long)(pc - pb);
+            for (int q = lane; q < k; q += kCutLanes) {
+                int cb, cs;
+                chunk_of(ni, k, q, cb, cs);
+                const int lanes = kItemShapes.lanes[v.ipl_max][cs], ipl = kItemShapes.ipl[v.ipl_max][cs];
+                items[out + q] = Item{tgt, ibeg + cb, cs, r, beg, cut, lanes, ipl};
+                if (cost)
+                    cost[out + q] = (unsigned)min(ns * ((long long)(kWave * ipl / (kWave / lanes)) + kStagePairs),
+                                                  0xffffffffll);
+            }
+            out += k;
         }
-        if (EMIT)
-            emit(beg, cut, (long long)(P[cut] - P[beg]));
+        if (cut >= k1)
+            return nr * k;
         beg = cut;
+        pb = pc;
     }
-    return nr * k;
 }
 
 __global__ void k_items_count(RowView v, int nrows, long long split, int *__restrict__ count)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / kCutLanes);
     if (r >= nrows)
         return;
     int ibeg, ni;
     const int tgt = v.row_tgt[r];
     row_i(v, tgt, ibeg, ni);
-    count[r] = row_ranges<false>(v, r, split, tgt, ibeg, ni, nullptr, nullptr, 0);
+    const int n = row_ranges<false>(v, r, split, tgt, ibeg, ni, nullptr, nullptr, 0);
+    if ((threadIdx.x & (kCutLanes - 1)) == 0)
+        count[r] = n;
 }
 
 // off: exclusive scan of the counts (nrows + 1 entries)
 __global__ void k_items_emit(RowView v, int nrows, long long split, const int *__restrict__ off,
                              Item *__restrict__ items, unsigned *__restrict__ cost)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / kCutLanes);
     if (r >= nrows)
         return;
     int ibeg, ni;
@@ -690,7 +702,8 @@ hipError_t items_count(const RowArgs &ra, long long split, int *count, int *off,
         return rocprim::exclusive_scan(nullptr, *temp_bytes, count, off, 0, (size_t)ra.nrows + 1,
                                        rocprim::plus<int>(), st);
     RowView v{ra.row_tgt, ra.row_off, ra.src, ra.rng, ra.nsx, ra.act_cnt, ra.act_off, ra.stage_ops, ra.ipl_max};
-    hipLaunchKernelGGL(k_items_count, dim3(grid_of(ra.nrows)), dim3(256), 0, st, v, ra.nrows, split, count);
+    hipLaunchKernelGGL(k_items_count, dim3(grid_of((long long)ra.nrows * kCutLanes)), dim3(256), 0, st, v, ra.nrows,
+                       split, count);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
@@ -701,7 +714,8 @@ hipError_t items_count(const RowArgs &ra, long long split, int *count, int *off,
 hipError_t items_emit(const RowArgs &ra, long long split, const int *off, Item *items, unsigned *cost, hipStream_t st)
 {
     RowView v{ra.row_tgt, ra.row_off, ra.src, ra.rng, ra.nsx, ra.act_cnt, ra.act_off, ra.stage_ops, ra.ipl_max};
-    hipLaunchKernelGGL(k_items_emit, dim3(grid_of(ra.nrows)), dim3(256), 0, st, v, ra.nrows, split, off, items, cost);
+    hipLaunchKernelGGL(k_items_emit, dim3(grid_of((long long)ra.nrows * kCutLanes)), dim3(256), 0, st, v, ra.nrows,
+                       split, off, items, cost);
     return hipGetLastError();
 }
 

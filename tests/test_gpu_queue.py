@@ -83,3 +83,32 @@ def test_small_lists(gpu_ctx, items, waves, law):
     assert gpu_ctx.list_stats()["nitems"] == items
     # the same items, each by one wave: equal to the bit
     assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[2])
+
+
+# rows about the 16 lanes that search a cut together (one probe each, a second
+# round, a partial last round): as many items as a scan of each row cuts
+@pytest.mark.parametrize("sources", [1, 2, 15, 16, 17, 18, 255, 256, 257, 273, 290, 4097])
+@pytest.mark.parametrize("split", [1, 700, 9000, 300000])
+def test_cuts_of_a_row(gpu_ctx, sources, split):
+    print(f"case: {sources} sources split={split}", flush=True)
+    g = np.random.default_rng(sources)
+    num = g.integers(1, 9, 300).astype(np.int32)
+    num[7], num[8] = 5, 200                                  # the targets: one chunk, and two
+    ip = (np.cumsum(num) - num).astype(np.int32)
+    gpu_ctx.set_tuning(split_pairs=split)
+    gpu_ctx.set_law(pp.ForceLaw(eps=0.05, rs=1.0))
+    gpu_ctx.set_particles(g.random((int(num.sum()), 3)), ip, num)
+    s = np.stack([g.integers(0, 300, sources) for _ in range(2)]).astype(np.int32)
+    gpu_ctx.set_tasks(np.repeat(np.array([7, 8], np.int32), sources), s.reshape(-1))
+    expect = 0
+    for ni, src in ((5, s[0]), (200, s[1])):
+        chunks = (ni + 191) // 192
+        wi = (ni + chunks - 1) // chunks + 24                # the staging counts as 24 pairs
+        run, ranges = 0, 1
+        for n in num[src]:
+            if run and (run + int(n)) * wi > split:
+                ranges, run = ranges + 1, 0
+            run += int(n)
+        expect += ranges * chunks
+    assert gpu_ctx.list_stats()["nitems"] == expect
+    gpu_ctx.set_tuning()
