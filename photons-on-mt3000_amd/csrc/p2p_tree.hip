@@ -234,8 +234,8 @@ __device__ __forceinline__ GroupUnits group_units(double v, double start, int la
     } else {
         all.out = __popcll(__ballot(run.out)) & 1;
     }
-    g.up = wave_sum(g.up);
-    g.down = wave_sum(g.down);
+    g.up = __ballot(g.up != 0.0) ? wave_sum(g.up) : 0.0;
+    g.down = __ballot(g.down != 0.0) ? wave_sum(g.down) : 0.0;
     g.info |= all.any | all.first << 1 | all.out << 2 | all.rest << 3;
     return g;
 }
@@ -279,6 +279,20 @@ __device__ __forceinline__ double add_groups(double s, const GroupUnits &u, int 
     return s;
 }
 
+// Plain sums: they only say where a group is expected to start.
+__device__ __forceinline__ float wave_sum_about(float v)
+{
+    auto step = [&](int moved) { v += __int_as_float(moved); };
+    const auto bits = [&] { return __float_as_int(v); };
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x111, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x112, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x114, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x118, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x142, 0xa, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, bits(), 0x143, 0xc, 0xf, true));
+    return __int_as_float(__builtin_amdgcn_readlane(bits(), 63));
+}
+
 // ------------------------------------------------------------- level passes
 
 // the segment holding a tile: the last s with toff[s] <= tile
@@ -303,7 +317,7 @@ __device__ __forceinline__ int seg_of_tile(const int *__restrict__ toff, int nse
 // change the binade, 2 us each with the load of their samples.  One workgroup
 // per segment doing all of it, one 4096 values after the other, was bound by
 // the loads and the rounding of a single CU where the segments are few: 9 levels of
-// 64^3 took 625 us and take 390, 16 of 256^3 (clustered) 2500 and take 1950.
+// 64^3 took 625 us and take 345, 16 of 256^3 (clustered) 2500 and take 1850.
 struct Samples {
     const int *x;                                    // the segment's coordinates
     long long mul;
@@ -357,13 +371,15 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_sums(TreeLevelView lv, cons
 }
 
 // the groups of each chunk in units
-__global__ __launch_bounds__(kTreeBlock) void k_tree_units(TreeLevelView lv, const int *__restrict__ nseg,
+constexpr int kUnitBlock = 1024;
+
+__global__ __launch_bounds__(kUnitBlock) void k_tree_units(TreeLevelView lv, const int *__restrict__ nseg,
                                                          const int *__restrict__ x, double int2pos,
                                                          const double *__restrict__ csum,
                                                          const int *__restrict__ tmap,
                                                          GroupUnits *__restrict__ units)
 {
-    constexpr int kGroups = kTreeTile / kGroup, kPerWave = kGroups / (kTreeBlock / 64);
+    constexpr int kGroups = kTreeTile / kGroup, kPerWave = kGroups / (kUnitBlock / 64);
     __shared__ double start[kGroups];
     const int n = *nseg, tile = blockIdx.x;
     if (n == 0 || tile >= lv.toff[n])
@@ -380,9 +396,9 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_units(TreeLevelView lv, con
         mine[u] = v(c * kTreeTile + (wave * kPerWave + u) * kGroup + lane);
 #pragma unroll
     for (int u = 0; u < kPerWave; ++u) {
-        const double g = wave_sum(mine[u]);
+        const float g = wave_sum_about((float)mine[u]);
         if (lane == 0)
-            start[wave * kPerWave + u] = g;
+            start[wave * kPerWave + u] = (double)g;
     }
     __syncthreads();
     if (wave == 0) {
@@ -1227,7 +1243,7 @@ hipError_t tree_level(const TreeScratch &w, const TreeLevelView &lv, const TreeL
     const unsigned nt = (unsigned)tiles;
     GroupUnits *u = reinterpret_cast<GroupUnits *>(units);
     k_tree_sums<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap);
-    k_tree_units<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap, u);
+    k_tree_units<<<nt, kUnitBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap, u);
     k_tree_mean<<<(unsigned)cap, 64, 0, st>>>(lv, ns, x, int2pos, u);
     k_tree_flags<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, mask, tcnt, tmap);
     k_tree_lists<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, mask, tcnt, tmap, w.la, w.lb);
