@@ -77,9 +77,14 @@ hipError_t rows_cost(const RowArgs &ra, unsigned long long *cost, unsigned long 
                      void *temp, size_t *temp_bytes, hipStream_t st);
 hipError_t items_count(const RowArgs &ra, long long split, int *count, int *off,
                        void *temp, size_t *temp_bytes, hipStream_t st);
-hipError_t items_emit(const RowArgs &ra, long long split, const int *off, Item *items, unsigned *cost,
+// The items in row order with their costs; buckets (2 kCostBuckets) is cleared
+// for items_sort.
+constexpr int kCostBuckets = 1024;
+hipError_t items_emit(const RowArgs &ra, long long split, const int *off, Item *items, unsigned *cost, int *buckets,
                       hipStream_t st);
-hipError_t items_sort(const unsigned *cost, unsigned *cost_sorted, int *idx, int *idx_sorted, const Item *items,
-                      Item *items_sorted, int n, void *temp, size_t *temp_bytes, hipStream_t st);
+// items_sorted = the items by falling cost: classes of costs within 1/32 of each
+// other, any order inside a class.
+hipError_t items_sort(const unsigned *cost, int *buckets, const Item *items, Item *items_sorted, int n,
+                      hipStream_t st);
 
 }  // namespace pp2p

@@ -168,8 +168,8 @@ struct pp2p_ctx {
     DevBuf<unsigned> nsx;               // prefix of the source sizes over the CSR
     DevBuf<int> item_count, item_off;
     DevBuf<Item> items_rows, items_q;     // row order / cost-sorted
-    DevBuf<unsigned> cost, cost_sorted;
-    DevBuf<int> idx, idx_sorted;
+    DevBuf<unsigned> cost;
+    DevBuf<int> buckets;
     int nitems = 0;
     long long split = 0;
     bool items_ready = false;
@@ -385,7 +385,7 @@ void pp2p_destroy(pp2p_ctx *c)
     c->ilist.release(); c->task_t.release(); c->task_s.release(); c->key_sorted.release(); c->src.release();
     c->flag.release(); c->rowidx.release(); c->row_tgt.release(); c->row_off.release(); c->row_cost.release();
     c->total.release(); c->item_count.release(); c->item_off.release(); c->items_rows.release();
-    c->items_q.release(); c->cost.release(); c->cost_sorted.release();
+    c->items_q.release(); c->cost.release(); c->buckets.release();
     c->wson.release(); c->wnc.release(); c->wnw.release(); c->wlc.release(); c->wlw.release(); c->wact.release();
     c->wcell.release(); c->wround.release(); c->wf.release(); c->wcode.release(); c->woff.release();
     c->wcnt.release(); c->wsep.release(); c->wlook.release(); c->wm2l_t.release(); c->wm2l_s.release();
@@ -406,7 +406,7 @@ void pp2p_destroy(pp2p_ctx *c)
     if (c->pm_fwd) (void)hipfftDestroy(c->pm_fwd);
     if (c->pm_inv) (void)hipfftDestroy(c->pm_inv);
     c->nsx.release();
-    c->idx.release(); c->idx_sorted.release(); c->counter.release(); c->temp.release();
+    c->counter.release(); c->temp.release();
     c->pair_count.release();
     c->acc32.release();
     c->pipe.release();
@@ -1493,7 +1493,9 @@ static ListView ctx_view(pp2p_ctx *c)
 }
 
 // Target CSR of the list (task_t, task_s): stable sort by target, then the
-// rows (src/gpu_entry.cu:132-138).  One host synchronisation (the row count).
+// rows (src/gpu_entry.cu:132-138), and the prefix of the source sizes, which
+// stays while the list and the leaves do (another active set does not change
+// it).  One host synchronisation (the row count).
 static int csr_build(pp2p_ctx *c, Space &sp, const int *tt, const int *ts, int n, ListView &L)
 {
     int *flag = nullptr, *rowidx = nullptr;
@@ -1506,18 +1508,22 @@ static int csr_build(pp2p_ctx *c, Space &sp, const int *tt, const int *ts, int n
     L.nrows = 0;
     if (n == 0)
         return PP2P_OK;
+    if ((st = sp.get(c->nsx, (size_t)n + 1, &L.nsx)))
+        return st;
     int bits = 1;
     while ((1ll << bits) < (long long)c->nleaf)
         ++bits;
-    size_t tb1 = 0, tb2 = 0;
+    size_t tb0 = 0, tb1 = 0, tb2 = 0;
+    HIPCHK(src_prefix(L.src, c->rng.p, n, L.nsx, nullptr, &tb0, c->stream));
     HIPCHK(csr_sort(tt, ts, L.key_sorted, L.src, n, bits, nullptr, &tb1, c->stream));
     HIPCHK(csr_rows(L.key_sorted, n, flag, rowidx, L.row_tgt, L.row_off, nullptr, &tb2, c->stream));
     void *tmp = nullptr;
-    if ((st = sp.temp(std::max(tb1, tb2), &tmp, &tb1)))
+    if ((st = sp.temp(std::max(tb0, std::max(tb1, tb2)), &tmp, &tb1)))
         return st;
-    tb2 = tb1;
+    tb0 = tb2 = tb1;
     HIPCHK(csr_sort(tt, ts, L.key_sorted, L.src, n, bits, tmp, &tb1, c->stream));
     HIPCHK(csr_rows(L.key_sorted, n, flag, rowidx, L.row_tgt, L.row_off, tmp, &tb2, c->stream));
+    HIPCHK(src_prefix(L.src, c->rng.p, n, L.nsx, tmp, &tb0, c->stream));
     int rows = 0;
     if ((st = fetch(c, &rows, rowidx + n - 1, sizeof(int))))
         return st;
@@ -1603,19 +1609,15 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L)
     L.pairs = 0;
     if (nr == 0)
         return PP2P_OK;
-    if ((st = sp.get(c->nsx, (size_t)L.ntask + 1, &L.nsx)))
-        return st;
     RowArgs ra = row_args(c, L);
-    size_t tb0 = 0, tb1 = 0, tb2 = 0;
-    HIPCHK(src_prefix(L.src, c->rng.p, L.ntask, L.nsx, nullptr, &tb0, c->stream));
+    size_t tb1 = 0, tb2 = 0;
     HIPCHK(rows_cost(ra, row_cost, total, nullptr, &tb1, c->stream));
     HIPCHK(items_count(ra, 0, item_count, item_off, nullptr, &tb2, c->stream));
     void *tmp = nullptr;
     size_t tlen = 0;
-    if ((st = sp.temp(std::max(tb0, std::max(tb1, tb2)), &tmp, &tlen)))
+    if ((st = sp.temp(std::max(tb1, tb2), &tmp, &tlen)))
         return st;
-    tb0 = tb1 = tb2 = tlen;
-    HIPCHK(src_prefix(L.src, c->rng.p, L.ntask, L.nsx, tmp, &tb0, c->stream));
+    tb1 = tb2 = tlen;
     HIPCHK(rows_cost(ra, row_cost, total, tmp, &tb1, c->stream));
     unsigned long long tot[2] = {0, 0};              // pairs, staged source particles
     if ((st = fetch(c, tot, total, sizeof(tot))))
@@ -1648,19 +1650,13 @@ static int items_build(pp2p_ctx *c, Space &sp, ListView &L)
         return st;
     if (nitems == 0)                                 // no target holds an active particle
         return PP2P_OK;
-    unsigned *cost = nullptr, *cost_sorted = nullptr;
-    int *idx = nullptr, *idx_sorted = nullptr;
+    unsigned *cost = nullptr;
+    int *buckets = nullptr;
     if ((st = sp.get(c->items_rows, nitems, &L.items_rows)) || (st = sp.get(c->items_q, nitems, &L.items_q)) ||
-        (st = sp.get(c->cost, nitems, &cost)) || (st = sp.get(c->cost_sorted, nitems, &cost_sorted)) ||
-        (st = sp.get(c->idx, nitems, &idx)) || (st = sp.get(c->idx_sorted, nitems, &idx_sorted)))
+        (st = sp.get(c->cost, nitems, &cost)) || (st = sp.get(c->buckets, 2 * kCostBuckets, &buckets)))
         return st;
-    HIPCHK(items_emit(ra, split, item_off, L.items_rows, cost, c->stream));
-    size_t tb3 = 0;
-    HIPCHK(items_sort(cost, cost_sorted, idx, idx_sorted, L.items_rows, L.items_q, nitems, nullptr, &tb3,
-                      c->stream));
-    if ((st = sp.temp(tb3, &tmp, &tb3)))
-        return st;
-    HIPCHK(items_sort(cost, cost_sorted, idx, idx_sorted, L.items_rows, L.items_q, nitems, tmp, &tb3, c->stream));
+    HIPCHK(items_emit(ra, split, item_off, L.items_rows, cost, buckets, c->stream));
+    HIPCHK(items_sort(cost, buckets, L.items_rows, L.items_q, nitems, c->stream));
     L.nitems = nitems;
     L.split = split;
     return PP2P_OK;

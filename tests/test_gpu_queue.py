@@ -112,3 +112,26 @@ def test_cuts_of_a_row(gpu_ctx, sources, split):
         expect += ranges * chunks
     assert gpu_ctx.list_stats()["nitems"] == expect
     gpu_ctx.set_tuning()
+
+
+# item counts about a workgroup of the cost sort (1024 items) with costs over many
+# classes: every item once in the sorted copy, so that both copies give the same
+# sums (one item per target: equal to the bit)
+@pytest.mark.parametrize("items", [1, 1023, 1024, 1025, 2049, 9000])
+def test_sorted_items(gpu_ctx, items):
+    print(f"case: {items} items", flush=True)
+    g = np.random.default_rng(items)
+    num = (10 ** (2.2 * g.random(9000))).astype(np.int32)    # 1 to 158 particles
+    gpu_ctx.set_tuning(split_pairs=1 << 30)
+    gpu_ctx.set_law(pp.ForceLaw(eps=0.05, rs=1.0))
+    gpu_ctx.set_particles(g.random((int(num.sum()), 3)), (np.cumsum(num) - num).astype(np.int32), num)
+    t = g.permutation(9000)[:items].astype(np.int32)
+    gpu_ctx.set_tasks(np.repeat(t, 3), g.integers(0, 9000, 3 * items).astype(np.int32))
+    out = []
+    for form in (pp.EXEC_QUEUE, pp.EXEC_GRID):
+        gpu_ctx.zero_acc()
+        gpu_ctx.compute(form)
+        out.append(gpu_ctx.acc())
+    assert gpu_ctx.list_stats()["nitems"] == items
+    assert np.array_equal(out[0], out[1])
+    gpu_ctx.set_tuning()
