@@ -152,6 +152,25 @@ __device__ __forceinline__ int lanes_parity(const SeqTies &run, int p, int lane,
     return before;
 }
 
+// s + the first cnt of a wave's 64 values, one after the other, the same in every
+// lane: 16 to 20 cycles a value, so 64 values cost less than the passes of add_run
+// that a group which leaves its binade needs (about 2 us).
+__device__ __forceinline__ double add_chain(double s, double v, int cnt)
+{
+    constexpr int kStep = 16;
+    if (cnt >= 64) {
+#pragma unroll
+        for (int k = 0; k < 64; ++k)
+            s += lane_value(v, k);
+        return s;
+    }
+    for (int k = 0; k < cnt; k += kStep)             // (+0.0 past the end)
+#pragma unroll
+        for (int u = 0; u < kStep; ++u)
+            s += lane_value(v, k + u);
+    return s;
+}
+
 // s + a wave's 64 kV values, lane l's before lane l + 1's, the same in every
 // lane.  A pass adds the lanes up to the first whose values may leave the sum's
 // binade by one prefix sum, then that lane's one after the other.  A sum from zero
@@ -270,10 +289,8 @@ __device__ __forceinline__ double add_groups(double s, const GroupUnits &u, int 
             const double m = (S + lane_value(t, first - 1)) * seq_unit(scale);
             s = s < 0.0 ? -m : m;
         }
-        if (first < cnt) {
-            const double one[1] = {value(base + first)};
-            s = add_run(s, one, lane);
-        }
+        if (first < cnt)
+            s = add_chain(s, value(base + first), 64);
         next = first + 1;
     }
     return s;
@@ -314,10 +331,11 @@ __device__ __forceinline__ int seg_of_tile(const int *__restrict__ toff, int nse
 // particles, or every (len / 10^5)-th) in chunks of 4096: sums of the chunks, the
 // groups of each chunk in units, and one wave per segment that composes them.
 // The first two are bound by HBM, the last by the chain of about ten groups that
-// change the binade, 2 us each with the load of their samples.  One workgroup
+// change the binade, 1 us each with the load of their samples (2 with add_run in
+// place of a plain chain: 9 levels of 64^3 280 -> 199 us, 18 of 256^3 890 -> 720).  One workgroup
 // per segment doing all of it, one 4096 values after the other, was bound by
 // the loads and the rounding of a single CU where the segments are few: 9 levels of
-// 64^3 took 625 us and take 345, 16 of 256^3 (clustered) 2500 and take 1850.
+// 64^3 took 625 us and take 315, 18 of 256^3 (clustered) 2500 and take 1700.
 struct Samples {
     const int *x;                                    // the segment's coordinates
     long long mul;
@@ -708,16 +726,26 @@ __global__ __launch_bounds__(kNextBlock) void k_tree_next(TreeLevelView lv, Tree
 
 // A whole subtree of at most kSubMax particles by one workgroup, the particles
 // in LDS from the first split to the last.  Per level: the means (one thread
-// per segment when there are many, one wave per segment with the parallel sums
-// otherwise), the masks, the partners, the swaps, the sons.  The nodes are
+// per segment from eight on, one wave per segment otherwise), the masks, the partners, the swaps, the sons.  The nodes are
 // numbered breadth first while they are made and depth first at the end.
 // Bound by the latencies of about eight levels (the means first, then seven
 // barriers each); it takes the place of as many passes over all particles in
-// HBM: 3.0 ms for 1.9 10^7 particles (256^3 clustered) where ten levels of
-// device-wide passes took about 8.  4096 particles with the records fill one
+// HBM: 2.6 ms for 1.9 10^7 particles (256^3 clustered; 3.0 with add_run for all
+// levels of fewer than 48 segments) where ten levels of device-wide passes took
+// about 8.  4096 particles with the records fill one
 // CU's LDS.  The whole build, uploads included, went from 28.2 to 15.7 ms
 // there, from 4.6 to 1.5 ms at 64^3 and from 1.5 to 0.58 ms at 16^3.
 constexpr int kSubBlock = 1024;
+constexpr int kBatch = 8;            // values of a thread's chain loaded together
+// How a level's segments are summed.  The parallel form (add_run) costs about
+// 2 us for each change of the binade and, with several waves on a SIMD, the
+// instructions of each; a plain chain costs its length.  Level by level of a subtree
+// of 3200 particles (segments of 3200, 1600, ...): add_run 15 to 25, 10 to 20, 7 to
+// 15, 13, 25 and 11 us; one wave's chain (segments of at most kSubChain) 9 us for
+// 800 values, 7 for 400; one thread per segment, 14 ns a value, 11 for 800, then
+// 6, 3.3 and 2.  With eight segments or more a level is as long as a thread's chain.
+constexpr int kSubChain = 1024;
+constexpr int kSubThreads = 8;
 
 struct SubLds {
     int x[3][kSubMax], idx[kSubMax];
@@ -780,21 +808,34 @@ __global__ __launch_bounds__(kSubBlock) void k_tree_sub(TreeScratch w, TreeSub *
         const int *x = m.x[axis];
         const unsigned short *beg = m.beg[cur], *slen = m.len[cur];
         // means and split values
-        if (nseg >= 48) {
+        if (nseg >= kSubThreads) {
             for (int s = tid; s < nseg; s += kSubBlock) {
                 const int b = beg[s], l = slen[s];
                 double sum = 0.0;
                 float sp = 0.0f;
                 if (l > 2) {
                     int j = 0;
-                    for (; j + 8 <= l; j += 8) {
-                        int r[8];
+                    if (l >= kBatch) {               // the next batch is read ahead of this one's chain
+                        int r[kBatch];
 #pragma unroll
-                        for (int q = 0; q < 8; ++q)
-                            r[q] = x[b + j + q];
+                        for (int q = 0; q < kBatch; ++q)
+                            r[q] = x[b + q];
+                        for (; j + 2 * kBatch <= l; j += kBatch) {
+                            int ahead[kBatch];
 #pragma unroll
-                        for (int q = 0; q < 8; ++q)
+                            for (int q = 0; q < kBatch; ++q)
+                                ahead[q] = x[b + j + kBatch + q];
+#pragma unroll
+                            for (int q = 0; q < kBatch; ++q)
+                                sum += int2pos * (double)r[q];
+#pragma unroll
+                            for (int q = 0; q < kBatch; ++q)
+                                r[q] = ahead[q];
+                        }
+#pragma unroll
+                        for (int q = 0; q < kBatch; ++q)
                             sum += int2pos * (double)r[q];
+                        j += kBatch;
                     }
                     for (; j < l; ++j)
                         sum += int2pos * (double)x[b + j];
@@ -811,7 +852,17 @@ __global__ __launch_bounds__(kSubBlock) void k_tree_sub(TreeScratch w, TreeSub *
                 const int b = beg[s], l = slen[s];
                 double sum = 0.0;
                 float sp = 0.0f;
-                if (l > 2) {
+                if (l > 2 && l <= kSubChain) {
+                    auto value = [&](int j) { return j < l ? int2pos * (double)x[b + j] : 0.0; };
+                    double v = value(lane);
+                    for (int c = 0; c < l; c += 64) {
+                        const double ahead = value(c + 64 + lane);
+                        sum = add_chain(sum, v, min(l - c, 64));
+                        v = ahead;
+                    }
+                    sum /= (double)l;
+                    sp = (float)sum;
+                } else if (l > 2) {
                     for (int c = 0; c < l; c += 512) {
                         double v[8];
 #pragma unroll

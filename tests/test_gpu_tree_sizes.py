@@ -128,3 +128,15 @@ def test_means_over_tiles(gpu_ctx, n, offset):
     posi = g.integers(-(1 << 27), 1 << 27, (n, 3)) + offset
     for k, step in enumerate(STEPS):
         _same(gpu_ctx, posi, step, 1000, n + k)
+
+
+# one subtree whose segments end at, before and after a batch of the threads' chains
+# (8), a wave's 64 values and the longest chain of a wave (1024)
+@pytest.mark.parametrize("n", [3, 15, 16, 17, 63, 64, 65, 127, 200, 1023, 1024, 1025, 2051])
+@pytest.mark.parametrize("offset", [0, 1 << 29])
+def test_segment_chains(gpu_ctx, n, offset):
+    print(f"case: n={n} offset={offset}", flush=True)
+    g = np.random.default_rng(n)
+    posi = g.integers(-(1 << 27), 1 << 27, (n, 3)) + offset
+    for k, step in enumerate(STEPS):
+        _same(gpu_ctx, posi, step, 1, n + k)
