@@ -140,7 +140,9 @@ int pp2p_set_active(pp2p_ctx *ctx, const unsigned char *act, int active_level);
 /*
  * Interaction list: ntask (target, source) leaf pairs.  pp2p_set_tasks
  * replaces the list of the context; pp2p_add_tasks appends (flushes of a
- * streamed list, LEN_TASK in src/fmm.c:500-515).  The list is not modified.
+ * streamed list, LEN_TASK in src/fmm.c:500-515).  The arrays are not modified.
+ * A refused pp2p_add_tasks leaves the list as it was, a refused
+ * pp2p_set_tasks an empty one.
  */
 int pp2p_set_tasks(pp2p_ctx *ctx, long long ntask, const int *task_t, const int *task_s);
 int pp2p_add_tasks(pp2p_ctx *ctx, long long ntask, const int *task_t, const int *task_s);

@@ -676,8 +676,8 @@ static int append_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
         c->task_s = ns;
     }
     if (n) {
-        // the leaf ids are checked while they are copied; a bad list leaves the
-        // context's as it is
+        // the leaf ids are checked while they are copied; with a bad one nothing
+        // is appended
         const unsigned nl = (unsigned)c->nleaf;
         std::atomic<bool> good{true};
         auto upload = [&](int *dst, const int *v) {
@@ -714,7 +714,10 @@ int pp2p_set_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
         return st;
     if (!c->have_particles)
         return fail(PP2P_ERR_STATE, "set_particles before set_tasks");
+    // the old list is gone whether or not the new one is accepted, and so are
+    // its CSR and items: a refused list leaves an empty one
     c->ntask = 0;
+    c->csr_ready = c->items_ready = false;
     return append_tasks(c, n, tt, ts);
 }
 
