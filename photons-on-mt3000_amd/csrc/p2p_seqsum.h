@@ -53,10 +53,10 @@ __host__ __device__ inline double seq_unit(double scale)
 // fails the binade test below).
 __host__ __device__ inline double seq_units(double v, double scale, bool &half)
 {
-    const double q = v * scale;
-    const double f = __builtin_floor(q);
-    half = q - f == 0.5;
-    return half ? f : __builtin_rint(q);
+    // q - r is exact (q - floor(q) is not: it rounds to 0.5 for q just above -0.5)
+    const double q = v * scale, r = __builtin_rint(q);
+    half = __builtin_fabs(q - r) == 0.5;
+    return half ? __builtin_floor(q) : r;
 }
 
 __host__ __device__ inline bool seq_odd(double r)
