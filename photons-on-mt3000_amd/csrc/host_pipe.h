@@ -1,6 +1,7 @@
 // Copies between pageable host memory and the device through a small ring of
 // pinned slots: the DMA engine moves one piece while a few host threads fill or
-// empty the others (internal to the library).
+// empty the others (internal to the library).  Memory that the DMA engine
+// reaches by itself (pinned by the caller) is copied straight, with no thread.
 //
 // A copy straight from pageable memory runs at half the pinned rate, and one
 // into memory that the caller has just allocated at 4 GB/s, since a single
@@ -138,10 +139,18 @@ public:
     // time.
     static constexpr size_t kLeast = 4 << 20;
 
-    // bytes from src to dst; the caller may reuse src when it returns.
+    // Whether a copy from or to p goes through the ring: not a small one, and not
+    // where the runtime knows the memory (both ends asked).
+    static bool staged(const void *p, size_t bytes)
+    {
+        return bytes >= kLeast && !(known(p) && known(static_cast<const char *>(p) + bytes - 1));
+    }
+
+    // bytes from src to dst; the caller may reuse a pageable src when it returns,
+    // a pinned one when the stream has passed the copy.
     hipError_t to_device(void *dst, const void *src, size_t bytes, hipStream_t st)
     {
-        if (bytes < kLeast)
+        if (!staged(src, bytes))
             return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
         const char *s = static_cast<const char *>(src);
         return to_device_filled(dst, bytes, 1, st, [s](char *at, size_t b, size_t n) { std::memcpy(at, s + b, n); });
@@ -179,7 +188,7 @@ public:
     // bytes from src to dst; complete when it returns.
     hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t st)
     {
-        if (bytes < kLeast) {
+        if (!staged(dst, bytes)) {
             hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st) : hipSuccess;
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }
@@ -216,6 +225,26 @@ public:
         return e;
     }
 
+    // fn(b, n) over slices of [0, bytes), their starts multiples of 64, on several
+    // threads from kLeast on
+    template <class Fn>
+    void each(size_t bytes, Fn fn)
+    {
+        if (bytes < kLeast) {
+            fn((size_t)0, bytes);
+            return;
+        }
+        if (!crew_)
+            crew_.reset(new Crew());
+        const int s = slices_of(bytes);
+        const size_t part = ((bytes + s - 1) / s + 63) / 64 * 64;
+        crew_->run(s, [&](int q) {
+            const size_t b = q * part;
+            if (b < bytes)
+                fn(b, std::min(part, bytes - b));
+        });
+    }
+
     void release()
     {
         for (auto &v : ev_) {
@@ -234,6 +263,18 @@ private:
     static constexpr size_t kSlot = 2 << 20;
     static constexpr int kSlots = 4;
     static constexpr size_t kBlock = 2 << 20;
+
+    // pinned, managed or device memory; pageable memory is an error to some
+    // versions of the runtime, which must not stay behind as the last one
+    static bool known(const void *p)
+    {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return a.type != hipMemoryTypeUnregistered;
+    }
 
     // four pieces of a copy below 8 MiB, so that it overlaps itself too
     static size_t piece_of(size_t bytes)

@@ -676,26 +676,29 @@ static int append_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
         c->task_s = ns;
     }
     if (n) {
-        // the leaf ids are checked while they are copied; with a bad one nothing
-        // is appended
+        // the leaf ids are checked while they are copied (a staged list on its way
+        // into the ring, another one beside the copy); with a bad one nothing is
+        // appended
         const unsigned nl = (unsigned)c->nleaf;
+        const size_t bytes = sizeof(int) * (size_t)n;
         std::atomic<bool> good{true};
+        auto check = [&](const int *v, size_t b, size_t m) {
+            if (!all_below(v + b / sizeof(int), m / sizeof(int), nl))
+                good = false;
+        };
         auto upload = [&](int *dst, const int *v) {
-            const size_t bytes = sizeof(int) * (size_t)n;
-            if (bytes < HostPipe::kLeast) {
-                if (!all_below(v, (size_t)n, nl))
-                    good = false;
+            if (!HostPipe::staged(v, bytes))
                 return c->pipe.to_device(dst, v, bytes, c->stream);
-            }
             return c->pipe.to_device_filled(dst, bytes, sizeof(int), c->stream, [&](char *at, size_t b, size_t m) {
-                const int *p = v + b / sizeof(int);
-                std::memcpy(at, p, m);
-                if (!all_below(p, m / sizeof(int), nl))
-                    good = false;
+                std::memcpy(at, v + b / sizeof(int), m);
+                check(v, b, m);
             });
         };
         HIPCHK(upload(c->task_t.p + c->ntask, tt));
         HIPCHK(upload(c->task_s.p + c->ntask, ts));
+        for (const int *v : {tt, ts})
+            if (!HostPipe::staged(v, bytes))
+                c->pipe.each(bytes, [&](size_t b, size_t m) { check(v, b, m); });
         HIPCHK(hipStreamSynchronize(c->stream));   // the caller may reuse its buffers on return
         if (!good)
             for (long long k = 0; k < n; ++k)
