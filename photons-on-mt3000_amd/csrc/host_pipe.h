@@ -8,9 +8,10 @@
 // thread takes every page fault; here up to twelve threads share the faults,
 // ahead of the copy and a 2 MiB block each (with large pages, threads that fault
 // in one block wait for each other).
-// The threads and the ring (four slots of a quarter of the largest copy so far,
-// 8 MiB at most: its first use costs up to 0.4 ms per MiB) belong to one context;
-// both start with its first large copy and end with it.  The threads sleep
+// The threads and the ring (four slots of 2 MiB) belong to one context; both start
+// with its first large copy and end with it.  That copy pays for them: 0.15 ms for
+// the threads, about 0.3 ms for pinning the ring and 0.1 ms for each MiB of it that
+// is used.  The threads sleep
 // between copies; within one they wait for the next piece for some tens of
 // microseconds before they sleep (spinning throughout took the processor time of
 // the caller's own threads: passes of ten times the usual length now and then).
@@ -260,7 +261,7 @@ public:
     }
 
 private:
-    static constexpr size_t kSlot = 2 << 20;
+    static constexpr size_t kSlot = 2 << 20, kSmallSlot = 256 << 10;
     static constexpr int kSlots = 4;
     static constexpr size_t kBlock = 2 << 20;
 
@@ -276,7 +277,7 @@ private:
         return a.type != hipMemoryTypeUnregistered;
     }
 
-    // four pieces of a copy below 8 MiB, so that it overlaps itself too
+    // about four pieces of a copy below 8 MiB, so that it overlaps itself too
     static size_t piece_of(size_t bytes)
     {
         const size_t p = (bytes / kSlots + 4095) / 4096 * 4096;
@@ -298,9 +299,15 @@ private:
 
     char *slot(size_t k) const { return ring_ + (k % kSlots) * slot_; }
 
-    // the threads, and slots of at least `slot` bytes with no copy in flight
+    // the threads, and slots of at least `slot` bytes with no copy in flight.  A ring
+    // has small slots or full ones, nothing between: pinning it takes about 0.3 ms
+    // whatever its size, and the first touch of its pages (0.4 ms per MiB on one
+    // thread) comes with the pieces that use them; a ring that grew with the longest
+    // copy so far was pinned and touched twice when a program's lists are longer than
+    // its positions (1 ms of its first pass).
     hipError_t open(size_t slot)
     {
+        slot = slot <= kSmallSlot ? kSmallSlot : kSlot;
         if (!crew_)
             crew_.reset(new Crew());
         for (auto &v : ev_) {

@@ -38,3 +38,10 @@ def test_pageable_arrays_are_staged(lib, n):
 def test_pinned_arrays_go_straight(lib, n, shift):
     c = _copies(lib, [n, n], True, shift)
     assert c == {"copies": 4, "user": 4, "allocs": 0, "bytes": 0}
+
+
+def test_the_ring_is_allocated_once(lib):
+    """A longer copy after a first one finds the ring: pinning it again, at its new
+    size, costs as much as the first time."""
+    c = _copies(lib, [4 * MIB, 5 * MIB, 9 * MIB, 7 * MIB, 64 * MIB], False)
+    assert c["allocs"] == 1 and c["bytes"] <= 8 * MIB
