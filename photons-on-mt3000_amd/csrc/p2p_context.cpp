@@ -653,58 +653,85 @@ int pp2p_set_active(pp2p_ctx *c, const unsigned char *a, int level)
     return PP2P_OK;
 }
 
+// b with room for n elements, its first `used` (of what it holds) kept.
+extern "C++" {
+template <typename T>
+static hipError_t grow_keep(DevBuf<T> &b, size_t n, size_t used, hipStream_t st)
+{
+    if (n <= b.cap)
+        return hipSuccess;
+    DevBuf<T> nb;
+    hipError_t e = nb.reserve(n);
+    used = std::min(used, b.cap);
+    if (e == hipSuccess && used)
+        e = hipMemcpyAsync(nb.p, b.p, sizeof(T) * used, hipMemcpyDeviceToDevice, st);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+        nb.release();
+        return e;
+    }
+    b.release();
+    b = nb;
+    return hipSuccess;
+}
+}  // extern "C++"
+
 static int append_tasks(pp2p_ctx *c, long long n, const int *tt, const int *ts)
 {
     if (n < 0 || (n > 0 && (!tt || !ts)))
         return fail(PP2P_ERR_ARG, "invalid task arrays");
     if (c->ntask + n > (1ll << 31) - 1)
         return fail(PP2P_ERR_ARG, "more than 2^31-1 tasks in one list");
-    const size_t need = (size_t)(c->ntask + n);
-    if (need > c->task_t.cap) {
-        // keep the existing tasks across the grow
-        DevBuf<int> nt, ns;
-        HIPCHK(nt.reserve(need));
-        HIPCHK(ns.reserve(need));
-        if (c->ntask) {
-            HIPCHK(hipMemcpyAsync(nt.p, c->task_t.p, sizeof(int) * c->ntask, hipMemcpyDeviceToDevice, c->stream));
-            HIPCHK(hipMemcpyAsync(ns.p, c->task_s.p, sizeof(int) * c->ntask, hipMemcpyDeviceToDevice, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
-        }
-        c->task_t.release();
-        c->task_s.release();
-        c->task_t = nt;
-        c->task_s = ns;
+    if (n == 0) {
+        c->csr_ready = c->items_ready = false;
+        return PP2P_OK;
     }
-    if (n) {
-        // the leaf ids are checked while they are copied (a staged list on its way
-        // into the ring, another one beside the copy); with a bad one nothing is
-        // appended
-        const unsigned nl = (unsigned)c->nleaf;
-        const size_t bytes = sizeof(int) * (size_t)n;
-        std::atomic<bool> good{true};
-        auto check = [&](const int *v, size_t b, size_t m) {
-            if (!all_below(v + b / sizeof(int), m / sizeof(int), nl))
-                good = false;
-        };
-        auto upload = [&](int *dst, const int *v) {
-            if (!HostPipe::staged(v, bytes))
-                return c->pipe.to_device(dst, v, bytes, c->stream);
-            return c->pipe.to_device_filled(dst, bytes, sizeof(int), c->stream, [&](char *at, size_t b, size_t m) {
-                std::memcpy(at, v + b / sizeof(int), m);
-                check(v, b, m);
-            });
-        };
-        HIPCHK(upload(c->task_t.p + c->ntask, tt));
-        HIPCHK(upload(c->task_s.p + c->ntask, ts));
+    const unsigned nl = (unsigned)c->nleaf;
+    const size_t need = (size_t)(c->ntask + n), bytes = sizeof(int) * (size_t)n;
+    std::atomic<bool> good{true};
+    auto check = [&](const int *v, size_t b, size_t m) {
+        if (!all_below(v + b / sizeof(int), m / sizeof(int), nl))
+            good = false;
+    };
+    auto check_all = [&](const int *v) { c->pipe.each(bytes, [&](size_t b, size_t m) { check(v, b, m); }); };
+    auto refuse = [&] {
+        for (long long k = 0; k < n; ++k)
+            if ((unsigned)tt[k] >= nl || (unsigned)ts[k] >= nl)
+                return fail(PP2P_ERR_ARG, "task " + std::to_string(k) + " names a leaf outside [0, nleaf)");
+        return fail(PP2P_ERR_ARG, "a task names a leaf outside [0, nleaf)");
+    };
+    // The leaf ids are checked while they are copied (a staged list on its way into
+    // the ring, another one beside the copy); with a bad one nothing is appended.
+    // Where the arrays have to grow they are checked first: a refused list takes
+    // no memory.
+    const bool first = need > c->task_t.cap || need > c->task_s.cap;
+    if (first) {
+        check_all(tt);
+        check_all(ts);
+        if (!good)
+            return refuse();
+        // keep the existing tasks across the grow
+        HIPCHK(grow_keep(c->task_t, need, (size_t)c->ntask, c->stream));
+        HIPCHK(grow_keep(c->task_s, need, (size_t)c->ntask, c->stream));
+    }
+    auto upload = [&](int *dst, const int *v) {
+        if (first || !HostPipe::staged(v, bytes))
+            return c->pipe.to_device(dst, v, bytes, c->stream);
+        return c->pipe.to_device_filled(dst, bytes, sizeof(int), c->stream, [&](char *at, size_t b, size_t m) {
+            std::memcpy(at, v + b / sizeof(int), m);
+            check(v, b, m);
+        });
+    };
+    HIPCHK(upload(c->task_t.p + c->ntask, tt));
+    HIPCHK(upload(c->task_s.p + c->ntask, ts));
+    if (!first)
         for (const int *v : {tt, ts})
             if (!HostPipe::staged(v, bytes))
-                c->pipe.each(bytes, [&](size_t b, size_t m) { check(v, b, m); });
-        HIPCHK(hipStreamSynchronize(c->stream));   // the caller may reuse its buffers on return
-        if (!good)
-            for (long long k = 0; k < n; ++k)
-                if ((unsigned)tt[k] >= nl || (unsigned)ts[k] >= nl)
-                    return fail(PP2P_ERR_ARG, "task " + std::to_string(k) + " names a leaf outside [0, nleaf)");
-    }
+                check_all(v);
+    HIPCHK(hipStreamSynchronize(c->stream));   // the caller may reuse its buffers on return
+    if (!good)
+        return refuse();
     c->ntask += n;
     c->csr_ready = c->items_ready = false;
     return PP2P_OK;
@@ -742,30 +769,6 @@ static int upload_boxes(pp2p_ctx *c, DevBuf<float4> &dst, int n, const float *xy
     HIPCHK(launch_pack_xyz(c->xyz.p, n, dst.p, c->stream));
     return PP2P_OK;
 }
-
-// b with room for n elements, its first `used` (of what it holds) kept.
-extern "C++" {
-template <typename T>
-static hipError_t grow_keep(DevBuf<T> &b, size_t n, size_t used, hipStream_t st)
-{
-    if (n <= b.cap)
-        return hipSuccess;
-    DevBuf<T> nb;
-    hipError_t e = nb.reserve(n);
-    used = std::min(used, b.cap);
-    if (e == hipSuccess && used)
-        e = hipMemcpyAsync(nb.p, b.p, sizeof(T) * used, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-        nb.release();
-        return e;
-    }
-    b.release();
-    b = nb;
-    return hipSuccess;
-}
-}  // extern "C++"
 
 // Room for `frames` frames and `tiles` tiles, the first ones of each kept.
 static int walk_room(pp2p_ctx *c, long long frames, long long keep, long long tiles, long long tkeep, WalkFrames *w)

@@ -1,9 +1,12 @@
 """A refused list: pp2p_set_tasks has dropped the old list, so that the next
 evaluation is that of an empty one; pp2p_add_tasks leaves the list as it was."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import photons_p2p as pp
+from test_zz_no_alloc import _hip_lib
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +49,27 @@ def test_refused_add_tasks_leaves_the_list(gpu_ctx):
     gpu_ctx.zero_acc()
     gpu_ctx.compute()
     assert np.allclose(gpu_ctx.acc(), want, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("n", [300000, 8 << 20])
+def test_a_refused_list_takes_no_memory(n):
+    """The ids are checked before the arrays grow, also those of a list that has
+    to be appended to another one."""
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _hip_lib().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    with pp.Context(0) as ctx:
+        t, s, want = _context(ctx)
+        bad = np.zeros(n, np.int32)
+        bad[n - 1] = 7
+        before = free()
+        for put in (ctx.add_tasks, ctx.set_tasks):
+            with pytest.raises(pp.P2PError, match=f"task {n - 1} "):
+                put(np.zeros(n, np.int32), bad)
+        assert free() > before - 8 * n // 2                  # two arrays of n would take 8 n bytes
+        ctx.set_tasks(t, s)
+        ctx.zero_acc()
+        ctx.compute()
+        assert np.allclose(ctx.acc(), want, rtol=1e-12, atol=0)
