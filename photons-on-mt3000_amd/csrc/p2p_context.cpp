@@ -20,6 +20,7 @@
 #include "p2p_launch.h"
 #include "p2p_m2l.h"
 #include "p2p_pm.h"
+#include "p2p_room.h"
 #include "p2p_scratch.h"
 #include "p2p_tree.h"
 #include "p2p_walk.h"
@@ -653,17 +654,22 @@ int pp2p_set_active(pp2p_ctx *c, const unsigned char *a, int level)
     return PP2P_OK;
 }
 
-// b with room for n elements, its first `used` (of what it holds) kept.
+// b with room for n elements, its first `used` (of what it holds) kept; with none
+// to keep the old array is gone before the new one is asked for.
 extern "C++" {
 template <typename T>
 static hipError_t grow_keep(DevBuf<T> &b, size_t n, size_t used, hipStream_t st)
 {
     if (n <= b.cap)
         return hipSuccess;
+    used = std::min(used, b.cap);
+    if (!used) {
+        b.release();
+        return b.reserve(n);
+    }
     DevBuf<T> nb;
     hipError_t e = nb.reserve(n);
-    used = std::min(used, b.cap);
-    if (e == hipSuccess && used)
+    if (e == hipSuccess)
         e = hipMemcpyAsync(nb.p, b.p, sizeof(T) * used, hipMemcpyDeviceToDevice, st);
     if (e == hipSuccess)
         e = hipStreamSynchronize(st);
@@ -770,15 +776,34 @@ static int upload_boxes(pp2p_ctx *c, DevBuf<float4> &dst, int n, const float *xy
     return PP2P_OK;
 }
 
-// Room for `frames` frames and `tiles` tiles, the first ones of each kept.
-static int walk_room(pp2p_ctx *c, long long frames, long long keep, long long tiles, long long tkeep, WalkFrames *w)
+// Room for `want` frames (`least` where memory is short) and their tiles with
+// `spare` more, the first `keep` frames and `tkeep` tiles kept.
+static int walk_room(pp2p_ctx *c, long long want, long long least, long long keep, long long spare, long long tkeep,
+                     WalkFrames *w)
 {
-    HIPCHK(grow_keep(c->wf, (size_t)frames, (size_t)keep, c->stream));
-    HIPCHK(grow_keep(c->wcode, (size_t)frames, (size_t)keep, c->stream));
-    HIPCHK(grow_keep(c->woff, (size_t)frames, (size_t)keep, c->stream));
-    HIPCHK(grow_keep(c->wcnt, (size_t)frames, 0, c->stream));
-    HIPCHK(grow_keep(c->wlook, (size_t)tiles, 0, c->stream));
-    HIPCHK(grow_keep(c->wsep, (size_t)tiles, (size_t)tkeep, c->stream));
+    const hipStream_t sm = c->stream;
+    HIPCHK(reserve_down(want, least, [&](long long frames) {
+        const long long tiles = std::max(frames, (long long)c->wf.cap) / kWalkTile + spare;
+        hipError_t e = grow_keep(c->wf, (size_t)frames, (size_t)keep, sm);
+        if (e == hipSuccess)
+            e = grow_keep(c->wcode, (size_t)frames, (size_t)keep, sm);
+        if (e == hipSuccess)
+            e = grow_keep(c->woff, (size_t)frames, (size_t)keep, sm);
+        if (e == hipSuccess)
+            e = grow_keep(c->wcnt, (size_t)frames, 0, sm);
+        if (e == hipSuccess)
+            e = grow_keep(c->wlook, (size_t)tiles, 0, sm);
+        if (e == hipSuccess)
+            e = grow_keep(c->wsep, (size_t)tiles, (size_t)tkeep, sm);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();               // or the next launch would report it
+            if (!keep) {
+                c->wf.release(); c->wcode.release(); c->woff.release();
+                c->wcnt.release(); c->wlook.release(); c->wsep.release();
+            }
+        }
+        return e;
+    }));
     const size_t cap = std::min(std::min(c->wf.cap, c->wcode.cap), std::min(c->woff.cap, c->wcnt.cap));
     *w = WalkFrames{c->wf.p, c->wcode.p, c->woff.p, c->wcnt.p, (long long)cap, c->wlook.p, c->wsep.p,
                     (long long)std::min(c->wlook.cap, c->wsep.cap)};
@@ -824,12 +849,22 @@ static int run_walk(pp2p_ctx *c, float open_angle, float cutoff_radius, long lon
             group += 2;
         WalkRound cur{};                           // the next round to run
         cur.n = 1;
-        long long need = 256ll * nleaf + 4096;     // frames: about 250 per leaf on the clustered configurations
+        // Frames to begin with: about 250 per leaf are opened on the clustered
+        // configurations, few with a small cutoff.  A large reservation takes at
+        // most a quarter of the free memory.
+        long long need = 256ll * nleaf + 4096, least = 4096;
+        if (need > (long long)c->wf.cap && need > (1ll << 30) / kWalkFrameBytes) {
+            size_t free_bytes = 0, all = 0;
+            HIPCHK(hipMemGetInfo(&free_bytes, &all));
+            need = modest(need, kWalkFrameBytes, free_bytes);
+        }
         std::vector<WalkRound> h;
         for (bool more = true; more;) {
-            const long long tiles = std::max(need, (long long)c->wf.cap) / kWalkTile + (long long)rounds.size() + group + 2;
-            if ((st = walk_room(c, need, cur.fbase + cur.n, tiles, cur.tbase, &w)))
+            // the frame of a first round is written by walk_begin
+            if ((st = walk_room(c, need, least, cur.fbase ? cur.fbase + cur.n : 0, (long long)rounds.size() + group + 2,
+                                cur.tbase, &w)))
                 return st;
+            need = least = w.cap;                  // no more until a round asks for it
             HIPCHK(c->wround.reserve((size_t)group + 1));
             HIPCHK(walk_begin(w, c->wround.p, group + 1, cur, sm));
             for (int k = 0; k < group; ++k) {
@@ -851,7 +886,8 @@ static int run_walk(pp2p_ctx *c, float open_angle, float cutoff_radius, long lon
                     break;
                 }
                 if (h[k].over) {                   // never the first: round 0 of a group has room
-                    need = std::max(2 * w.cap, h[k].fbase + (long long)h[k].n);
+                    least = h[k].fbase + (long long)h[k].n;
+                    need = std::max(2 * w.cap, least);
                     cur = rounds.back();
                     rounds.pop_back();
                     break;

@@ -5,6 +5,7 @@
 namespace pp2p {
 
 constexpr int kWalkTile = 256;      // fewest frames per tile of a round
+constexpr int kWalkFrameBytes = 17; // of WalkFrames
 constexpr int kWalkSmall = 1024;    // most tiles of that size; larger rounds have tiles of 1024 frames
 
 // The kd-tree as the walk reads it.  son[k] = the two children of node k
