@@ -38,6 +38,17 @@ constexpr int kTreeBlock = 256;
 
 inline unsigned grid_of(long long n) { return (unsigned)((n + kTreeBlock - 1) / kTreeBlock); }
 
+// One workgroup per tile, segment or subtree: a grid holds fewer than 2^32 work
+// items in x, 2^22 workgroups of 1024, and a tree with leaves of one particle has that
+// many segments from 2^23 particles on.
+inline dim3 wide_grid(long long blocks)
+{
+    constexpr long long kWide = 1 << 20;
+    return blocks <= kWide ? dim3((unsigned)blocks) : dim3((unsigned)kWide, (unsigned)((blocks + kWide - 1) / kWide));
+}
+
+__device__ __forceinline__ int block_id() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 __device__ __forceinline__ long long gid() { return (long long)blockIdx.x * kTreeBlock + threadIdx.x; }
 
 __global__ __launch_bounds__(kTreeBlock) void k_tree_init(const int *__restrict__ posi, long long n,
@@ -362,7 +373,7 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_sums(TreeLevelView lv, cons
                                                         double *__restrict__ csum, int *__restrict__ tmap)
 {
     __shared__ double part[kTreeBlock / 64];
-    const int n = *nseg, tile = blockIdx.x;
+    const int n = *nseg, tile = block_id();
     if (n == 0 || tile >= lv.toff[n])
         return;
     const int s = seg_of_tile(lv.toff, n, tile);
@@ -399,7 +410,7 @@ __global__ __launch_bounds__(kUnitBlock) void k_tree_units(TreeLevelView lv, con
 {
     constexpr int kGroups = kTreeTile / kGroup, kPerWave = kGroups / (kUnitBlock / 64);
     __shared__ double start[kGroups];
-    const int n = *nseg, tile = blockIdx.x;
+    const int n = *nseg, tile = block_id();
     if (n == 0 || tile >= lv.toff[n])
         return;
     const int s = tmap[tile];
@@ -440,7 +451,7 @@ __global__ __launch_bounds__(64) void k_tree_mean(TreeLevelView lv, const int *_
                                                 const int *__restrict__ x, double int2pos,
                                                 const GroupUnits *__restrict__ units)
 {
-    const int s = blockIdx.x, lane = threadIdx.x;
+    const int s = block_id(), lane = threadIdx.x;
     if (s >= *nseg)
         return;
     const int2 sg = lv.seg[s];
@@ -480,7 +491,7 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_flags(TreeLevelView lv, con
                                                          int *__restrict__ tcnt, const int *__restrict__ tmap)
 {
     __shared__ int part[kTreeBlock / 64];
-    const int ns = *nseg, tile = blockIdx.x;
+    const int ns = *nseg, tile = block_id();
     if (ns == 0 || tile >= lv.toff[ns])
         return;
     const int s = tmap[tile];
@@ -534,7 +545,7 @@ __global__ __launch_bounds__(kTreeBlock) void k_tree_lists(TreeLevelView lv, con
     __shared__ int before_s[kTreeBlock / 64], total_s[kTreeBlock / 64];
     __shared__ unsigned long long word[kWords];
     __shared__ int wpre[kWords];
-    const int ns = *nseg, tile = blockIdx.x;
+    const int ns = *nseg, tile = block_id();
     if (ns == 0 || tile >= lv.toff[ns])
         return;
     const int s = tmap[tile];
@@ -628,7 +639,7 @@ __device__ __forceinline__ void swap_part(int *x0, int *x1, int *x2, int *idx, i
 __global__ __launch_bounds__(kTreeBlock) void k_tree_swap(TreeLevelView lv, const int *__restrict__ nseg,
                                                         const int *__restrict__ tmap, TreeScratch w)
 {
-    const int ns = *nseg, tile = blockIdx.x;
+    const int ns = *nseg, tile = block_id();
     if (ns == 0 || tile >= lv.toff[ns])
         return;
     const int s = tmap[tile];
@@ -776,13 +787,15 @@ __device__ __forceinline__ int sub_small_before(const SubLds &m, int p)
     return m.wpre[w] + ((p & 63) ? __popcll(m.mask[w] & ((1ull << (p & 63)) - 1ull)) : 0);
 }
 
-__global__ __launch_bounds__(kSubBlock) void k_tree_sub(TreeScratch w, TreeSub *__restrict__ sub, double int2pos,
-                                                      int maxleaf, unsigned short *__restrict__ off_all,
-                                                      TreeCounts *counts)
+__global__ __launch_bounds__(kSubBlock) void k_tree_sub(TreeScratch w, TreeSub *__restrict__ sub, int nsub,
+                                                      double int2pos, int maxleaf,
+                                                      unsigned short *__restrict__ off_all, TreeCounts *counts)
 {
     __shared__ SubLds m;
-    TreeSub &me = sub[blockIdx.x];
-    unsigned short *off = off_all + (size_t)blockIdx.x * kSubLevels;
+    if (block_id() >= nsub)
+        return;
+    TreeSub &me = sub[block_id()];
+    unsigned short *off = off_all + (size_t)block_id() * kSubLevels;
     const int start = me.start, n = me.len, depth = me.depth;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int i = tid; i < kSubMax; i += kSubBlock) {
@@ -1291,11 +1304,11 @@ hipError_t tree_level(const TreeScratch &w, const TreeLevelView &lv, const TreeL
 {
     const int *ns = &counts->nseg[level];
     const int *x = w.x[level % 3];
-    const unsigned nt = (unsigned)tiles;
+    const dim3 nt = wide_grid(tiles);
     GroupUnits *u = reinterpret_cast<GroupUnits *>(units);
     k_tree_sums<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap);
     k_tree_units<<<nt, kUnitBlock, 0, st>>>(lv, ns, x, int2pos, csum, tmap, u);
-    k_tree_mean<<<(unsigned)cap, 64, 0, st>>>(lv, ns, x, int2pos, u);
+    k_tree_mean<<<wide_grid(cap), 64, 0, st>>>(lv, ns, x, int2pos, u);
     k_tree_flags<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, int2pos, mask, tcnt, tmap);
     k_tree_lists<<<nt, kTreeBlock, 0, st>>>(lv, ns, x, mask, tcnt, tmap, w.la, w.lb);
     k_tree_swap<<<nt, kTreeBlock, 0, st>>>(lv, ns, tmap, w);
@@ -1307,7 +1320,7 @@ hipError_t tree_subs(const TreeScratch &w, TreeSub *sub, int nsub, double int2po
                      TreeCounts *counts, hipStream_t st)
 {
     if (nsub > 0)
-        k_tree_sub<<<(unsigned)nsub, kSubBlock, 0, st>>>(w, sub, int2pos, maxleaf, off, counts);
+        k_tree_sub<<<wide_grid(nsub), kSubBlock, 0, st>>>(w, sub, nsub, int2pos, maxleaf, off, counts);
     return hipGetLastError();
 }
 
