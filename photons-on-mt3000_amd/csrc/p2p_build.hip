@@ -364,9 +364,7 @@ __device__ int row_ranges(const RowView &v, int r, long long split, int tgt, int
         int cut = k1;
         if (split > 0)
             cut = cut_search(beg, k1, [&](long long lo, long long step, int n) {
-                const bool over = lane < n && cut_over(P, pb, lo + (lane + 1) * step - 1, wi + kStagePairs, split);
-                const unsigned m = (unsigned)(__ballot(over) >> group) & ((1u << kCutLanes) - 1u);
-                return m ? __builtin_ctz(m) : n;
+                return first_over(__ballot(lane_over(P, pb, lo, step, n, lane, wi + kStagePairs, split)), group, n);
             });
         ++nr;
         const unsigned pc = P(cut);

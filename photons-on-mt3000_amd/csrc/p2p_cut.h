@@ -40,6 +40,22 @@ __host__ __device__ inline bool cut_over(const Prefix &P, unsigned pb, long long
     return (long long)(P((int)(k + 1)) - pb) * wi > split;
 }
 
+// The form of kCutLanes lanes that search together: probe j, taken by lane j ...
+template <class Prefix>
+__host__ __device__ inline bool lane_over(const Prefix &P, unsigned pb, long long lo, long long step, int n, int j,
+                                         long long wi, long long split)
+{
+    return j < n && cut_over(P, pb, lo + (j + 1) * step - 1, wi, split);
+}
+
+// ... and the first lane over the limit of the group that starts at lane `group`
+// of the wave, n when none is (votes: one bit per lane of the wave).
+__host__ __device__ inline int first_over(unsigned long long votes, int group, int n)
+{
+    const unsigned m = (unsigned)(votes >> group) & ((1u << kCutLanes) - 1u);
+    return m ? __builtin_ctz(m) : n;
+}
+
 // one thread's form
 template <class Prefix>
 __host__ __device__ inline int range_cut(const Prefix &P, int beg, int end, long long wi, long long split)
