@@ -30,6 +30,7 @@
 #include <functional>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -151,8 +152,11 @@ public:
     // a pinned one when the stream has passed the copy.
     hipError_t to_device(void *dst, const void *src, size_t bytes, hipStream_t st)
     {
-        if (!staged(src, bytes))
+        hipError_t e = hipSuccess;
+        if (!staged(src, bytes) || ((e = open(piece_of(bytes))) == hipSuccess && !ring_))
             return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
+        if (e != hipSuccess)
+            return e;
         const char *s = static_cast<const char *>(src);
         return to_device_filled(dst, bytes, 1, st, [s](char *at, size_t b, size_t n) { std::memcpy(at, s + b, n); });
     }
@@ -166,9 +170,15 @@ public:
             return hipSuccess;
         hipError_t e = open(piece_of(bytes));
         const size_t piece = piece_of(bytes) / unit * unit;
+        std::unique_ptr<char[]> plain;               // one piece where nothing can be pinned
+        if (e == hipSuccess && !ring_) {
+            plain.reset(new (std::nothrow) char[piece]);
+            if (!plain)
+                return hipErrorOutOfMemory;
+        }
         for (size_t b = 0, k = 0; b < bytes && e == hipSuccess; b += piece, ++k) {
             const size_t n = std::min(piece, bytes - b);
-            char *at = slot(k);
+            char *at = plain ? plain.get() : slot(k);
             e = hipEventSynchronize(ev_[k % kSlots]);            // the copy that last used the slot
             if (e != hipSuccess)
                 break;
@@ -181,7 +191,7 @@ public:
             });
             e = hipMemcpyAsync(static_cast<char *>(dst) + b, at, n, hipMemcpyHostToDevice, st);
             if (e == hipSuccess)
-                e = hipEventRecord(ev_[k % kSlots], st);
+                e = plain ? hipStreamSynchronize(st) : hipEventRecord(ev_[k % kSlots], st);
         }
         return e;
     }
@@ -189,12 +199,12 @@ public:
     // bytes from src to dst; complete when it returns.
     hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t st)
     {
-        if (!staged(dst, bytes)) {
-            hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st) : hipSuccess;
+        const size_t piece = piece_of(bytes), pieces = (bytes + piece - 1) / piece;
+        hipError_t e = hipSuccess;
+        if (!staged(dst, bytes) || ((e = open(piece)) == hipSuccess && !ring_)) {
+            e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st) : hipSuccess;
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }
-        const size_t piece = piece_of(bytes), pieces = (bytes + piece - 1) / piece;
-        hipError_t e = open(piece);
         size_t issued = 0, touched = 0;
         for (size_t k = 0; k < pieces && e == hipSuccess; ++k) {
             for (; issued < pieces && issued < k + kSlots && e == hipSuccess; ++issued) {      // into the emptied slots
@@ -299,7 +309,8 @@ private:
 
     char *slot(size_t k) const { return ring_ + (k % kSlots) * slot_; }
 
-    // the threads, and slots of at least `slot` bytes with no copy in flight.  A ring
+    // the threads, and slots of at least `slot` bytes with no copy in flight, or no
+    // ring where none can be pinned (the copies are then the runtime's).  A ring
     // has small slots or full ones, nothing between: pinning it takes about 0.3 ms
     // whatever its size, and the first touch of its pages (0.4 ms per MiB on one
     // thread) comes with the pieces that use them; a ring that grew with the longest
@@ -323,12 +334,13 @@ private:
         ring_ = nullptr;
         slot_ = 0;
         void *p = nullptr;
-        hipError_t e = hipHostMalloc(&p, kSlots * slot, hipHostMallocDefault);
-        if (e == hipSuccess) {
+        if (hipHostMalloc(&p, kSlots * slot, hipHostMallocDefault) == hipSuccess) {
             ring_ = static_cast<char *>(p);
             slot_ = slot;
+        } else {
+            (void)hipGetLastError();
         }
-        return e;
+        return hipSuccess;
     }
 
     char *ring_ = nullptr;

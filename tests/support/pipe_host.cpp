@@ -19,6 +19,7 @@ struct Op {
 std::deque<Op> g_queue;
 std::map<const char *, size_t> g_pinned;
 long long g_copies, g_allocs, g_alloc_bytes, g_mark, g_done, g_last_error;
+bool g_no_pinning;              // pinned allocations fail
 const char *g_user;             // copies to or from the caller's own array
 size_t g_user_n;
 long long g_user_copies;
@@ -86,6 +87,10 @@ hipError_t hipEventSynchronize(hipEvent_t e)
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
     ++g_allocs;
+    if (g_no_pinning) {
+        g_last_error = hipErrorOutOfMemory;
+        return hipErrorOutOfMemory;
+    }
     g_alloc_bytes += (long long)n;
     *p = std::malloc(n);
     g_pinned[static_cast<char *>(*p)] = n;
@@ -159,6 +164,42 @@ int pipe_copies(const long long *sizes, int count, int pin, size_t shift, long l
     out[1] = user;
     out[2] = allocs;
     out[3] = bytes;
+    return bad;
+}
+
+// Ordinary arrays and records of 40 bytes (their first 12 packed) where nothing
+// can be pinned.  0 when all data arrived and no error stayed behind.
+int pipe_without_pinning(long long n)
+{
+    pp2p::HostPipe pipe;
+    g_no_pinning = true;
+    const size_t bytes = 12 * (size_t)n;
+    char *rec = static_cast<char *>(std::malloc(40 * (size_t)n)), *dev = static_cast<char *>(std::calloc(bytes + 1, 1));
+    char *flat = static_cast<char *>(std::malloc(bytes));
+    for (size_t i = 0; i < 40 * (size_t)n; ++i)
+        rec[i] = (char)(i * 2654435761u >> 13);
+    for (size_t i = 0; i < (size_t)n; ++i)
+        std::memcpy(flat + 12 * i, rec + 40 * i, 12);
+    int bad = pipe.to_device_filled(dev, bytes, 12, nullptr, [&](char *at, size_t b, size_t m) {
+                  for (size_t i = 0; i < m / 12; ++i)
+                      std::memcpy(at + 12 * i, rec + 40 * (b / 12 + i), 12);
+              }) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess;
+    bad |= std::memcmp(dev, flat, bytes) != 0;
+    std::memset(dev, 1, bytes);
+    g_user = flat;
+    g_user_n = bytes;
+    bad |= pipe.to_device(dev, flat, bytes, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess;
+    bad |= std::memcmp(dev, flat, bytes) != 0;
+    std::memset(flat, 1, bytes);
+    bad |= pipe.to_host(flat, dev, bytes, nullptr) != hipSuccess;
+    bad |= std::memcmp(dev, flat, bytes) != 0 || hipGetLastError() != hipSuccess;
+    pipe.release();
+    g_user = nullptr;
+    g_user_n = 0;
+    g_no_pinning = false;
+    std::free(rec);
+    std::free(dev);
+    std::free(flat);
     return bad;
 }
 

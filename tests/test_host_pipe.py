@@ -14,6 +14,7 @@ MIB = 1 << 20
 @pytest.fixture(scope="module")
 def lib():
     h = ctypes.CDLL(LIB)
+    h.pipe_without_pinning.argtypes = [ctypes.c_longlong]
     h.pipe_copies.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p]
     return h
 
@@ -45,3 +46,9 @@ def test_the_ring_is_allocated_once(lib):
     size, costs as much as the first time."""
     c = _copies(lib, [4 * MIB, 5 * MIB, 9 * MIB, 7 * MIB, 64 * MIB], False)
     assert c["allocs"] == 1 and c["bytes"] <= 8 * MIB
+
+
+@pytest.mark.parametrize("n", [1, 100, 349525, 349526, 1000003])
+def test_where_nothing_can_be_pinned(lib, n):
+    """The copies are then the runtime's, records are packed in ordinary memory."""
+    assert lib.pipe_without_pinning(n) == 0
