@@ -1351,9 +1351,8 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
         HIPCHK(hipEventCreate(&c->ev_m1));
     }
     const FmmTree t{nleaf, nnode, c->wson.p, c->wnc.p, c->wlc.p, c->rng.p, c->x3.p};
-    hipEvent_t e0, e1;
-    HIPCHK(hipEventCreate(&e0));
-    HIPCHK(hipEventCreate(&e1));
+    // each pass is read before the next one records
+    const hipEvent_t e0 = c->ev_m0, e1 = c->ev_m1;
     HIPCHK(hipEventRecord(e0, sm));
     // upward: P2M of the leaves, M2M level by level from the deepest
     HIPCHK(launch_cell_centers(t, c->mcenter.p, sm));
@@ -1373,11 +1372,8 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
     if (!st)
         st = walked ? m2l_core(c, (int)ncell, c->walk_m2l_n, c->wm2l_t.p, c->wm2l_s.p, (float)c->params.rs, &m2l_ms)
                     : m2l_core(c, (int)ncell, nm2l, c->mtt.p, c->mts.p, (float)c->params.rs, &m2l_ms);
-    if (st) {
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+    if (st)
         return st;
-    }
     // downward: L2L level by level from the root, then L2P into the accumulator
     HIPCHK(hipEventRecord(e0, sm));
     for (int l = 0; l < c->tree_levels; ++l)
@@ -1389,8 +1385,6 @@ int pp2p_fmm_short(pp2p_ctx *c, long long nm2l, const int *m2l_t, const int *m2l
     HIPCHK(hipEventSynchronize(e1));
     float down_ms = 0.f;
     HIPCHK(hipEventElapsedTime(&down_ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     c->fmm_ready = true;
     if (device_ms)
         *device_ms = up_ms + m2l_ms + down_ms;
