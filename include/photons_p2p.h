@@ -91,9 +91,9 @@ typedef struct {
     int segs_per_octave;  /* table law: 16 or 32 segments per octave of s (0 = 32) */
     int no_cull;          /* 1 disables the per-item j-culling (for measurement) */
     int chunk_model;      /* largest i-chunk of a target per work item: <= 0 the
-                             kernel maximum of 256 (64 lanes x 4 per lane), > 0
+                             kernel maximum of 192 (64 lanes x 3 per lane), > 0
                              at most this many (balanced chunks) */
-    int ipl_max;          /* most i-particles per lane an item may use, 1..4
+    int ipl_max;          /* most i-particles per lane an item may use, 1..3
                              (0 = 4); fewer trades idle lanes for registers */
     int reserved[2];
 } pp2p_tuning;
@@ -280,7 +280,8 @@ int pp2p_compute(pp2p_ctx *ctx, int exec);
  * context's (set beforehand).  task_t, task_s: ntask device ints in
  * [0, nleaf); acc: 3 planes of npart device doubles (x, y, z).  A list
  * whose CSR and items need more than the scratch is refused with
- * PP2P_ERR_ARG (about 1.5 M leaf pairs of leaves of up to 64 particles).
+ * PP2P_ERR_ARG (32 bytes a pair: 2.09 M leaf pairs; fewer where they have
+ * hundreds of thousands of targets, 1.5 M with 3e5).
  * The call synchronises the context stream while it builds the list, then
  * enqueues the force launch; acc is complete after pp2p_sync(ctx).  Every
  * call on one GPU shares that GPU's scratch, which keeps the last call's

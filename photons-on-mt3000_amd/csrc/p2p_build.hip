@@ -4,7 +4,7 @@
 // Target CSR (what the reference builds with thrust in src/gpu_entry.cu:
 // 132-138): a stable radix sort of (task_t, task_s) by target, then the
 // unique targets (rows) and their offsets.  Work items: each row is cut into
-// i-chunks of <= 64 particles and, for the queue form, into source ranges of
+// i-chunks of <= 192 particles and, for the queue form, into source ranges of
 // about `split` pair-interactions; queue items are sorted by cost, largest
 // first (longest-processing-time order for the persistent kernel).
 #include <cstring>
@@ -320,7 +320,7 @@ constexpr ItemShapes item_shapes()
 
 __device__ constexpr ItemShapes kItemShapes = item_shapes();
 
-// i-chunks of a target with ni particles: k = ceil(ni / 256) near-equal chunks
+// i-chunks of a target with ni particles: k = ceil(ni / (64 ipl_max)) near-equal chunks
 // (chunk_model > 0 asks for chunks of at most that many particles instead)
 __device__ __forceinline__ int n_chunks(int ni, float max_chunk, int ipl_max)
 {

@@ -1599,7 +1599,7 @@ static RowArgs row_args(pp2p_ctx *c, const ListView &L)
     ra.act_cnt = c->has_act ? c->act_cnt.p : (c->order_ready ? c->ocnt.p : nullptr);
     ra.act_off = c->has_act ? c->act_off.p : (c->order_ready ? c->ooff.p : nullptr);
     ra.nrows = L.nrows;
-    // chunk_model > 0: at most that many i-particles per item (default 256)
+    // chunk_model > 0: at most that many i-particles per item (default 192)
     ra.stage_ops = c->tuning.chunk_model > 0 ? (float)c->tuning.chunk_model : -1.0f;
     ra.ipl_max = c->tuning.ipl_max >= 1 && c->tuning.ipl_max <= kIplMax ? c->tuning.ipl_max : kIplMax;
     return ra;

@@ -79,7 +79,7 @@ __host__ __device__ constexpr int force_waves_per_group(int law) { return law ==
 struct alignas(16) Item {
     int tgt;      // target leaf id
     int i_beg;    // first i-particle (index into pos) or into ilist
-    int ni;       // number of i-particles, 1..256
+    int ni;       // number of i-particles, 1..192
     int row;      // CSR row
     int s_beg;    // source range [s_beg, s_end) into src[]
     int s_end;

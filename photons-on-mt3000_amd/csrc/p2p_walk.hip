@@ -15,7 +15,8 @@
 // all pairs are leaf pairs, another eighth is dropped.  Three passes turn
 // the rounds into the task list in the order the recursive walk emits it:
 //   forward   codes of the children, and the opened ones placed as round
-//             r + 1 by a prefix sum over the round within the same launch
+//             r + 1 by a prefix sum over the round within the same launch (the
+//             decoupled look-back of Merrill and Garland)
 //   backward  tasks below each frame: its own plus its opened children's, which
 //             lie next to each other
 //   positions each frame's first task position, handed from parent to child;
